@@ -19,6 +19,7 @@
 // drift1 -> conv1st -> update_CompDom -> charge -> update3O -> cvbkforth1st ->
 // kick1 -> drift1 -> diagnostic1.  cvbkforth1st(conv1st(P)) is the 0th-order
 // transform of the wrapped z-frame state, so the pass gathers there directly.
+#include <algorithm>
 #include <climits>
 #include <cmath>
 #include <cstring>
@@ -306,6 +307,16 @@ __device__ inline void wave_count_add(uint32_t *counters, uint32_t key, bool tak
   if (count) atomicAdd(&counters[key], count);
 }
 
+// Tiles up to which a pass counts its new keys in LDS and adds each block's
+// counts once at its end.  Straight global adds (one per key and wavefront)
+// all land on the same few counters on a coarse grid: with 64 tiles (32^3)
+// and 4M particles the keys made an in-place pass 4.9x as long (633 against
+// 130 us, mixed), with 512 tiles and 2M particles 1.7x (203 against 122 us,
+// FP64).  From 4096 tiles on the counters are many enough that the LDS copy
+// changed nothing, so its space (4 KB) stays below the gather box's limit of
+// two (FP32 in place: three) blocks per CU.
+constexpr int kPassLdsTiles = 1024;
+
 // Slot range of a block: contiguous, and the blocks one XCD receives (block
 // b runs on XCD b mod 8) cover adjacent ranges, so each XCD's L2 holds the
 // field of its own part of the sorted bunch.  gridDim.x is a multiple of 8.
@@ -440,6 +451,12 @@ __global__ void __launch_bounds__(kBlock, (pass_blocks_per_cu<T, MODE, KB>(KA)))
   __shared__ GatherLds<T> gbox;
   constexpr bool kStage = kScatter && kStagedScatter;
   __shared__ ScatterStage<T, kStage> sg;
+  __shared__ uint32_t key_hist[kKeys ? kPassLdsTiles : 1];
+  const bool lds_hist = kKeys && c.ntiles <= kPassLdsTiles;
+  if (lds_hist) {
+    for (int t = threadIdx.x; t < c.ntiles; t += kBlock) key_hist[t] = 0u;
+    __syncthreads();
+  }
   if constexpr (kStage) {
     for (int par = 0; par < 2; par++) {
       sg.key[par][threadIdx.x] = kDeadKey;
@@ -708,7 +725,10 @@ __global__ void __launch_bounds__(kBlock, (pass_blocks_per_cu<T, MODE, KB>(KA)))
                         c.tnx * ((cj >> c.tshift[1]) + c.tny * (ck >> c.tshift[2])));
     }
     // histogram of the new keys for the next pass's scatter
-    if constexpr (kKeys) wave_count_add(c.hist_new, knew, knew != kDeadKey);
+    if constexpr (kKeys) {
+      if (lds_hist) wave_count_add(key_hist, knew, knew != kDeadKey);
+      else wave_count_add(c.hist_new, knew, knew != kDeadKey);
+    }
     if constexpr (kStage) {
       // every key's cursor run is known; stage each particle at its place
       if (run_owner) sg.base[threadIdx.x] = run_base;
@@ -807,6 +827,13 @@ __global__ void __launch_bounds__(kBlock, (pass_blocks_per_cu<T, MODE, KB>(KA)))
   }
 
   if (nerr) atomicAdd((unsigned long long *)&c.err->err, (unsigned long long)nerr);
+  if (lds_hist) {
+    __syncthreads();
+    for (int t = threadIdx.x; t < c.ntiles; t += kBlock) {
+      const uint32_t v = key_hist[t];
+      if (v) atomicAdd(&c.hist_new[t], v);
+    }
+  }
   __shared__ double sh[kBlock / 64][kMoments];
   // partials are quantity-major: value q of block b at part[q * kMaxRedBlocks + b]
   double *out = c.part + blockIdx.x;
@@ -907,18 +934,37 @@ k_prologue_range(const double *__restrict__ X, const double *__restrict__ PX,
   }
 }
 
-__global__ void __launch_bounds__(kBlock)
+// The keys of the uploaded (unsorted) particles and their histogram.  A
+// wavefront's 64 particles hold about as many tiles, so counting by global
+// atomics made one per particle: 8.3 ms at 50M particles and 8192 tiles,
+// 0.50 ms at 2M and 512, where the rows take 0.5 ms and 0.02 ms to read.
+// With LDS the block counts all its particles there (one LDS add each) and
+// adds its nonzero counts once; few, large blocks (kKeysBlocks: two per CU)
+// keep those adds below one per eight particles of such bunches.  LDS: the
+// tile count fits kKeysLdsTiles (64 KB, two blocks per CU), else the global
+// counters, which are then many.
+constexpr int kKeysThreads = 512;
+constexpr int kKeysBlocks = 512;
+constexpr int kKeysLdsTiles = 16384;
+
+template <bool LDS>
+__global__ void __launch_bounds__(kKeysThreads)
 k_prologue_keys(const double *__restrict__ X, const double *__restrict__ PX,
                 const double *__restrict__ Y, const double *__restrict__ PY,
                 const double *__restrict__ PH, const double *__restrict__ PT,
                 int64_t n, double gam, double xl, const double *__restrict__ box,
                 int nx, int ny, int nz, int s0, int s1, int s2, int tnx, int tny,
-                uint32_t *__restrict__ key, uint32_t *__restrict__ hist) {
+                int ntiles, uint32_t *__restrict__ key, uint32_t *__restrict__ hist) {
+  extern __shared__ uint32_t keys_lds[];
+  if constexpr (LDS) {
+    for (int t = threadIdx.x; t < ntiles; t += kKeysThreads) keys_lds[t] = 0u;
+    __syncthreads();
+  }
   // box = reduced (min x, min y, min z, max x, max y, max z)
   const double h[3] = {(box[3] - box[0]) / nx, (box[4] - box[1]) / ny,
                        (box[5] - box[2]) / nz};
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t base = (int64_t)blockIdx.x * blockDim.x; base < n; base += stride) {
+  const int64_t stride = (int64_t)gridDim.x * kKeysThreads;
+  for (int64_t base = (int64_t)blockIdx.x * kKeysThreads; base < n; base += stride) {
     const int64_t i = base + threadIdx.x;
     uint32_t k = kDeadKey;
     if (i < n) {
@@ -934,8 +980,16 @@ k_prologue_keys(const double *__restrict__ X, const double *__restrict__ PX,
       }
       k = (uint32_t)((ci[0] >> s0) + tnx * ((ci[1] >> s1) + tny * (ci[2] >> s2)));
       key[i] = k;
+      if constexpr (LDS) atomicAdd(&keys_lds[k], 1u);
     }
-    wave_count_add(hist, k, k != kDeadKey);
+    if constexpr (!LDS) wave_count_add(hist, k, k != kDeadKey);
+  }
+  if constexpr (LDS) {
+    __syncthreads();
+    for (int t = threadIdx.x; t < ntiles; t += kKeysThreads) {
+      const uint32_t v = keys_lds[t];
+      if (v) atomicAdd(&hist[t], v);
+    }
   }
 }
 
@@ -1336,9 +1390,13 @@ struct Runner {
                          b->r[1], b->r[2], b->r[3], b->r[4], b->r[5], b->n, gam,
                          b->c.scxl, b->d_part);
       IZH_CHECK(launch_reduce(st, b->d_part, nb, 6, 0x7ull, 0x38ull, b->d_out));
-      hipLaunchKernelGGL(k_prologue_keys, dim3(nb), dim3(kBlock), 0, st, b->r[0],
-                         b->r[1], b->r[2], b->r[3], b->r[4], b->r[5], b->n, gam,
-                         b->c.scxl, b->d_out, nx, ny, nz, s0, s1, s2, tnx, tny,
+      const bool lds = ntiles <= kKeysLdsTiles;
+      const int kb = (int)std::min<int64_t>((b->n + kKeysThreads - 1) / kKeysThreads,
+                                            lds ? kKeysBlocks : kMaxRedBlocks);
+      hipLaunchKernelGGL(lds ? k_prologue_keys<true> : k_prologue_keys<false>, dim3(kb),
+                         dim3(kKeysThreads), lds ? ntiles * sizeof(uint32_t) : 0, st,
+                         b->r[0], b->r[1], b->r[2], b->r[3], b->r[4], b->r[5], b->n, gam,
+                         b->c.scxl, b->d_out, nx, ny, nz, s0, s1, s2, tnx, tny, ntiles,
                          b->key, hist);
       hipLaunchKernelGGL(k_prologue_dom, dim3(1), dim3(64), 0, st, b->d_out, f->d_dom,
                          nx, ny, nz);
