@@ -724,15 +724,36 @@ k_deposit_chunks(const P *__restrict__ X, const P *__restrict__ Y,
 // follow how far particles move in cells between the key and the deposit
 // (one or two steps): transversely several cells in a drift step, along the
 // bunch (the t-frame phase) about one.  Same fixed-point arithmetic and
-// node order as k_deposit_chunks.
+// node order as k_deposit_chunks.  A block of few particles is bound by
+// clearing and flushing its window (5733 nodes): the window's pitch is fixed
+// and it is cleared 16 bytes a lane, which took a flush's cell index from two
+// integer divisions to multiplies (100k particles on 32^3: 9.4 -> 7.9 us).
+// 512 threads a block gained where chunks are full (4M on 32^3: 38 -> 34 us)
+// and lost more where tiles are sparse (10M on 128x128x256: 264 -> 300 us).
 constexpr int kTileMarginT = 6;
 constexpr int kTileMarginL = 2;
 constexpr int kTileWinEdgeT = (1 << kTileShift) + 1 + 2 * kTileMarginT;
 constexpr int kTileWinEdgeL = (1 << kTileShift) + 1 + 2 * kTileMarginL;
 constexpr int kTileWinCells = kTileWinEdgeT * kTileWinEdgeT * kTileWinEdgeL;
 
+constexpr int kDepThreads = 256;
+// Consecutive chunks one XCD takes in a row (a row of tiles at 128 nodes):
+// their windows overlap, and one L2 then merges the flushes (100k on 32^3:
+// 8.5 -> 7.9 us, 2M on 64^3 59 -> 57 us, 50M on 128x128x256 474 -> 470 us;
+// runs of 64 unbalance the XCDs between core and halo: 507 us).
+constexpr int kDepRun = 16;
+
+// Chunk of physical block p of n: XCD p mod 8 takes every eighth run of
+// kDepRun consecutive chunks.
+__device__ inline int dep_chunk(int p, int n) {
+  const int span = 8 * kDepRun, s = p / span;
+  if ((s + 1) * span > n) return p;  // the incomplete last span: in order
+  const int r = p - s * span;
+  return s * span + (r & 7) * kDepRun + (r >> 3);
+}
+
 template <typename P, bool FAST>
-__global__ void __launch_bounds__(kBlock)
+__global__ void __launch_bounds__(kDepThreads)
 k_deposit_tiles(const P *__restrict__ X, const P *__restrict__ Y,
                 const P *__restrict__ Z, const uint32_t *__restrict__ orig,
                 const double *__restrict__ w0, double w_uniform, int uniform,
@@ -740,9 +761,10 @@ k_deposit_tiles(const P *__restrict__ X, const P *__restrict__ Y,
                 const KeyGrid *__restrict__ kgrid, const DevDom *__restrict__ dom, int nx,
                 int ny, int nz, int s0, int s1, int s2, int tnx, int tny, double scale,
                 unsigned long long *__restrict__ rho, int64_t *__restrict__ spill) {
-  __shared__ unsigned long long win[kTileWinCells];
-  if (blockIdx.x >= *d_nchunks) return;
-  const Chunk ch = chunks[blockIdx.x];
+  __shared__ __align__(16) unsigned long long win[kTileWinCells + 1];
+  const int64_t nchunks = *d_nchunks;
+  if (blockIdx.x >= nchunks) return;
+  const Chunk ch = chunks[dep_chunk((int)blockIdx.x, (int)nchunks)];
   const int tz = (int)(ch.tile / ((uint32_t)tnx * (uint32_t)tny));
   const int rem = (int)(ch.tile % ((uint32_t)tnx * (uint32_t)tny));
   const int ty = rem / tnx, tx = rem % tnx;
@@ -756,8 +778,14 @@ k_deposit_tiles(const P *__restrict__ X, const P *__restrict__ Y,
                                          dom->hinv[1]) - kTileMarginT, 0), ny - wy);
   const int bz = min(max(tile_first_node(tz << s2, kg.lo[2], kg.h[2], dom->range[4],
                                          dom->hinv[2]) - kTileMarginL, 0), nz - wz);
-  const int wcells = wx * wy * wz;
-  for (int c = threadIdx.x; c < wcells; c += kBlock) win[c] = 0ull;
+  // the window's rows keep the full pitch on a smaller grid too, so the
+  // flush splits a cell's index by constants
+  constexpr int kWx = kTileWinEdgeT, kWy = kTileWinEdgeT;
+  const int wcells = kWx * kWy * wz;
+  {
+    ulonglong2 *w2 = reinterpret_cast<ulonglong2 *>(win);
+    for (int c = threadIdx.x; 2 * c < wcells; c += kDepThreads) w2[c] = make_ulonglong2(0ull, 0ull);
+  }
   __syncthreads();
   const P xmin = (P)dom->range[0], ymin = (P)dom->range[2], zmin = (P)dom->range[4];
   const P hx = (P)dom->msize[0], hy = (P)dom->msize[1], hz = (P)dom->msize[2];
@@ -766,12 +794,12 @@ k_deposit_tiles(const P *__restrict__ X, const P *__restrict__ Y,
   uint32_t nspill = 0;
   // kDepBatch slots per thread per round: all their loads are issued first
   constexpr int kDepBatch = 4;
-  for (uint32_t t0 = threadIdx.x; t0 < ch.len; t0 += kDepBatch * kBlock) {
+  for (uint32_t t0 = threadIdx.x; t0 < ch.len; t0 += kDepBatch * kDepThreads) {
     P px[kDepBatch], py[kDepBatch], pz[kDepBatch];
     double pw[kDepBatch];
 #pragma unroll
     for (int u = 0; u < kDepBatch; u++) {
-      const uint32_t t = t0 + u * kBlock;
+      const uint32_t t = t0 + u * kDepThreads;
       const int64_t i = (int64_t)ch.start + (t < ch.len ? t : ch.len - 1);
       px[u] = t < ch.len ? X[i] : (P)NAN;
       py[u] = Y[i];
@@ -791,10 +819,10 @@ k_deposit_tiles(const P *__restrict__ X, const P *__restrict__ Y,
       cic_contrib<P, FAST>(c, pw[u] * scale, v);
       const int li = c.i - bx, lj = c.j - by, lk = c.k - bz;
       if (li >= 0 && li + 1 < wx && lj >= 0 && lj + 1 < wy && lk >= 0 && lk + 1 < wz) {
-        const int l0 = li + wx * (lj + wy * lk);
+        const int l0 = li + kWx * (lj + kWy * lk);
 #pragma unroll
         for (int q = 0; q < 8; q++)
-          atomicAdd(&win[l0 + kNode[q][0] + wx * (kNode[q][1] + wy * kNode[q][2])],
+          atomicAdd(&win[l0 + kNode[q][0] + kWx * (kNode[q][1] + kWy * kNode[q][2])],
                     (unsigned long long)v[q]);
       } else {
         const int64_t g0 = c.i + sy * c.j + sz * c.k;
@@ -807,10 +835,10 @@ k_deposit_tiles(const P *__restrict__ X, const P *__restrict__ Y,
     }
   }
   __syncthreads();
-  for (int c = threadIdx.x; c < wcells; c += kBlock) {
+  for (int c = threadIdx.x; c < wcells; c += kDepThreads) {
     const unsigned long long v = win[c];
     if (v == 0ull) continue;
-    const int lx = c % wx, ly = (c / wx) % wy, lz = c / (wx * wy);
+    const int lx = c % kWx, ly = (c / kWx) % kWy, lz = c / (kWx * kWy);
     atomicAdd(&rho[(bx + lx) + sy * (by + ly) + sz * (bz + lz)], v);
   }
   if (spill) {
@@ -1111,7 +1139,7 @@ int launch_deposit(izh_bunch *b, izh_field *f, const Chunk *chunks, const KeyGri
       const int tnx = f->nx >> s0, tny = f->ny >> s1;
       int64_t *spill = b->d_scal ? &b->d_scal->overflow : nullptr;
       const auto go = [&](auto kern, const auto *tp) {
-        hipLaunchKernelGGL(kern, dim3((unsigned)max_chunks), dim3(kBlock), 0, f->stream, tp,
+        hipLaunchKernelGGL(kern, dim3((unsigned)max_chunks), dim3(kDepThreads), 0, f->stream, tp,
                            tp + b->cap, tp + 2 * b->cap, b->orig, b->w0, b->w_value,
                            b->w_uniform, chunks, d_nchunks, kgrid, f->d_dom, f->nx, f->ny,
                            f->nz, s0, s1, s2, tnx, tny, f->fixed_scale, f->rho_fx, spill);

@@ -1023,6 +1023,7 @@ struct FinCfg {
   const uint32_t *hist;     // histogram of the keys just written
   uint32_t *cursor;         // -> exclusive offsets of hist
   Chunk *chunks;            // -> deposit chunks of that grouping
+  uint32_t chunk;           // slots per chunk at most
   int64_t *nchunks;         // -> their number
   uint32_t *hist_zero;      // histogram the next pass fills
   int scan;                 // the pass computed keys: scan their histogram
@@ -1145,7 +1146,7 @@ __global__ void __launch_bounds__(1024) k_finalize(FinCfg f) {
   for (int t = t0; t < t1; t++) {
     uint32_t h = f.hist[t];
     cnt += h;
-    nch += (h + kChunk - 1) / kChunk;
+    nch += (h + f.chunk - 1) / f.chunk;
   }
   ssum[tid] = cnt;
   csum[tid] = nch;
@@ -1162,9 +1163,9 @@ __global__ void __launch_bounds__(1024) k_finalize(FinCfg f) {
   for (int t = t0; t < t1; t++) {
     uint32_t h = f.hist[t];
     f.cursor[t] = off;
-    for (uint32_t s = 0; s < h; s += kChunk) {
+    for (uint32_t s = 0; s < h; s += f.chunk) {
       f.chunks[coff].start = off + s;
-      f.chunks[coff].len = min((uint32_t)kChunk, h - s);
+      f.chunks[coff].len = min(f.chunk, h - s);
       f.chunks[coff].tile = (uint32_t)t;
       coff++;
     }
@@ -1195,7 +1196,7 @@ int bunch_alloc_fused(izh_bunch *b, int ntiles, int64_t nseg) {
   if (!b->r_alt[0]) IZH_CHECK(bunch_alloc_alt(b));
   if (!b->h_scal)
     IZH_HIP(hipHostMalloc((void **)&b->h_scal, sizeof(DevScal), hipHostMallocDefault));
-  const int64_t nch = b->cap / kChunk + ntiles + 1;
+  const int64_t nch = b->cap / chunk_len(b->cap) + ntiles + 1;
   if (ntiles > b->ntiles_cap || nch > b->nchunks_cap) {
     for (int k = 0; k < 2; k++)
       if (b->hist[k]) (void)hipFree(b->hist[k]);
@@ -1376,6 +1377,7 @@ struct Runner {
     fc.dom = f->d_dom;
     fc.moments = b->d_moments;
     fc.ntiles = ntiles;
+    fc.chunk = (uint32_t)chunk_len(b->cap);
     fc.nx = nx; fc.ny = ny; fc.nz = nz;
     fc.gam = gam; fc.scfreq = b->c.scfreq; fc.clight = b->c.clight; fc.pi = b->c.pi;
     fc.scxl = b->c.scxl; fc.mass = b->mass; fc.charge = b->charge;

@@ -1,6 +1,6 @@
 """izh_run against izh_step at the sizes where a kernel of the fused run
 changes its form: tile counts around the limits of the LDS key histograms,
-and bunches from a few particles up.  The bar is the fused run's own: 1e-10
+deposit chunks of every length, grids narrower than the deposit's window.  The bar is the fused run's own: 1e-10
 relative in the diagnostics and the particles."""
 import pytest
 
@@ -35,3 +35,14 @@ def run_against_step(gpu, n, grid, period, steps=5, seed=3):
 ])
 def test_key_histograms(gpu, n, grid, period):
     run_against_step(gpu, n, grid, period)
+
+
+@pytest.mark.parametrize("n,grid,period", [
+    (50, (4, 8, 16), 1),             # a grid inside one window
+    (700, (8, 16, 4), 2),
+    (262_143, (32, 32, 32), 4),      # the last bunch of 1024-slot chunks
+    (262_145, (32, 16, 64), 4),      # the first of 2048
+    (4_194_305, (32, 32, 32), 2),    # full-length chunks
+])
+def test_deposit_chunks(gpu, n, grid, period):
+    run_against_step(gpu, n, grid, period, steps=3)
