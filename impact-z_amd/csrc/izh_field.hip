@@ -45,7 +45,12 @@ constexpr int kFftPoints = 2048;  // points per block in LDS
 constexpr int kFftPointsZ = 4096; // the fused z pass: 8 lines of 512 at 128x128x256
 constexpr int kFftMinLine = 8;    // shortest line (a mesh of 4 nodes doubled)
 
-enum Load { kLoadReal = 0, kLoadCplx = 1, kLoadEven = 2, kLoadHerm = 3 };
+// kLoadFx: the deposit's fixed-point charge, converted to the grid type as it
+// is read; the pass also leaves the converted grid in Lines::rho and the
+// accumulator cleared for the next deposit.  kLoadIgf: an even line of the
+// integrated Green function, the 8-corner difference of its antiderivative.
+enum Load { kLoadReal = 0, kLoadCplx = 1, kLoadEven = 2, kLoadHerm = 3, kLoadFx = 4,
+            kLoadIgf = 5 };
 enum Store { kStoreCplx = 0, kStoreReal = 1 };
 
 struct Lines {
@@ -62,7 +67,19 @@ struct Lines {
   const void *green;
   int64_t gkx, gky;        // G^ strides of ky and kz: ldx*(nz+1), ldx
   int my;                  // doubled y length, for folding the line's y index
+  void *rho;               // kLoadFx: the converted grid
+  double fx_inv;           // kLoadFx: grid value of one fixed-point unit
+  int tx, ty;              // kLoadIgf: corners per row, rows per plane
 };
+
+// 8-corner difference of the antiderivative at the cells' corners
+// (src/Appl/Field.f90:420-428), node (i, j, k) at c of a grid of tx x ty
+// corners per plane.
+__device__ inline double igf_diff(const double *__restrict__ t, int64_t c, int64_t tx,
+                                  int64_t txy) {
+  return t[c + 1 + tx + txy] - t[c + tx + txy] - t[c + 1 + txy] + t[c + txy] -
+         t[c + 1 + tx] + t[c + tx] + t[c + 1] - t[c];
+}
 
 // Logical block of physical block p of n: the hardware deals blocks to the
 // 8 XCDs in turn (block p to XCD p mod 8), each XCD with its own L2.  XCD x
@@ -225,10 +242,14 @@ __device__ inline void map_thread(int t, int64_t estride, int log2L, int log2B, 
 // other than 1, or the fused z pass's multiply) do not all hit one bank.
 // LL: log2 of the line length when it is fixed at compile time (the common
 // lengths, so every index split and LDS position folds), 0 to take it from p.
+// buf: kFftLds<PTS> points of LDS, tw: L/2 twiddles of it; block bid of nb.
+template <int PTS>
+constexpr int kFftLds = PTS + PTS / kFftMinLine;
+
 template <typename T, int LOAD, int STORE, bool CONV, bool PAIR, int PTS, int LL>
-__global__ void __launch_bounds__(kFftThreads)
-k_fft_lines(Lines p, const cx<T> *__restrict__ twg, int inverse) {
-  __shared__ cx<T> buf[PTS + PTS / kFftMinLine];
+__device__ __attribute__((always_inline)) inline void fft_lines_block(
+    const Lines &p, const cx<T> *__restrict__ twg, int inverse, int bid, int nb, cx<T> *buf,
+    cx<T> *tw) {
   static_assert(PTS == 2048 || PTS == 4096, "points per block");
   constexpr int kLog2Pts = PTS == 4096 ? 12 : 11;
   const int log2L = LL ? LL : p.log2L;
@@ -237,8 +258,6 @@ k_fft_lines(Lines p, const cx<T> *__restrict__ twg, int inverse) {
   const int B = 1 << log2B;
   const int LP = L + 1;
   const int mask = L >= 64 ? 15 : 0;
-  extern __shared__ __align__(16) unsigned char fft_dyn[];  // L/2 twiddles
-  cx<T> *tw = reinterpret_cast<cx<T> *>(fft_dyn);
   // twiddles are written to LDS together with the line data below
   constexpr int kTwPer = PTS / 2 / kFftThreads;  // L/2 <= PTS/2
   cx<T> twv[kTwPer];
@@ -254,7 +273,7 @@ k_fft_lines(Lines p, const cx<T> *__restrict__ twg, int inverse) {
   }
   const int nf = (int)p.nf;
   const int nlines = nf * (int)p.ns;
-  const int line0 = xcd_block((int)blockIdx.x, (int)gridDim.x) * B;
+  const int line0 = xcd_block(bid, nb) * B;
   // fused z pass: fetch the G^ values of the thread's group of the fused
   // middle run first, so their latency hides behind the forward transform.
   // Lanes walk across the block's lines first (neighbouring x indices,
@@ -334,12 +353,50 @@ k_fft_lines(Lines p, const cx<T> *__restrict__ twg, int inverse) {
     }
     __syncthreads();
     first = 3;
+  } else if constexpr (LOAD == kLoadIgf) {
+    // ---- even lines of G: each value is formed once and written to both of
+    // its places, m and L-m (thread m = 0 also takes m = L/2)
+    static_assert(LOAD != kLoadIgf || PAIR, "even lines travel in pairs");
+    const double *src = (const double *)p.src;
+    const int64_t txy = (int64_t)p.tx * p.ty;
+    const int half = L >> 1;
+    constexpr int kPer = PTS / 2 / kFftThreads;
+#pragma unroll
+    for (int it = 0; it < kPer; it++) {
+      const int t = threadIdx.x + it * kFftThreads;
+      const int lb = t >> (log2L - 1), m = t & (half - 1);
+      const int l0 = 2 * (line0 + lb), l1 = l0 + 1;
+      const bool has0 = l0 < nlines, has1 = l1 < nlines;
+      int j0, k0, j1, k1;
+      line_fs(has0 ? l0 : 0, p, j0, k0);
+      line_fs(has1 ? l1 : 0, p, j1, k1);
+      const int64_t c0 = j0 * (int64_t)p.tx + k0 * txy, c1 = j1 * (int64_t)p.tx + k1 * txy;
+      const double a = igf_diff(src, c0 + m, p.tx, txy);
+      const double b = igf_diff(src, c1 + m, p.tx, txy);
+      const cx<T> v = {has0 ? (T)a : (T)0, has1 ? (T)b : (T)0};
+      cx<T> *row = buf + lb * LP;
+      row[lds_pos(m, mask)] = v;
+      if (m > 0) {
+        row[lds_pos(L - m, mask)] = v;
+      } else {
+        const double ah = igf_diff(src, c0 + half, p.tx, txy);
+        const double bh = igf_diff(src, c1 + half, p.tx, txy);
+        row[lds_pos(half, mask)] = {has0 ? (T)ah : (T)0, has1 ? (T)bh : (T)0};
+      }
+    }
+#pragma unroll
+    for (int it = 0; it < kTwPer; it++) {
+      const int t = threadIdx.x + it * kFftThreads;
+      if (t < (L >> 1)) tw[t] = twv[it];
+    }
+    __syncthreads();
   } else {
     // ---- load (zero padding / even extension / Hermitian completion): all of
     // a thread's loads are issued before the first LDS write
     constexpr int kPer = PTS / kFftThreads;  // B * L == PTS
     cx<T> ld[kPer];
     int slot[kPer];
+    int64_t at[kPer][2];  // kLoadFx: where the pair's values came from (-1: nowhere)
 #pragma unroll
     for (int it = 0; it < kPer; it++) {
       const int t = threadIdx.x + it * kFftThreads;
@@ -348,6 +405,7 @@ k_fft_lines(Lines p, const cx<T> *__restrict__ twg, int inverse) {
       const int line = line0 + lb;
       slot[it] = lb * LP + lds_pos(m, mask);
       T re = (T)0, im = (T)0;
+      if (LOAD == kLoadFx) at[it][0] = at[it][1] = -1;
       if (PAIR) {
         const int l0 = 2 * line, l1 = l0 + 1;
         const T *src = (const T *)p.src;
@@ -367,6 +425,16 @@ k_fft_lines(Lines p, const cx<T> *__restrict__ twg, int inverse) {
             if (m < p.Lin) {
               re = src[b0 + m * p.se];
               im = has1 ? src[b1 + m * p.se] : (T)0;
+            }
+          } else if (LOAD == kLoadFx) {
+            if (m < p.Lin) {
+              const long long *fx = (const long long *)p.src;
+              at[it][0] = b0 + m * p.se;
+              re = (T)((double)fx[at[it][0]] * p.fx_inv);
+              if (has1) {
+                at[it][1] = b1 + m * p.se;
+                im = (T)((double)fx[at[it][1]] * p.fx_inv);
+              }
             }
           } else {  // kLoadHerm: Z = X + iY of the completed spectra
             const bool lo = m <= (L >> 1);
@@ -404,6 +472,15 @@ k_fft_lines(Lines p, const cx<T> *__restrict__ twg, int inverse) {
     }
 #pragma unroll
     for (int it = 0; it < kPer; it++) buf[slot[it]] = ld[it];
+    if (LOAD == kLoadFx) {
+      T *rho = (T *)p.rho;
+      unsigned long long *fx = (unsigned long long *)const_cast<void *>(p.src);
+#pragma unroll
+      for (int it = 0; it < kPer; it++) {
+        if (at[it][0] >= 0) { rho[at[it][0]] = ld[it].re; fx[at[it][0]] = 0ull; }
+        if (at[it][1] >= 0) { rho[at[it][1]] = ld[it].im; fx[at[it][1]] = 0ull; }
+      }
+    }
 #pragma unroll
     for (int it = 0; it < kTwPer; it++) {
       const int t = threadIdx.x + it * kFftThreads;
@@ -497,16 +574,47 @@ k_fft_lines(Lines p, const cx<T> *__restrict__ twg, int inverse) {
   }
 }
 
+template <typename T, int LOAD, int STORE, bool CONV, bool PAIR, int PTS, int LL>
+__global__ void __launch_bounds__(kFftThreads)
+k_fft_lines(Lines p, const cx<T> *__restrict__ twg, int inverse) {
+  __shared__ cx<T> buf[kFftLds<PTS>];
+  extern __shared__ __align__(16) unsigned char fft_dyn[];  // L/2 twiddles
+  fft_lines_block<T, LOAD, STORE, CONV, PAIR, PTS, LL>(
+      p, twg, inverse, (int)blockIdx.x, (int)gridDim.x, buf,
+      reinterpret_cast<cx<T> *>(fft_dyn));
+}
+
+// Two independent forward passes along one axis in one launch: nba blocks of
+// the Green function's lines (pairs of even real lines), then, from the next
+// multiple of eight on (which keeps xcd_block's dealing), those of the charge.
+// The Green function's transform and the charge's have the same depth, so a
+// step's chain is as long as the charge's alone, with no second stream.
+template <typename T, int LOADA, int LOADB, int STOREB, bool PAIRB, int LL>
+__global__ void __launch_bounds__(kFftThreads)
+k_fft_two(Lines a, Lines b, int nba, int nbb, const cx<T> *__restrict__ twg) {
+  __shared__ cx<T> buf[kFftLds<kFftPoints>];
+  extern __shared__ __align__(16) unsigned char fft_dyn[];
+  cx<T> *tw = reinterpret_cast<cx<T> *>(fft_dyn);
+  const int first_b = (nba + 7) & ~7, bid = (int)blockIdx.x;
+  if (bid < first_b) {
+    if (bid < nba)
+      fft_lines_block<T, LOADA, kStoreReal, false, true, kFftPoints, LL>(a, twg, 0, bid, nba,
+                                                                         buf, tw);
+  } else {
+    fft_lines_block<T, LOADB, STOREB, false, PAIRB, kFftPoints, LL>(b, twg, 0, bid - first_b,
+                                                                    nbb, buf, tw);
+  }
+}
+
 // ------------------------------------------------------ Green function
 // IGF antiderivative at cell corners (src/Appl/Field.f90:384-418), FP64,
-// mesh sizes from the device domain.
-__global__ void k_igf_corner(double *__restrict__ out, int tx, int ty, int tz,
-                             const DevDom *__restrict__ dom) {
+// mesh sizes from the device domain; corners first, first + stride, ...
+__device__ inline void igf_corners(double *__restrict__ out, int tx, int ty, int tz,
+                                   const DevDom *__restrict__ dom, int first, int stride) {
   const double hx = dom->msize[0], hy = dom->msize[1], hz = dom->msize[2];
   const double vol = hx * hy * hz;
   const int n = tx * ty * tz;
-  for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < n;
-       c += gridDim.x * blockDim.x) {
+  for (int c = first; c < n; c += stride) {
     int i = c % tx;
     int j = (c / tx) % ty;
     int k = c / (tx * ty);
@@ -522,34 +630,14 @@ __global__ void k_igf_corner(double *__restrict__ out, int tx, int ty, int tz,
   }
 }
 
-// 8-corner difference (src/Appl/Field.f90:420-428) -> g on (nx+1,ny+1,nz+1).
-template <typename T>
-__global__ void k_igf_diff(const double *__restrict__ t, T *__restrict__ g,
-                           int nx, int ny, int nz) {
-  const int tx = nx + 2, ty = ny + 2;
-  const int gx = nx + 1, gy = ny + 1, gz = nz + 1;
-  const int n = gx * gy * gz;
-  for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < n;
-       c += gridDim.x * blockDim.x) {
-    int i = c % gx;
-    int j = (c / gx) % gy;
-    int k = c / (gx * gy);
-#define TT(a, b, cc) t[(a) + tx * ((b) + ty * (cc))]
-    double v = TT(i + 1, j + 1, k + 1) - TT(i, j + 1, k + 1) - TT(i + 1, j, k + 1) +
-               TT(i, j, k + 1) - TT(i + 1, j + 1, k) + TT(i, j + 1, k) +
-               TT(i + 1, j, k) - TT(i, j, k);
-#undef TT
-    g[c] = (T)v;
-  }
+__global__ void __launch_bounds__(kBlock)
+k_igf_corner(double *__restrict__ out, int tx, int ty, int tz,
+             const DevDom *__restrict__ dom) {
+  igf_corners(out, tx, ty, tz, dom, blockIdx.x * blockDim.x + threadIdx.x,
+              gridDim.x * blockDim.x);
 }
 
 // --------------------------------------------------------------- deposit
-__global__ void k_zero_u64(unsigned long long *__restrict__ p, int64_t n) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x)
-    p[i] = 0ull;
-}
-
 // Lower-node cell (0-based) and CIC weights of deposit_BeamBunch
 // (src/Appl/BeamBunch.f90:3737-3744) in the position type P.
 template <typename P>
@@ -760,11 +848,21 @@ k_deposit_tiles(const P *__restrict__ X, const P *__restrict__ Y,
                 const Chunk *__restrict__ chunks, const int64_t *__restrict__ d_nchunks,
                 const KeyGrid *__restrict__ kgrid, const DevDom *__restrict__ dom, int nx,
                 int ny, int nz, int s0, int s1, int s2, int tnx, int tny, double scale,
-                unsigned long long *__restrict__ rho, int64_t *__restrict__ spill) {
+                unsigned long long *__restrict__ rho, int64_t *__restrict__ spill,
+                double *__restrict__ corner, int ncorner) {
   __shared__ __align__(16) unsigned long long win[kTileWinCells + 1];
+  // the first ncorner blocks (a multiple of eight) form the corners of the
+  // step's Green function, which needs only the domain: arithmetic beside
+  // the deposit's LDS traffic, and no launch of its own
+  if ((int)blockIdx.x < ncorner) {
+    igf_corners(corner, nx + 2, ny + 2, nz + 2, dom,
+                (int)blockIdx.x * kDepThreads + (int)threadIdx.x, ncorner * kDepThreads);
+    return;
+  }
+  const int bid = (int)blockIdx.x - ncorner;
   const int64_t nchunks = *d_nchunks;
-  if (blockIdx.x >= nchunks) return;
-  const Chunk ch = chunks[dep_chunk((int)blockIdx.x, (int)nchunks)];
+  if (bid >= nchunks) return;
+  const Chunk ch = chunks[dep_chunk(bid, (int)nchunks)];
   const int tz = (int)(ch.tile / ((uint32_t)tnx * (uint32_t)tny));
   const int rem = (int)(ch.tile % ((uint32_t)tnx * (uint32_t)tny));
   const int ty = rem / tnx, tx = rem % tnx;
@@ -849,12 +947,17 @@ k_deposit_tiles(const P *__restrict__ X, const P *__restrict__ Y,
   }
 }
 
+// The grid charge of one izh_charge, and the accumulator cleared for the next
+// deposit (field_alloc clears it first; the fused run's forward x pass does
+// both as it reads).
 template <typename T>
-__global__ void k_fx_to_grid(const unsigned long long *__restrict__ fx,
-                             T *__restrict__ rho, int64_t n, double inv) {
+__global__ void k_fx_to_grid(unsigned long long *__restrict__ fx, T *__restrict__ rho,
+                             int64_t n, double inv) {
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x)
+       i += (int64_t)gridDim.x * blockDim.x) {
     rho[i] = (T)((double)(long long)fx[i] * inv);
+    fx[i] = 0ull;
+  }
 }
 
 // ------------------------------------------------------------- E field
@@ -894,11 +997,9 @@ int ilog2(int v) {
   return r;
 }
 
-template <typename T, int LOAD, int STORE, bool CONV, bool PAIR = false>
-int run_lines(hipStream_t stream, Lines p, const void *tw, bool inverse) {
-  // the fused z pass takes twice the lines per block: its rows of the
-  // spectrum and of G^ are read across the lines
-  constexpr int pts = CONV ? kFftPointsZ : kFftPoints;
+// Completes a pass's description (block shape, index multiplier) and checks it
+// against what the kernel assumes; *nblk: its blocks.
+int lines_setup(Lines &p, int pts, bool pair, int64_t *nblk) {
   p.log2L = ilog2(p.L);
   if (p.nfv == 0) p.nfv = p.nf;
   if (p.L < kFftMinLine || p.L > pts || (1 << p.log2L) != p.L)
@@ -912,8 +1013,18 @@ int run_lines(hipStream_t stream, Lines p, const void *tw, bool inverse) {
                 (long long)p.nf, (long long)p.ns);
   p.nf_mul = ((1ull << 40) + (uint64_t)p.nf - 1) / (uint64_t)p.nf;
   const int64_t nlines = p.nf * p.ns;
-  const int64_t nfft = PAIR ? (nlines + 1) / 2 : nlines;
-  const int64_t nblk = (nfft + p.B - 1) / p.B;
+  const int64_t nfft = pair ? (nlines + 1) / 2 : nlines;
+  *nblk = (nfft + p.B - 1) / p.B;
+  return IZH_OK;
+}
+
+template <typename T, int LOAD, int STORE, bool CONV, bool PAIR = false>
+int run_lines(hipStream_t stream, Lines p, const void *tw, bool inverse) {
+  // the fused z pass takes twice the lines per block: its rows of the
+  // spectrum and of G^ are read across the lines
+  constexpr int pts = CONV ? kFftPointsZ : kFftPoints;
+  int64_t nblk = 0;
+  IZH_CHECK(lines_setup(p, pts, PAIR, &nblk));
   const size_t tw_bytes = (size_t)(p.L / 2) * sizeof(cx<T>);
   const dim3 g((unsigned)nblk), b(kFftThreads);
   const cx<T> *twc = (const cx<T> *)tw;
@@ -941,56 +1052,45 @@ int run_lines(hipStream_t stream, Lines p, const void *tw, bool inverse) {
   return IZH_OK;
 }
 
-// G^ of the field's current domain: IGF corners, 8-corner difference and
-// three even real transforms, on stream gs.
-template <typename T>
-int green_t(izh_field *f, hipStream_t gs) {
-  const int nx = f->nx, ny = f->ny, nz = f->nz;
-  const int mx = 2 * nx, my = 2 * ny, mz = 2 * nz, kx = nx + 1;
-  {
-    ScopedTimer tm_(IZH_T_GREEN, gs);
-    int nc = (nx + 2) * (ny + 2) * (nz + 2);
-    hipLaunchKernelGGL(k_igf_corner, dim3(grid_for(nc)), dim3(kBlock), 0,
-                       gs, f->corner, nx + 2, ny + 2, nz + 2, f->d_dom);
-    int ng = (nx + 1) * (ny + 1) * (nz + 1);
-    hipLaunchKernelGGL(k_igf_diff<T>, dim3(grid_for(ng)), dim3(kBlock), 0,
-                       gs, f->corner, (T *)f->green_t, nx, ny, nz);
-    IZH_HIP(hipGetLastError());
-    Lines p{};
-    // x: lines (j<=ny, k<=nz), contiguous; green_t -> green
-    p.src = f->green_t; p.dst = f->green;
-    p.nf = ny + 1; p.ns = nz + 1;
-    p.sf = kx; p.ss = (int64_t)kx * (ny + 1); p.se = 1;
-    p.df = kx; p.ds = (int64_t)kx * (ny + 1); p.de = 1;
-    p.L = mx; p.Lin = p.L; p.Lout = nx + 1; p.out_scale = 1.0;
-    IZH_CHECK((run_lines<T, kLoadEven, kStoreReal, false, true>(gs, p, f->tw_x, false)));
-    // y: lines (i<=nx, k<=nz); green -> green_t
-    p.src = f->green; p.dst = f->green_t;
-    p.nf = kx; p.ns = nz + 1;
-    p.sf = 1; p.ss = (int64_t)kx * (ny + 1); p.se = kx;
-    p.df = 1; p.ds = (int64_t)kx * (ny + 1); p.de = kx;
-    p.L = my; p.Lin = p.L; p.Lout = ny + 1;
-    IZH_CHECK((run_lines<T, kLoadEven, kStoreReal, false, true>(gs, p, f->tw_y, false)));
-    // z: lines (i<=nx, j<=ny); green_t -> green, scaled by 1/(mx my mz).
-    // G^ is stored [j][k][i] with i rows at the spectra's pitch ldx: the
-    // fused z pass of a block of x lines then reads, for its one y index,
-    // aligned runs of neighbouring i at neighbouring k, one contiguous
-    // region of ldx*(nz+1) values instead of one value run per z plane.
-    const int64_t ld = f->ldx;
-    p.src = f->green_t; p.dst = f->green;
-    p.nf = kx; p.ns = ny + 1;
-    p.sf = 1; p.ss = kx; p.se = (int64_t)kx * (ny + 1);
-    p.df = 1; p.ds = ld * (nz + 1); p.de = ld;
-    p.L = mz; p.Lin = p.L; p.Lout = nz + 1;
-    p.out_scale = 1.0 / ((double)mx * my * mz);
-    IZH_CHECK((run_lines<T, kLoadEven, kStoreReal, false, true>(gs, p, f->tw_z, false)));
+// k_fft_two: the Green function's lines ga and the charge's lines cb, of one
+// length.
+template <typename T, int LOADA, int LOADB, int STOREB, bool PAIRB>
+int run_two(hipStream_t stream, Lines ga, Lines cb, const void *tw) {
+  int64_t nba = 0, nbb = 0;
+  if (ga.L != cb.L) return fail(IZH_ERR_ARG, "FFT passes of %d and %d points", ga.L, cb.L);
+  IZH_CHECK(lines_setup(ga, kFftPoints, true, &nba));
+  IZH_CHECK(lines_setup(cb, kFftPoints, PAIRB, &nbb));
+  const size_t tw_bytes = (size_t)(ga.L / 2) * sizeof(cx<T>);
+  const dim3 g((unsigned)(((nba + 7) & ~(int64_t)7) + nbb)), b(kFftThreads);
+  const cx<T> *twc = (const cx<T> *)tw;
+  const int na = (int)nba, nb = (int)nbb;
+  switch (ga.log2L) {
+    case 7:
+      hipLaunchKernelGGL((k_fft_two<T, LOADA, LOADB, STOREB, PAIRB, 7>), g, b, tw_bytes,
+                         stream, ga, cb, na, nb, twc);
+      break;
+    case 8:
+      hipLaunchKernelGGL((k_fft_two<T, LOADA, LOADB, STOREB, PAIRB, 8>), g, b, tw_bytes,
+                         stream, ga, cb, na, nb, twc);
+      break;
+    case 9:
+      hipLaunchKernelGGL((k_fft_two<T, LOADA, LOADB, STOREB, PAIRB, 9>), g, b, tw_bytes,
+                         stream, ga, cb, na, nb, twc);
+      break;
+    default:
+      hipLaunchKernelGGL((k_fft_two<T, LOADA, LOADB, STOREB, PAIRB, 0>), g, b, tw_bytes,
+                         stream, ga, cb, na, nb, twc);
+      break;
   }
+  IZH_HIP(hipGetLastError());
   return IZH_OK;
 }
 
-// The convolution with the G^ in place: forward x, forward y, the fused z
-// pass, inverse y, inverse x, on the field's stream.
-template <typename T>
+// The convolution: the transforms of G (from its corners) and of the charge,
+// pass by pass in common launches, the fused z pass, inverse y, inverse x, on
+// the field's stream.  FX: the charge is the deposit's fixed-point
+// accumulator, converted (and cleared) as it is read; else the grid rho.
+template <typename T, bool FX>
 int convolve_t(izh_field *f) {
   const int nx = f->nx, ny = f->ny, nz = f->nz;
   const int mx = 2 * nx, my = 2 * ny, mz = 2 * nz, kx = nx + 1;
@@ -1000,21 +1100,46 @@ int convolve_t(izh_field *f) {
   // passes run over all ld x lines, so a block's run of neighbouring lines
   // starts on a 128-byte boundary; lines kx..ld-1 are padding.
   const int64_t ld = f->ldx;
-  // ---- forward x: rho (nx,ny,nz) real -> A (kx of ld, ny, nz)
-  Lines p{};
-  p.src = f->rho; p.dst = f->spec_a;
+  Lines g{}, p{};
+  // ---- x: lines (j<=ny, k<=nz) of G's corner difference -> green, and
+  // rho (nx,ny,nz) real -> A (kx of ld, ny, nz)
+  g.src = f->corner; g.dst = f->green;
+  g.tx = nx + 2; g.ty = ny + 2;
+  g.nf = ny + 1; g.ns = nz + 1;
+  g.df = kx; g.ds = (int64_t)kx * (ny + 1); g.de = 1;
+  g.L = mx; g.Lin = g.L; g.Lout = nx + 1; g.out_scale = 1.0;
+  p.src = FX ? (const void *)f->rho_fx : f->rho; p.dst = f->spec_a;
+  p.rho = f->rho; p.fx_inv = f->rho_scale / f->fixed_scale;
   p.nf = ny; p.ns = nz;
   p.sf = nx; p.ss = (int64_t)nx * ny; p.se = 1;
   p.df = ld; p.ds = ld * ny; p.de = 1;
   p.L = mx; p.Lin = nx; p.Lout = kx; p.out_scale = 1.0;
-  IZH_CHECK((run_lines<T, kLoadReal, kStoreCplx, false, true>(fs, p, f->tw_x, false)));
-  // ---- forward y: A -> B (kx of ld, my, nz)
+  IZH_CHECK((run_two<T, kLoadIgf, FX ? kLoadFx : kLoadReal, kStoreCplx, true>(fs, g, p,
+                                                                            f->tw_x)));
+  // ---- y: lines (i<=nx, k<=nz) of green -> green_t, and A -> B (kx of ld, my, nz)
+  g.src = f->green; g.dst = f->green_t;
+  g.nf = kx; g.ns = nz + 1;
+  g.sf = 1; g.ss = (int64_t)kx * (ny + 1); g.se = kx;
+  g.df = 1; g.ds = (int64_t)kx * (ny + 1); g.de = kx;
+  g.L = my; g.Lin = g.L; g.Lout = ny + 1;
   p.src = f->spec_a; p.dst = f->spec_b;
   p.nf = ld; p.nfv = kx; p.ns = nz;
   p.sf = 1; p.ss = ld * ny; p.se = ld;
   p.df = 1; p.ds = ld * my; p.de = ld;
   p.L = my; p.Lin = ny; p.Lout = my;
-  IZH_CHECK((run_lines<T, kLoadCplx, kStoreCplx, false>(fs, p, f->tw_y, false)));
+  IZH_CHECK((run_two<T, kLoadEven, kLoadCplx, kStoreCplx, false>(fs, g, p, f->tw_y)));
+  // ---- z of G: lines (i<=nx, j<=ny); green_t -> green, scaled by
+  // 1/(mx my mz).  G^ is stored [j][k][i] with i rows at the spectra's pitch
+  // ldx: the fused z pass of a block of x lines then reads, for its one y
+  // index, aligned runs of neighbouring i at neighbouring k, one contiguous
+  // region of ldx*(nz+1) values instead of one value run per z plane.
+  g.src = f->green_t; g.dst = f->green;
+  g.nf = kx; g.ns = ny + 1;
+  g.sf = 1; g.ss = kx; g.se = (int64_t)kx * (ny + 1);
+  g.df = 1; g.ds = ld * (nz + 1); g.de = ld;
+  g.L = mz; g.Lin = g.L; g.Lout = nz + 1;
+  g.out_scale = 1.0 / ((double)mx * my * mz);
+  IZH_CHECK((run_lines<T, kLoadEven, kStoreReal, false, true>(fs, g, f->tw_z, false)));
   // ---- z: FFT, * G^, IFFT, keep k < nz; in place in B
   p.src = f->spec_b; p.dst = f->spec_b;
   p.nf = ld; p.nfv = kx; p.ns = my;
@@ -1085,6 +1210,7 @@ int field_alloc(izh_field *f) {
   const int64_t row = 128 / (2 * (int64_t)es);
   f->ldx = (kx + row - 1) / row * row;
   IZH_HIP(hipMalloc((void **)&f->rho_fx, g * sizeof(unsigned long long)));
+  IZH_HIP(hipMemset(f->rho_fx, 0, g * sizeof(unsigned long long)));
   IZH_HIP(hipMalloc(&f->rho, g * es));
   IZH_HIP(hipMalloc(&f->phi, g * es));
   IZH_HIP(hipMalloc(&f->e, 4 * g * es));
@@ -1118,53 +1244,67 @@ int field_set_domain(izh_field *f, const izh_compdom *dom) {
   return IZH_OK;
 }
 
-// Zero the accumulator, deposit, convert to the grid type.  With a chunk
-// list (the fused run) the positions are the t-frame buffer (T) of the
-// tile-sorted bunch; without one, the bunch's own rows (t frame, FP64) in
-// chunks of kChunk consecutive particles.
+// The grid value of the charge a deposit accumulates, FP64: charge itself;
+// mixed: charge / sum|w| (O(1) values).
+static void deposit_scales(const izh_bunch *b, izh_field *f) {
+  f->fixed_scale = fixed_point_scale(b->wabs_sum);
+  const double wsum = b->wabs_sum > 0 ? b->wabs_sum : 1.0;
+  f->rho_scale = f->precision == IZH_FP64 ? 1.0 : 1.0 / wsum;
+}
+
+// The fused run's deposit: the t positions (T) of the tile-sorted bunch, by
+// its chunk list, into the (cleared) fixed-point accumulator, and in the same
+// launch the corners of the step's Green function; launch_convolve_fx
+// follows and leaves rho, the cleared accumulator and phi.
 int launch_deposit(izh_bunch *b, izh_field *f, const Chunk *chunks, const KeyGrid *kgrid,
                    const int64_t *d_nchunks, int64_t max_chunks) {
-  f->fixed_scale = fixed_point_scale(b->wabs_sum);
+  if (!chunks || !kgrid || max_chunks < 1)
+    return fail(IZH_ERR_ARG, "deposit: no chunk list or key grid");
+  deposit_scales(b, f);
   // every contribution is at most |w| * scale: below 2^50 the fused
   // deposit rounds with the short form
   const bool fast = b->wabs_max * f->fixed_scale < 0x1p50;
-  hipLaunchKernelGGL(k_zero_u64, dim3(grid_for(f->g)), dim3(kBlock), 0, f->stream,
-                     f->rho_fx, f->g);
-  if (max_chunks > 0) {
+  ScopedTimer tm_(IZH_T_DEPOSIT, f->stream);
+  const int s0 = tile_shift(f->nx), s1 = tile_shift(f->ny), s2 = tile_shift(f->nz);
+  const int tnx = f->nx >> s0, tny = f->ny >> s1;
+  int64_t *spill = b->d_scal ? &b->d_scal->overflow : nullptr;
+  const int64_t nc = (int64_t)(f->nx + 2) * (f->ny + 2) * (f->nz + 2);
+  const int ncorner = (grid_for(nc, kDepThreads) + 7) & ~7;
+  const auto go = [&](auto kern, const auto *tp) {
+    hipLaunchKernelGGL(kern, dim3((unsigned)(ncorner + max_chunks)), dim3(kDepThreads), 0,
+                       f->stream, tp, tp + b->cap, tp + 2 * b->cap, b->orig, b->w0, b->w_value,
+                       b->w_uniform, chunks, d_nchunks, kgrid, f->d_dom, f->nx, f->ny, f->nz,
+                       s0, s1, s2, tnx, tny, f->fixed_scale, f->rho_fx, spill, f->corner,
+                       ncorner);
+  };
+  if (f->precision == IZH_MIXED) {
+    const float *tp = (const float *)b->tpos;
+    if (fast) go(k_deposit_tiles<float, true>, tp);
+    else go(k_deposit_tiles<float, false>, tp);
+  } else {
+    const double *tp = (const double *)b->tpos;
+    if (fast) go(k_deposit_tiles<double, true>, tp);
+    else go(k_deposit_tiles<double, false>, tp);
+  }
+  IZH_HIP(hipGetLastError());
+  f->have_rho = 0;
+  f->have_phi = 0;
+  return IZH_OK;
+}
+
+// izh_charge: the bunch's own rows (t frame, FP64) in chunks of kChunk
+// consecutive particles, then the grid charge.
+int launch_deposit_granular(izh_bunch *b, izh_field *f) {
+  deposit_scales(b, f);
+  const int64_t nch = (b->n + kChunk - 1) / kChunk;
+  if (nch > 0) {
     ScopedTimer tm_(IZH_T_DEPOSIT, f->stream);
-    if (chunks) {
-      // the fused run: chunks of the tile-sorted bunch, t positions in T
-      if (!kgrid) return fail(IZH_ERR_ARG, "deposit: chunk list without its key grid");
-      const int s0 = tile_shift(f->nx), s1 = tile_shift(f->ny), s2 = tile_shift(f->nz);
-      const int tnx = f->nx >> s0, tny = f->ny >> s1;
-      int64_t *spill = b->d_scal ? &b->d_scal->overflow : nullptr;
-      const auto go = [&](auto kern, const auto *tp) {
-        hipLaunchKernelGGL(kern, dim3((unsigned)max_chunks), dim3(kDepThreads), 0, f->stream, tp,
-                           tp + b->cap, tp + 2 * b->cap, b->orig, b->w0, b->w_value,
-                           b->w_uniform, chunks, d_nchunks, kgrid, f->d_dom, f->nx, f->ny,
-                           f->nz, s0, s1, s2, tnx, tny, f->fixed_scale, f->rho_fx, spill);
-      };
-      if (f->precision == IZH_MIXED) {
-        const float *tp = (const float *)b->tpos;
-        if (fast) go(k_deposit_tiles<float, true>, tp);
-        else go(k_deposit_tiles<float, false>, tp);
-      } else {
-        const double *tp = (const double *)b->tpos;
-        if (fast) go(k_deposit_tiles<double, true>, tp);
-        else go(k_deposit_tiles<double, false>, tp);
-      }
-    } else {
-      // one call's bunch in the t frame, in its own (unsorted) order
-      hipLaunchKernelGGL(k_deposit_chunks<double>, dim3((unsigned)max_chunks),
-                         dim3(kBlock), 0, f->stream, b->r[0], b->r[2], b->r[4],
-                         b->orig, b->w0, b->w_value, b->w_uniform, b->n, f->d_dom,
-                         f->nx, f->ny, f->nz, f->fixed_scale, f->rho_fx);
-    }
+    hipLaunchKernelGGL(k_deposit_chunks<double>, dim3((unsigned)nch), dim3(kBlock), 0,
+                       f->stream, b->r[0], b->r[2], b->r[4], b->orig, b->w0, b->w_value,
+                       b->w_uniform, b->n, f->d_dom, f->nx, f->ny, f->nz, f->fixed_scale,
+                       f->rho_fx);
     IZH_HIP(hipGetLastError());
   }
-  // FP64: the grid holds charge itself; mixed: charge / sum|w| (O(1) values)
-  double wsum = b->wabs_sum > 0 ? b->wabs_sum : 1.0;
-  f->rho_scale = f->precision == IZH_FP64 ? 1.0 : 1.0 / wsum;
   const double inv = f->rho_scale / f->fixed_scale;
   if (f->precision == IZH_FP64)
     hipLaunchKernelGGL(k_fx_to_grid<double>, dim3(grid_for(f->g)), dim3(kBlock), 0,
@@ -1178,24 +1318,25 @@ int launch_deposit(izh_bunch *b, izh_field *f, const Chunk *chunks, const KeyGri
   return IZH_OK;
 }
 
-int launch_deposit_granular(izh_bunch *b, izh_field *f) {
-  const int64_t nch = (b->n + kChunk - 1) / kChunk;
-  return launch_deposit(b, f, nullptr, nullptr, nullptr, nch);
-}
-
-int launch_green(izh_field *f, hipStream_t gs) {
-  return f->precision == IZH_FP64 ? green_t<double>(f, gs) : green_t<float>(f, gs);
-}
-
-int launch_convolve(izh_field *f) {
-  int rc = f->precision == IZH_FP64 ? convolve_t<double>(f) : convolve_t<float>(f);
-  if (rc == IZH_OK) f->have_phi = 1;
+int launch_convolve_fx(izh_field *f) {
+  const int rc = f->precision == IZH_FP64 ? convolve_t<double, true>(f)
+                                          : convolve_t<float, true>(f);
+  if (rc == IZH_OK) f->have_rho = f->have_phi = 1;
   return rc;
 }
 
 int launch_solve(izh_field *f) {
-  const int rc = launch_green(f, f->stream);
-  return rc == IZH_OK ? launch_convolve(f) : rc;
+  {
+    ScopedTimer tm_(IZH_T_GREEN, f->stream);
+    const int nc = (f->nx + 2) * (f->ny + 2) * (f->nz + 2);
+    hipLaunchKernelGGL(k_igf_corner, dim3(grid_for(nc)), dim3(kBlock), 0, f->stream,
+                       f->corner, f->nx + 2, f->ny + 2, f->nz + 2, f->d_dom);
+    IZH_HIP(hipGetLastError());
+  }
+  const int rc = f->precision == IZH_FP64 ? convolve_t<double, false>(f)
+                                          : convolve_t<float, false>(f);
+  if (rc == IZH_OK) f->have_phi = 1;
+  return rc;
 }
 
 int launch_efield(izh_field *f) {

@@ -2,6 +2,7 @@
 changes its form: tile counts around the limits of the LDS key histograms,
 deposit chunks of every length, grids narrower than the deposit's window.  The bar is the fused run's own: 1e-10
 relative in the diagnostics and the particles."""
+import numpy as np
 import pytest
 
 from conftest import col_err, full_row_err
@@ -46,3 +47,47 @@ def test_key_histograms(gpu, n, grid, period):
 ])
 def test_deposit_chunks(gpu, n, grid, period):
     run_against_step(gpu, n, grid, period, steps=3)
+
+
+def open_potential(rho, h):
+    """The open-boundary potential of rho[k][j][i] in numpy FP64: the doubled
+    convolution with the integrated Green function."""
+    nz, ny, nx = rho.shape
+    ax = [np.arange(n + 2) * d - d / 2.0 for n, d in zip((nx, ny, nz), h)]
+    x, y, z = ax[0][None, None, :], ax[1][None, :, None], ax[2][:, None, None]
+    r = np.sqrt(x * x + y * y + z * z)
+    t = (-z * z * np.arctan(x * y / (z * r)) - y * y * np.arctan(x * z / (y * r))
+         - x * x * np.arctan(y * z / (x * r))) / 2.0
+    t += y * z * np.log(x + r) + x * z * np.log(y + r) + x * y * np.log(z + r)
+    g = np.diff(np.diff(np.diff(t, axis=0), axis=1), axis=2) / (h[0] * h[1] * h[2])
+
+    def fold(n):
+        m = np.arange(2 * n)
+        return np.where(m <= n, m, 2 * n - m)
+    g = g[np.ix_(fold(nz), fold(ny), fold(nx))]
+    s = (2 * nz, 2 * ny, 2 * nx)
+    return np.fft.irfftn(np.fft.rfftn(g) * np.fft.rfftn(rho, s=s), s=s)[:nz, :ny, :nx]
+
+
+@pytest.mark.parametrize("grid", [(4, 4, 4), (8, 64, 4), (128, 8, 16), (16, 256, 8),
+                                  (4, 32, 128), (64, 16, 512), (512, 4, 8)])
+def test_solve_line_lengths(gpu, grid):
+    """The transforms of G and of the charge at every kind of line length:
+    runtime and compile-time, one block's worth and more, along each axis.
+    FP64 within 1e-10 of the maximum; the mixed form's FP32 transforms
+    round each of their about 3 log2(8 g) stages to 6e-8, so 1e-5 bounds
+    them."""
+    print(f"solve {grid}", flush=True)
+    nx, ny, nz = grid
+    h = (1.0e-3, 0.8e-3, 2.0e-3)
+    rho = np.random.default_rng(5).random((nz, ny, nx))
+    want = open_potential(rho, h)
+    for prec, tol in ((gpu.FP64, TOL), (gpu.MIXED, 1e-5)):
+        f = gpu.FieldQuant(*grid, precision=prec)
+        d = gpu.CompDom(*grid)
+        d.set([0, h[0] * (nx - 1), 0, h[1] * (ny - 1), 0, h[2] * (nz - 1)], h)
+        f.upload_rho(rho)
+        f.update3O(d)
+        err = np.max(np.abs(f.download(gpu.PHI) - want)) / np.max(np.abs(want))
+        f.close()
+        assert err < tol, (prec, err)
