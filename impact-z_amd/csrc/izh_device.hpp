@@ -21,6 +21,43 @@ __device__ inline double wave_min(double v) {
   return v;
 }
 
+// Reductions over the 16-lane rows of a wavefront by DPP rotations.  A block
+// reduces each value within its rows and combines the rows through LDS: three
+// or four rotations (two moves and an add each) and one LDS word per row,
+// where a reduction over the wavefront by shuffles makes twelve LDS permutes
+// per value.  The 44 moments cost a block of the fused pass about 540 of
+// those per wavefront, 5-8 us beside 2-3 us per group of particles: 100k
+// particles on 32^3 (one group per block) passed in 27 us.
+template <int N>
+__device__ inline double row_rotate(double v) {
+  const int lo = __double2loint(v), hi = __double2hiint(v);
+  const int slo = __builtin_amdgcn_update_dpp(0, lo, 0x120 + N, 0xF, 0xF, false);
+  const int shi = __builtin_amdgcn_update_dpp(0, hi, 0x120 + N, 0xF, 0xF, false);
+  return __hiloint2double(shi, slo);
+}
+// over the row's lanes of this lane's parity
+__device__ inline double row_sum_parity(double v) {
+  v += row_rotate<8>(v);
+  v += row_rotate<4>(v);
+  return v + row_rotate<2>(v);
+}
+__device__ inline double row_max_parity(double v) {
+  v = fmax(v, row_rotate<8>(v));
+  v = fmax(v, row_rotate<4>(v));
+  return fmax(v, row_rotate<2>(v));
+}
+// over the whole row
+__device__ inline double row_sum(double v) {
+  v = row_sum_parity(v);
+  return v + row_rotate<1>(v);
+}
+__device__ inline double row_max(double v) {
+  v = row_max_parity(v);
+  return fmax(v, row_rotate<1>(v));
+}
+__device__ inline double row_min(double v) { return -row_max(-v); }
+constexpr int kRows = kBlock / 16;  // DPP rows of a kBlock block
+
 // diagnostic1_Output sums (src/Contrl/Output.f90:119-199) in the reference's
 // tmplc order, then |x|,|px|,|y|,|py|,|z|,|pz| maxima and max(x^2+y^2).
 struct Mom {
@@ -59,26 +96,27 @@ __device__ inline void mom_add(Mom &a, double x, double px, double y, double py,
 }
 
 // Block-reduce a per-thread accumulator and store kMoments values at out
-// (sums, then maxima).  sh: [blockDim/64][kMoments] in LDS.
+// (sums, then maxima).  sh: [kRows][kMoments] in LDS; kBlock threads.
 __device__ inline void mom_block_store(const Mom &a, double (*sh)[kMoments],
                                        double *out) {
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int nw = blockDim.x >> 6;
+  const int row = threadIdx.x >> 4;
+  const bool first = (threadIdx.x & 15) == 0;
 #pragma unroll
   for (int k = 0; k < 37; k++) {
-    double v = wave_sum(a.s[k]);
-    if (lane == 0) sh[wv][k] = v;
+    const double v = row_sum(a.s[k]);
+    if (first) sh[row][k] = v;
   }
 #pragma unroll
   for (int k = 0; k < 7; k++) {
-    double v = wave_max(a.m[k]);
-    if (lane == 0) sh[wv][37 + k] = v;
+    const double v = row_max(a.m[k]);
+    if (first) sh[row][37 + k] = v;
   }
   __syncthreads();
   if ((int)threadIdx.x < kMoments) {
     int k = threadIdx.x;
     double r = sh[0][k];
-    for (int w = 1; w < nw; w++) r = (k < 37) ? r + sh[w][k] : fmax(r, sh[w][k]);
+#pragma unroll
+    for (int w = 1; w < kRows; w++) r = (k < 37) ? r + sh[w][k] : fmax(r, sh[w][k]);
     out[k] = r;
   }
 }
@@ -147,47 +185,42 @@ __device__ inline void pmom_add(PairMom &a, double x, double px, double y, doubl
 }
 
 // Block-reduce PairMom into the kMoments values of Mom's layout, value k at
-// out[k * ostride].  sh: [blockDim/64][kMoments] in LDS.
+// out[k * ostride].  sh: [kRows][kMoments] in LDS; kBlock threads.
 __device__ inline void pmom_block_store(const PairMom &a, double (*sh)[kMoments],
                                         double *out, int64_t ostride) {
   constexpr int kx[14] = {0, 6, 15, 16, 12, 27, 28, 29, 30, 31, 1, 7, 17, 18};
   constexpr int ky[14] = {2, 8, 19, 20, 13, 32, 33, 34, 35, 36, 3, 9, 21, 22};
   constexpr int kz[4] = {4, 10, 23, 24}, kp[4] = {5, 11, 25, 26};
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int nw = blockDim.x >> 6;
-  const bool odd = lane & 1;
+  constexpr int kme[3] = {37, 38, 41}, kmo[3] = {39, 40, 42};
+  // the first even and the first odd lane of each row store its two planes
+  const int row = threadIdx.x >> 4, col = threadIdx.x & 15;
+  const bool odd = col & 1, store = col < 2;
 #pragma unroll
   for (int k = 0; k < 14; k++) {
-    const double e = wave_sum(odd ? 0.0 : a.p[k]);
-    const double o = wave_sum(odd ? a.p[k] : 0.0);
-    if (lane == 0) { sh[wv][kx[k]] = e; sh[wv][ky[k]] = o; }
+    const double v = row_sum_parity(a.p[k]);
+    if (store) sh[row][odd ? ky[k] : kx[k]] = v;
   }
 #pragma unroll
   for (int k = 0; k < 4; k++) {
-    const double e = wave_sum(odd ? 0.0 : a.w[k]);
-    const double o = wave_sum(odd ? a.w[k] : 0.0);
-    if (lane == 0) { sh[wv][kz[k]] = e; sh[wv][kp[k]] = o; }
+    const double v = row_sum_parity(a.w[k]);
+    if (store) sh[row][odd ? kp[k] : kz[k]] = v;
   }
-  {
-    const double v = wave_sum(a.zp);
-    if (lane == 0) sh[wv][14] = v;
-  }
-  constexpr int kme[3] = {37, 38, 41}, kmo[3] = {39, 40, 42};
 #pragma unroll
   for (int k = 0; k < 3; k++) {
-    const double e = wave_max(odd ? 0.0 : a.m[k]);
-    const double o = wave_max(odd ? a.m[k] : 0.0);
-    if (lane == 0) { sh[wv][kme[k]] = e; sh[wv][kmo[k]] = o; }
+    const double v = row_max_parity(a.m[k]);
+    if (store) sh[row][odd ? kmo[k] : kme[k]] = v;
   }
-  {
-    const double v = wave_max(a.m[3]);
-    if (lane == 0) sh[wv][43] = v;
+  const double zp = row_sum(a.zp), r2 = row_max(a.m[3]);
+  if (col == 0) {
+    sh[row][14] = zp;
+    sh[row][43] = r2;
   }
   __syncthreads();
   if ((int)threadIdx.x < kMoments) {
     const int k = threadIdx.x;
     double r = sh[0][k];
-    for (int w = 1; w < nw; w++) r = (k < 37) ? r + sh[w][k] : fmax(r, sh[w][k]);
+#pragma unroll
+    for (int w = 1; w < kRows; w++) r = (k < 37) ? r + sh[w][k] : fmax(r, sh[w][k]);
     out[k * ostride] = r;
   }
 }
@@ -235,10 +268,10 @@ __device__ inline void cic8_e4(const E4<T> *__restrict__ e, int64_t o, int64_t s
           o, sy, sz, ab, cd, ef, gx, gy, gz);
 }
 
-// Single-block reduction of per-block partials (nq <= 64 quantities each) in
-// a fixed tree order; bit q of min_mask / max_mask selects min / max for
-// quantity q, sums otherwise.
-__global__ void __launch_bounds__(1024)
+// Reduction of per-block partials (nq quantities each), one block of kBlock
+// threads per quantity, in a fixed tree order; bit q of min_mask / max_mask
+// selects min / max for quantity q, sums otherwise.
+__global__ void __launch_bounds__(kBlock)
 k_reduce_partials(const double *__restrict__ part, int nparts, int nq,
                   unsigned long long min_mask, unsigned long long max_mask,
                   double *__restrict__ out);

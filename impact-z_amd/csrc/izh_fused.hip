@@ -834,7 +834,7 @@ __global__ void __launch_bounds__(kBlock, (pass_blocks_per_cu<T, MODE, KB>(KA)))
       if (v) atomicAdd(&c.hist_new[t], v);
     }
   }
-  __shared__ double sh[kBlock / 64][kMoments];
+  __shared__ double sh[kRows][kMoments];
   // partials are quantity-major: value q of block b at part[q * kMaxRedBlocks + b]
   double *out = c.part + blockIdx.x;
   if (has_kick) {
@@ -843,18 +843,18 @@ __global__ void __launch_bounds__(kBlock, (pass_blocks_per_cu<T, MODE, KB>(KA)))
     out[(int64_t)threadIdx.x * kMaxRedBlocks] = 0.0;
   }
   __syncthreads();
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   double v[kConvRed];
-  for (int k = 0; k < 3; k++) { v[k] = wave_min(mn[k]); v[3 + k] = wave_max(mxv[k]); }
-  v[6] = wave_sum((double)nlost);
-  v[7] = wave_sum((double)nalive);
-  if (lane == 0)
-    for (int k = 0; k < kConvRed; k++) sh[wv][k] = v[k];
+  for (int k = 0; k < 3; k++) { v[k] = row_min(mn[k]); v[3 + k] = row_max(mxv[k]); }
+  v[6] = row_sum((double)nlost);
+  v[7] = row_sum((double)nalive);
+  if ((threadIdx.x & 15) == 0)
+    for (int k = 0; k < kConvRed; k++) sh[threadIdx.x >> 4][k] = v[k];
   __syncthreads();
   if (threadIdx.x < kConvRed) {
     int k = threadIdx.x;
     double r = sh[0][k];
-    for (int w = 1; w < kBlock / 64; w++)
+#pragma unroll
+    for (int w = 1; w < kRows; w++)
       r = k < 3 ? fmin(r, sh[w][k]) : (k < 6 ? fmax(r, sh[w][k]) : r + sh[w][k]);
     out[(int64_t)(kMoments + k) * kMaxRedBlocks] = r;
   }
@@ -919,17 +919,16 @@ k_prologue_range(const double *__restrict__ X, const double *__restrict__ PX,
     double p[3] = {X[i] * xl, Y[i] * xl, -gam * betai * wrap_phase(PH[i]) * xl};
     for (int a = 0; a < 3; a++) { mn[a] = fmin(mn[a], p[a]); mx[a] = fmax(mx[a], p[a]); }
   }
-  __shared__ double sh[kBlock / 64][6];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  __shared__ double sh[kRows][6];
   double v[6];
-  for (int a = 0; a < 3; a++) { v[a] = wave_min(mn[a]); v[3 + a] = wave_max(mx[a]); }
-  if (lane == 0)
-    for (int k = 0; k < 6; k++) sh[wv][k] = v[k];
+  for (int a = 0; a < 3; a++) { v[a] = row_min(mn[a]); v[3 + a] = row_max(mx[a]); }
+  if ((threadIdx.x & 15) == 0)
+    for (int k = 0; k < 6; k++) sh[threadIdx.x >> 4][k] = v[k];
   __syncthreads();
   if (threadIdx.x < 6) {
     int k = threadIdx.x;
     double r = sh[0][k];
-    for (int w = 1; w < kBlock / 64; w++) r = k < 3 ? fmin(r, sh[w][k]) : fmax(r, sh[w][k]);
+    for (int w = 1; w < kRows; w++) r = k < 3 ? fmin(r, sh[w][k]) : fmax(r, sh[w][k]);
     part[blockIdx.x * 6 + k] = r;
   }
 }
@@ -1035,41 +1034,69 @@ struct FinCfg {
   const double *prologue_box;  // mode 0: the box k_prologue_keys used
 };
 
-__global__ void __launch_bounds__(1024) k_finalize(FinCfg f) {
+// One block, so its time is a chain of latencies: every wavefront issues the
+// loads of all its quantities before it reduces any, the scalars the step
+// updates are read before the reduction, and the tile scan runs in wavefronts
+// (two barriers) instead of a tree over the block (twenty).
+constexpr int kFinThreads = 1024;
+
+__global__ void __launch_bounds__(kFinThreads) k_finalize(FinCfg f) {
   __shared__ double red[kPartStride];
-  __shared__ uint32_t ssum[1024];
-  __shared__ uint32_t csum[1024];
+  __shared__ uint32_t wsum[kFinThreads / 64][2];
   const int tid = threadIdx.x;
-  // ---- reduce the pass partials: one wavefront per quantity, fixed order
+  const int lane = tid & 63, wv = tid >> 6;
+  constexpr int kWaves = kFinThreads / 64;
+  DevScal S0{};
+  if (tid == 0) S0 = *f.scal;
+  const int64_t rec = f.scal->rec;
+  // ---- reduce the pass partials: kPartStride / kWaves quantities per
+  // wavefront, fixed order
   if (f.mode != 0) {
-    const int lane = tid & 63, wv = tid >> 6, nw = blockDim.x >> 6;
-    for (int q = wv; q < kPartStride; q += nw) {
-      const bool isconv = q >= kMoments;
+    constexpr int kQ = (kPartStride + kWaves - 1) / kWaves;
+    constexpr int kU = 8;  // loads in flight per lane and quantity
+    const auto op_of = [](int q) {
       const int cq = q - kMoments;
-      const int op = !isconv ? (q < 37 ? 0 : 2) : (cq < 3 ? 1 : (cq < 6 ? 2 : 0));
-      const double ident = op == 1 ? 1e300 : (op == 2 ? -1e300 : 0.0);
-      double acc = ident;
-      // eight loads in flight per lane, combined in slot order
-      constexpr int kU = 8;
-      const double *src = f.part + (int64_t)q * kMaxRedBlocks;
-      for (int b0 = lane; b0 < f.nparts; b0 += 64 * kU) {
-        double v[kU];
+      return q < kMoments ? (q < 37 ? 0 : 2) : (cq < 3 ? 1 : (cq < 6 ? 2 : 0));
+    };
+    const auto ident_of = [](int op) { return op == 1 ? 1e300 : (op == 2 ? -1e300 : 0.0); };
+    double acc[kQ];
+#pragma unroll
+    for (int i = 0; i < kQ; i++) acc[i] = ident_of(op_of(wv + kWaves * i));
+    for (int b0 = lane; b0 < f.nparts; b0 += 64 * kU) {
+      double v[kQ][kU];
+#pragma unroll
+      for (int i = 0; i < kQ; i++) {
+        const int q = wv + kWaves * i;
+        const double *src = f.part + (int64_t)min(q, kPartStride - 1) * kMaxRedBlocks;
 #pragma unroll
         for (int u = 0; u < kU; u++) {
           const int b = b0 + 64 * u;
-          v[u] = b < f.nparts ? src[b] : ident;
+          v[i][u] = b < f.nparts ? src[b] : ident_of(op_of(q));
         }
+      }
+#pragma unroll
+      for (int i = 0; i < kQ; i++) {
+        const int op = op_of(wv + kWaves * i);
 #pragma unroll
         for (int u = 0; u < kU; u++)
-          acc = op == 1 ? fmin(acc, v[u]) : (op == 2 ? fmax(acc, v[u]) : acc + v[u]);
+          acc[i] = op == 1 ? fmin(acc[i], v[i][u])
+                           : (op == 2 ? fmax(acc[i], v[i][u]) : acc[i] + v[i][u]);
       }
-      acc = op == 1 ? wave_min(acc) : (op == 2 ? wave_max(acc) : wave_sum(acc));
-      if (lane == 0) red[q] = acc;
+    }
+#pragma unroll
+    for (int i = 0; i < kQ; i++) {
+      const int q = wv + kWaves * i, op = op_of(q);
+      const double r = op == 1 ? wave_min(acc[i]) : (op == 2 ? wave_max(acc[i])
+                                                             : wave_sum(acc[i]));
+      if (lane == 0 && q < kPartStride) red[q] = r;
     }
     __syncthreads();
+    // the record of the step just finished; its last value is Npt
+    if (f.want_moments && tid <= kMoments)
+      f.moments[rec * kRunRecord + tid] = red[tid < kMoments ? tid : kMoments + 7];
   }
   if (tid == 0) {
-    DevScal &S = *f.scal;
+    DevScal S = S0;
     // the keys the pass just wrote were computed in the domain as it stands
     // before this step's update; k_prologue_keys used the unpadded box
     if (f.scan) {
@@ -1081,12 +1108,7 @@ __global__ void __launch_bounds__(1024) k_finalize(FinCfg f) {
         D.kgrid[f.kg].h[a] = f.mode == 0 ? (pb[3 + a] - pb[a]) / nn[a] : D.msize[a];
       }
     }
-    if (f.mode != 0 && f.want_moments) {
-      double *o = f.moments + S.rec * kRunRecord;
-      for (int k = 0; k < kMoments; k++) o[k] = red[k];
-      o[kMoments] = red[kMoments + 7];  // Npt of those moments
-      S.rec++;
-    }
+    if (f.mode != 0 && f.want_moments) S.rec++;
     if (f.mode == 1) {
       const double *cv = red + kMoments;
       const int64_t alive_in = (int64_t)cv[7];
@@ -1135,12 +1157,20 @@ __global__ void __launch_bounds__(1024) k_finalize(FinCfg f) {
       // prologue: the input slots are the uploaded particles
       S.nslots = S.nalive;
     }
+    // the chunk counts are written below, overflow and err by other kernels
+    DevScal &G = *f.scal;
+    G.current = S.current;
+    G.npt = S.npt;
+    G.xycon = S.xycon;
+    G.tcon = S.tcon;
+    G.nalive = S.nalive;
+    G.nslots = S.nslots;
+    G.rec = S.rec;
   }
-  __syncthreads();
   if (!f.scan) return;
   // ---- exclusive scan of the tile histogram and the chunk list (after the
   // last pass: of the keys the next run starts from)
-  const int per = (f.ntiles + blockDim.x - 1) / blockDim.x;
+  const int per = (f.ntiles + kFinThreads - 1) / kFinThreads;
   const int t0 = tid * per, t1 = min(t0 + per, f.ntiles);
   uint32_t cnt = 0, nch = 0;
   for (int t = t0; t < t1; t++) {
@@ -1148,18 +1178,20 @@ __global__ void __launch_bounds__(1024) k_finalize(FinCfg f) {
     cnt += h;
     nch += (h + f.chunk - 1) / f.chunk;
   }
-  ssum[tid] = cnt;
-  csum[tid] = nch;
-  __syncthreads();
-  for (int off = 1; off < (int)blockDim.x; off <<= 1) {
-    uint32_t a = tid >= off ? ssum[tid - off] : 0u;
-    uint32_t b2 = tid >= off ? csum[tid - off] : 0u;
-    __syncthreads();
-    ssum[tid] += a;
-    csum[tid] += b2;
-    __syncthreads();
+  // inclusive scans within the wavefront, then over the wavefronts' totals
+  uint32_t off = cnt, coff = nch;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const uint32_t a = (uint32_t)__shfl_up((int)off, d, 64);
+    const uint32_t c = (uint32_t)__shfl_up((int)coff, d, 64);
+    if (lane >= d) { off += a; coff += c; }
   }
-  uint32_t off = ssum[tid] - cnt, coff = csum[tid] - nch;
+  if (lane == 63) { wsum[wv][0] = off; wsum[wv][1] = coff; }
+  __syncthreads();
+  for (int w = 0; w < wv; w++) { off += wsum[w][0]; coff += wsum[w][1]; }
+  if (tid == kFinThreads - 1) *f.nchunks = coff;
+  off -= cnt;
+  coff -= nch;
   for (int t = t0; t < t1; t++) {
     uint32_t h = f.hist[t];
     f.cursor[t] = off;
@@ -1171,9 +1203,8 @@ __global__ void __launch_bounds__(1024) k_finalize(FinCfg f) {
     }
     off += h;
   }
-  if (tid == blockDim.x - 1) *f.nchunks = csum[tid];
   __syncthreads();  // hist_zero may be hist itself
-  for (int t = tid; t < f.ntiles; t += blockDim.x) f.hist_zero[t] = 0u;
+  for (int t = tid; t < f.ntiles; t += kFinThreads) f.hist_zero[t] = 0u;
 }
 
 __global__ void k_zero_u32(uint32_t *__restrict__ p, int64_t n) {
@@ -1402,7 +1433,7 @@ struct Runner {
       fc.nchunks = &b->d_scal->nchunks[g_next];
       {
         ScopedTimer tm_(IZH_T_FINAL, st);
-        hipLaunchKernelGGL(k_finalize, dim3(1), dim3(1024), 0, st, fc);
+        hipLaunchKernelGGL(k_finalize, dim3(1), dim3(kFinThreads), 0, st, fc);
       }
       IZH_HIP(hipGetLastError());
     }
@@ -1498,7 +1529,7 @@ struct Runner {
     }
     if (!dry) {
       ScopedTimer tm_(IZH_T_FINAL, st);
-      hipLaunchKernelGGL(k_finalize, dim3(1), dim3(1024), 0, st, fc);
+      hipLaunchKernelGGL(k_finalize, dim3(1), dim3(kFinThreads), 0, st, fc);
       IZH_HIP(hipGetLastError());
     }
     s++;

@@ -66,7 +66,8 @@ def open_potential(rho, h):
         return np.where(m <= n, m, 2 * n - m)
     g = g[np.ix_(fold(nz), fold(ny), fold(nx))]
     s = (2 * nz, 2 * ny, 2 * nx)
-    return np.fft.irfftn(np.fft.rfftn(g) * np.fft.rfftn(rho, s=s), s=s)[:nz, :ny, :nx]
+    return np.fft.irfftn(np.fft.rfftn(g) * np.fft.rfftn(rho, s=s, axes=(0, 1, 2)), s=s,
+                         axes=(0, 1, 2))[:nz, :ny, :nx]
 
 
 @pytest.mark.parametrize("grid", [(4, 4, 4), (8, 64, 4), (128, 8, 16), (16, 256, 8),
