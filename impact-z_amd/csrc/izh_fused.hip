@@ -317,6 +317,22 @@ __device__ inline void wave_count_add(uint32_t *counters, uint32_t key, bool tak
 // two (FP32 in place: three) blocks per CU.
 constexpr int kPassLdsTiles = 1024;
 
+// Blocks of a pass over n slots in ntiles tiles.  512 fill the card (two per
+// CU; FP32 in place three fit): a block then pays its start (chunk search,
+// first gather box) and its reduction once, and k_finalize reads one CU's
+// worth of partials in 9 us where 2048 blocks' take 20.  A bunch over many
+// tiles spreads unevenly, its halo's tiles of few particles changing the
+// gather box most, so large ones take shorter ranges that even out.  Run time
+// per step at 512 / 1024 / 2048 blocks: 500k on 64^3 (FP64) 135 / 147 / 163
+// us, 2M on 64^3 203 / 205 / 219, 4M on 32^3 (mixed) 247 / 260 / 273, 2.3M on
+// 128^3 527 / 510 / 526, 10M on 128x128x256 (mixed) 1198 / 1120 / 1079, 50M
+// (FP64) 4315 / 4044 / 3910.
+inline int pass_blocks(int64_t n, int ntiles) {
+  const int most = ntiles < 1024 || n < 1500000 ? 512 : (n < 4000000 ? 1024 : kMaxRedBlocks);
+  const int64_t groups = (n + kBlock - 1) / kBlock;
+  return ((int)std::min<int64_t>(groups, most) + 7) / 8 * 8;  // as block_range needs
+}
+
 // Slot range of a block: contiguous, and the blocks one XCD receives (block
 // b runs on XCD b mod 8) cover adjacent ranges, so each XCD's L2 holds the
 // field of its own part of the sorted bunch.  gridDim.x is a multiple of 8.
@@ -326,6 +342,30 @@ __device__ inline void block_range(int64_t n, int64_t &lo, int64_t &hi) {
   const int64_t per = ((n + nb - 1) / nb + kBlock - 1) / kBlock * kBlock;
   lo = (int64_t)vb * per;
   hi = lo + per < n ? lo + per : n;
+}
+
+// Last of nch chunks that starts at or before slot lo (0 if none does), by
+// the whole block: each round cuts the candidates into kBlock steps and
+// counts the steps that start at or before lo, so two dependent loads cover
+// 65536 chunks where a binary search makes sixteen.  red: kBlock / 64 words.
+__device__ inline int last_chunk_at(const Chunk *__restrict__ chs, int nch, int64_t lo,
+                                    int *red) {
+  int a = 0, n = nch;
+  while (n > 1) {
+    const int step = (n + kBlock - 1) / kBlock, k = (int)threadIdx.x * step;
+    const bool before = k < n && (int64_t)chs[a + k].start <= lo;
+    const int c = __popcll(__ballot(before));
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = c;
+    __syncthreads();
+    int t = 0;
+#pragma unroll
+    for (int w = 0; w < kBlock / 64; w++) t += red[w];
+    const int at = max(t - 1, 0) * step;
+    a += at;
+    n = min(step, n - at);
+  }
+  return __builtin_amdgcn_readfirstlane(a);
 }
 
 // E of a neighbourhood of the block's current sort tile (kGBoxT nodes
@@ -338,6 +378,14 @@ constexpr int kGBoxL = 12;
 constexpr int kGBoxCells = kGBoxT * kGBoxT * kGBoxL;
 constexpr int kGBoxLowT = 2;  // nodes below the tile's first node, x and y
 constexpr int kGBoxLowL = 2;  // and z
+// A group restages the box only for a tile it has this many slots of: where
+// tiles hold few particles it would restage at every group for a minority of
+// its lanes (10M on 128x128x256, mixed, quadrupole step: 451 -> 419 us).
+constexpr int kStageMin = 192;
+constexpr int kWalk = 8;      // chunk starts read at a time across sparse tiles
+// Nodes a thread loads before it stores them: two rounds of loads per box
+// instead of four (2M on 64^3: 95 -> 91 us a pass).
+constexpr int kBoxBatch = 4;
 
 template <typename T> struct GatherLds;
 template <> struct GatherLds<double> {
@@ -479,39 +527,16 @@ __global__ void __launch_bounds__(kBlock, (pass_blocks_per_cu<T, MODE, KB>(KA)))
   // constant address space: scalar loads, which no vector-memory wait counts.
   using ConstChunk = __attribute__((address_space(4))) const Chunk;
   const ConstChunk *chs = (const ConstChunk *)c.in_chunks;
-  int64_t nch = 0, ci = 0, nxt_start = INT64_MAX;
+  int nch = 0, ci = 0;
+  int64_t nxt_start = INT64_MAX;
   uint32_t cur_tile = kDeadKey;
-  if (has_kick) {
-    nch = *(__attribute__((address_space(4))) const int64_t *)c.in_nchunks;
-    int64_t a = 0, b = nch;  // last chunk starting at or before lo
-    while (b - a > 1) {
-      const int64_t m = (a + b) >> 1;
-      if ((int64_t)chs[m].start <= lo) a = m; else b = m;
-    }
-    ci = a;
-    if (nch > 0) {
-      cur_tile = chs[ci].tile;
-      nxt_start = ci + 1 < nch ? (int64_t)chs[ci + 1].start : INT64_MAX;
-    }
-  }
-
   // Loads of the slot group starting at base (called while lo < hi).  Every
   // lane loads (an index past the range is clamped to its last slot and the
   // lane is marked empty), so no branch skips the loads and the waits for
   // them and for the atomics before them can be counted exactly.
-  auto load = [&](int64_t base, SlotIn &sl) {
+  auto load_rows = [&](int64_t base, SlotIn &sl) {
     const int64_t j = base + threadIdx.x;
     const int64_t jj = j < hi ? j : hi - 1;
-    uint32_t k0 = kDeadKey;
-    if (has_kick && base < hi) {
-      // the next chunk's start is held, so only a crossing loads
-      while (nxt_start <= base) {
-        ci++;
-        cur_tile = chs[ci].tile;
-        nxt_start = ci + 1 < nch ? (int64_t)chs[ci + 1].start : INT64_MAX;
-      }
-      k0 = cur_tile;
-    }
     uint32_t key = 0u, og = 0u;
     if constexpr (kScatter) {
       key = c.in_key[jj];
@@ -522,9 +547,35 @@ __global__ void __launch_bounds__(kBlock, (pass_blocks_per_cu<T, MODE, KB>(KA)))
 #pragma unroll
     for (int k = 0; k < 6; k++) sl.r[k] = c.in[k * cap + jj];
     sl.in = j < hi;
-    sl.k0 = k0;
     sl.key = key;
     sl.orig = og;
+  };
+  auto load = [&](int64_t base, SlotIn &sl) {
+    uint32_t k0 = kDeadKey;
+    if (has_kick && base < hi) {
+      // the next chunk's start is held, so only a crossing loads; between
+      // sparse tiles a group crosses many chunks, eight starts at a time
+      if (nxt_start <= base) {
+        int ahead;
+        do {
+          uint32_t st[kWalk];
+#pragma unroll
+          for (int u = 0; u < kWalk; u++)
+            st[u] = chs[min(ci + 1 + u, nch - 1)].start;
+          ahead = 0;
+#pragma unroll
+          for (int u = 0; u < kWalk; u++)
+            ahead += ci + 1 + u < nch && (int64_t)st[u] <= base ? 1 : 0;
+          ci += ahead;
+        } while (ahead == kWalk);
+        cur_tile = chs[ci].tile;
+        nxt_start = ci + 1 < nch ? (int64_t)chs[ci + 1].start : INT64_MAX;
+      }
+      // a tile with few slots left in the group is not worth a box
+      k0 = nxt_start - base >= kStageMin ? cur_tile : kDeadKey;
+    }
+    sl.k0 = k0;
+    load_rows(base, sl);
   };
 
   auto step = [&](SlotIn &sl, uint32_t k0, int64_t base, int par, auto &&prefetch) {
@@ -603,10 +654,10 @@ __global__ void __launch_bounds__(kBlock, (pass_blocks_per_cu<T, MODE, KB>(KA)))
                      kGBoxLowL, 0), c.nz - bdz);
         __syncthreads();  // the previous box is no longer read
         const int bxy = bdx * bdy, nb = bxy * bdz;
-        for (int q0 = threadIdx.x; q0 < nb; q0 += 2 * kBlock) {
-          E4<T> ev[2];
+        for (int q0 = threadIdx.x; q0 < nb; q0 += kBoxBatch * kBlock) {
+          E4<T> ev[kBoxBatch];
 #pragma unroll
-          for (int u = 0; u < 2; u++) {
+          for (int u = 0; u < kBoxBatch; u++) {
             const int q = q0 + u * kBlock;
             E4<T> v{};
             if (q < nb) {
@@ -616,7 +667,7 @@ __global__ void __launch_bounds__(kBlock, (pass_blocks_per_cu<T, MODE, KB>(KA)))
             ev[u] = v;
           }
 #pragma unroll
-          for (int u = 0; u < 2; u++)
+          for (int u = 0; u < kBoxBatch; u++)
             if (q0 + u * kBlock < nb) box_store(gbox, q0 + u * kBlock, ev[u]);
         }
         __syncthreads();
@@ -814,7 +865,18 @@ __global__ void __launch_bounds__(kBlock, (pass_blocks_per_cu<T, MODE, KB>(KA)))
   // top of the loop can be counted exactly.
   SlotIn sa, sb;
   if (lo < hi) {
-    load(lo, sa);
+    // the first group's rows are on their way while the block finds its chunk
+    load_rows(lo, sa);
+    if (has_kick) {
+      __shared__ int red[kBlock / 64];
+      nch = (int)*(__attribute__((address_space(4))) const int64_t *)c.in_nchunks;
+      if (nch > 0) {
+        ci = last_chunk_at(c.in_chunks, nch, lo, red);
+        cur_tile = chs[ci].tile;
+        nxt_start = ci + 1 < nch ? (int64_t)chs[ci + 1].start : INT64_MAX;
+      }
+    }
+    sa.k0 = nxt_start - lo >= kStageMin ? cur_tile : kDeadKey;
     step(sa, (uint32_t)__builtin_amdgcn_readfirstlane((int)sa.k0), lo, 0,
          [&] { load(lo + kBlock, sb); });
     for (int64_t base = lo + kBlock; base < hi; base += 2 * kBlock) {
@@ -1365,7 +1427,7 @@ struct Runner {
     gam_sc = gam;
     const double wsum = b->wabs_sum > 0 ? b->wabs_sum : 1.0;
     const double rho_scale = f->precision == IZH_FP64 ? 1.0 : 1.0 / wsum;
-    nb = (grid_for(b->n) + 7) / 8 * 8;  // multiple of 8 for block_range
+    nb = pass_blocks(b->n, ntiles);
     period = b->resort_period > 0 ? b->resort_period : kDefaultResortPeriod;
     refpt_after.assign(2 * (size_t)total, 0.0);
     // Two chunk lists (with their key grids and counts) describe groupings

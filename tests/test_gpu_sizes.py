@@ -19,9 +19,18 @@ def run_against_step(gpu, n, grid, period, steps=5, seed=3):
     a = Simulation(pts, B.Beam(), B.fodo(1), grid)
     b = Simulation(pts, B.Beam(), B.fodo(1), grid)
     b.bunch.resort_period = period
-    rows = [a.diag(a.step(e)) for _, e in zip(range(steps), a.segments())]
+    moms, rows = [], []
+    for _, e in zip(range(steps), a.segments()):
+        moms.append(a.step(e))
+        rows.append(a.diag(moms[-1]) if n > 2 else None)
     rec = b.run_fused(steps)
-    worst = max(full_row_err(b.diag(rec[k]), rows[k]) for k in range(steps))
+    # two particles lie on a line of each plane: emittance zero, the derived
+    # columns undefined; their squares, products and maxima still compare
+    pick = list(range(6, 12)) + list(range(37, 44))
+    worst = max(float(np.max(np.abs(rec[k][pick] / moms[k][pick] - 1))) for k in range(steps))
+    if n > 2:
+        worst = max([worst] + [full_row_err(b.diag(rec[k]), rows[k])
+                               for k in range(steps)])
     pe = col_err(b.bunch.getpts(), a.bunch.getpts())
     a.close()
     b.close()
@@ -92,3 +101,15 @@ def test_solve_line_lengths(gpu, grid):
         err = np.max(np.abs(f.download(gpu.PHI) - want)) / np.max(np.abs(want))
         f.close()
         assert err < tol, (prec, err)
+
+
+@pytest.mark.parametrize("n,grid,period", [
+    (2, (8, 8, 8), 1),               # fewer particles than a wavefront
+    (257, (16, 16, 16), 2),          # two blocks, one of a single slot
+    (3_000, (128, 128, 128), 2),     # a group crosses hundreds of tiles
+    (131_073, (64, 64, 128), 3),     # the first bunch of two groups a block
+    (1_500_001, (64, 64, 128), 2),   # the first pass of 1024 blocks
+    (4_000_001, (64, 64, 128), 2),   # and of 2048
+])
+def test_pass_blocks(gpu, n, grid, period):
+    run_against_step(gpu, n, grid, period, steps=3)
