@@ -1129,7 +1129,7 @@ int izh_field_destroy(izh_field *f) {
   if (f->stream) (void)hipStreamSynchronize(f->stream);
   void *bufs[] = {f->rho_fx, f->rho,  f->phi,    f->e,    f->spec_a,
                   f->spec_b, f->green, f->green_t, f->corner, f->tw_x,
-                  f->tw_y,   f->tw_z, f->d_dom,  f->chunks, f->d_wake};
+                  f->tw_y,   f->tw_z, f->d_dom,  f->bin, f->d_wake};
   for (void *p : bufs)
     if (p) (void)hipFree(p);
   if (f->h_dom) (void)hipHostFree(f->h_dom);

@@ -276,6 +276,53 @@ k_reduce_partials(const double *__restrict__ part, int nparts, int nq,
                   unsigned long long min_mask, unsigned long long max_mask,
                   double *__restrict__ out);
 
+// Exclusive scan of a tile histogram by one block of THREADS: cursor[t] = the
+// first slot of tile t, chunks = each tile's slots in runs of at most `chunk`,
+// in tile order, *nchunks their number; hist_zero (hist itself, or the next
+// one) is cleared.  wsum: THREADS / 64 pairs of LDS.
+template <int THREADS>
+__device__ inline void tile_scan(const uint32_t *__restrict__ hist, int ntiles,
+                                 uint32_t chunk, uint32_t *__restrict__ cursor,
+                                 Chunk *__restrict__ chunks, int64_t *__restrict__ nchunks,
+                                 uint32_t *hist_zero, uint32_t (*wsum)[2]) {
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int per = (ntiles + THREADS - 1) / THREADS;
+  const int t0 = tid * per, t1 = min(t0 + per, ntiles);
+  uint32_t cnt = 0, nch = 0;
+  for (int t = t0; t < t1; t++) {
+    const uint32_t h = hist[t];
+    cnt += h;
+    nch += (h + chunk - 1) / chunk;
+  }
+  // inclusive scans within the wavefront, then over the wavefronts' totals
+  uint32_t off = cnt, coff = nch;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const uint32_t a = (uint32_t)__shfl_up((int)off, d, 64);
+    const uint32_t c = (uint32_t)__shfl_up((int)coff, d, 64);
+    if (lane >= d) { off += a; coff += c; }
+  }
+  if (lane == 63) { wsum[wv][0] = off; wsum[wv][1] = coff; }
+  __syncthreads();
+  for (int w = 0; w < wv; w++) { off += wsum[w][0]; coff += wsum[w][1]; }
+  if (tid == THREADS - 1) *nchunks = coff;
+  off -= cnt;
+  coff -= nch;
+  for (int t = t0; t < t1; t++) {
+    const uint32_t h = hist[t];
+    cursor[t] = off;
+    for (uint32_t s = 0; s < h; s += chunk) {
+      chunks[coff].start = off + s;
+      chunks[coff].len = min(chunk, h - s);
+      chunks[coff].tile = (uint32_t)t;
+      coff++;
+    }
+    off += h;
+  }
+  __syncthreads();  // hist_zero may be hist itself
+  for (int t = tid; t < ntiles; t += THREADS) hist_zero[t] = 0u;
+}
+
 int launch_reduce(hipStream_t s, const double *part, int nparts, int nq,
                   unsigned long long min_mask, unsigned long long max_mask,
                   double *out);

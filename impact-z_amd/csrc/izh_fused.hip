@@ -1232,41 +1232,8 @@ __global__ void __launch_bounds__(kFinThreads) k_finalize(FinCfg f) {
   if (!f.scan) return;
   // ---- exclusive scan of the tile histogram and the chunk list (after the
   // last pass: of the keys the next run starts from)
-  const int per = (f.ntiles + kFinThreads - 1) / kFinThreads;
-  const int t0 = tid * per, t1 = min(t0 + per, f.ntiles);
-  uint32_t cnt = 0, nch = 0;
-  for (int t = t0; t < t1; t++) {
-    uint32_t h = f.hist[t];
-    cnt += h;
-    nch += (h + f.chunk - 1) / f.chunk;
-  }
-  // inclusive scans within the wavefront, then over the wavefronts' totals
-  uint32_t off = cnt, coff = nch;
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const uint32_t a = (uint32_t)__shfl_up((int)off, d, 64);
-    const uint32_t c = (uint32_t)__shfl_up((int)coff, d, 64);
-    if (lane >= d) { off += a; coff += c; }
-  }
-  if (lane == 63) { wsum[wv][0] = off; wsum[wv][1] = coff; }
-  __syncthreads();
-  for (int w = 0; w < wv; w++) { off += wsum[w][0]; coff += wsum[w][1]; }
-  if (tid == kFinThreads - 1) *f.nchunks = coff;
-  off -= cnt;
-  coff -= nch;
-  for (int t = t0; t < t1; t++) {
-    uint32_t h = f.hist[t];
-    f.cursor[t] = off;
-    for (uint32_t s = 0; s < h; s += f.chunk) {
-      f.chunks[coff].start = off + s;
-      f.chunks[coff].len = min(f.chunk, h - s);
-      f.chunks[coff].tile = (uint32_t)t;
-      coff++;
-    }
-    off += h;
-  }
-  __syncthreads();  // hist_zero may be hist itself
-  for (int t = tid; t < f.ntiles; t += kFinThreads) f.hist_zero[t] = 0u;
+  tile_scan<kFinThreads>(f.hist, f.ntiles, f.chunk, f.cursor, f.chunks, f.nchunks,
+                         f.hist_zero, wsum);
 }
 
 __global__ void k_zero_u32(uint32_t *__restrict__ p, int64_t n) {

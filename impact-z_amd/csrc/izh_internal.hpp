@@ -42,7 +42,6 @@ constexpr int kPartStride = kMoments + kConvRed;
 constexpr int kChunk = 16384;        // most particles per deposit chunk
 constexpr int kChunkMin = 1024;      // and the smallest such limit
 constexpr int kChunkBlocks = 256;    // chunks a bunch is cut into at least
-constexpr int kWindowCells = 4096;   // LDS deposit window (int64 cells)
 constexpr int kTileShift = 3;        // sort tiles of 8x8x8 cells
 constexpr uint32_t kDeadKey = 0xffffffffu;
 constexpr int kSinkBytes = 64 * 8 * 16;  // one 8-byte word per lane, 16 rows
@@ -201,8 +200,10 @@ struct izh_field {
   void *tw_x = nullptr, *tw_y = nullptr, *tw_z = nullptr;  // twiddles per length
   izh::DevDom *d_dom = nullptr; // domain the kernels read
   izh::DevDom *h_dom = nullptr; // pinned staging for host-set domains
-  izh::Chunk *chunks = nullptr; // uniform chunks for unsorted deposits
-  int64_t nchunks_cap = 0;
+  // izh_charge's bins (launch_deposit_granular), made by its first large bunch
+  char *bin = nullptr;
+  int64_t bin_cap = 0, bin_at_rows = 0;
+  int bin_rows = 0, bin_tiles = 0;
   double rho_scale = 1.0;       // grid value = physical charge * rho_scale
   int have_rho = 0, have_phi = 0;
   double fixed_scale = 0;       // 2^e used by the fixed-point deposit

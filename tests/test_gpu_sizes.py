@@ -113,3 +113,48 @@ def test_solve_line_lengths(gpu, grid):
 ])
 def test_pass_blocks(gpu, n, grid, period):
     run_against_step(gpu, n, grid, period, steps=3)
+
+
+@pytest.mark.parametrize("n,grid", [
+    (4_096, (32, 32, 32)),           # straight to the grid
+    (4_097, (16, 16, 32)),           # the whole grid in LDS: its largest
+    (4_097, (4, 8, 16)),             # and a small one
+    (4_097, (32, 16, 32)),           # binned: 16 tiles
+    (50_001, (128, 64, 16)),         # uneven tiles, a ragged last block
+    (5_000, (128, 256, 256)),        # 16384 tiles of 8 nodes: tiles of 16
+    (4_500, (4, 1024, 8)),           # a tile as wide as the grid
+])
+@pytest.mark.parametrize("uniform", [True, False])
+def test_charge_forms(gpu, n, grid, uniform):
+    """izh_charge against numpy: the contributions, rounded to the deposit's
+    fixed point (2^e with sum |w| 2^e <= 2^61), sum exactly in any order, so
+    what remains is the rounding of the weights and of each contribution:
+    1e-13 of the largest node bounds both."""
+    print(f"charge {n} {grid} uniform {uniform}", flush=True)
+    from impactz import beam as B
+    pts = B.gaussian_bunch(n, seed=8)
+    if not uniform:
+        pts[:, 7] *= np.random.default_rng(9).uniform(0.5, 2.0, n)
+    b = gpu.BeamBunch.from_beam(pts, B.Beam())
+    f = gpu.FieldQuant(*grid)
+    d = gpu.CompDom(*grid)
+    pr, _, _ = b.conv1st(0.0, 1.0, 1.0)
+    d.update(pr)
+    for _ in range(2):               # the second from the scratch the first made
+        b.charge(d, f)
+    rho = f.download(gpu.RHO)
+    p = b.getpts()
+    lo, h = d.range[0::2], d.msize
+    want = np.zeros(grid[0] * grid[1] * grid[2])
+    pos = p[:, [0, 2, 4]]
+    i = ((pos - lo) * (1.0 / h) + 1.0).astype(np.int64)
+    a = ((lo - pos) + i * h) * (1.0 / h)
+    for c in range(8):
+        o = np.array([c & 1, (c >> 1) & 1, c >> 2])
+        w = np.prod(np.where(o, 1.0 - a, a), axis=1) * p[:, 7]
+        k = i - 1 + o
+        np.add.at(want, k[:, 0] + grid[0] * (k[:, 1] + grid[1] * k[:, 2]), w)
+    err = np.max(np.abs(rho.ravel() - want)) / np.max(np.abs(want))
+    b.close()
+    f.close()
+    assert err < 1e-13, err
