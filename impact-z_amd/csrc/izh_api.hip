@@ -106,7 +106,7 @@ static void physconst(double freq, izh_const *c) {
 
 template <typename P>
 static int dmalloc(P **p, int64_t count) {
-  if (hipMalloc((void **)p, (size_t)(count > 0 ? count : 1) * sizeof(P)) != hipSuccess)
+  if (dev_malloc_n(p, (size_t)(count > 0 ? count : 1)) != hipSuccess)
     return fail(IZH_ERR_NOMEM, "device allocation of %lld x %zu bytes failed",
                 (long long)count, sizeof(P));
   return IZH_OK;
@@ -114,8 +114,18 @@ static int dmalloc(P **p, int64_t count) {
 
 template <typename P>
 static void dfree(P *&p) {
-  if (p) (void)hipFree((void *)p);
+  dev_release((void *)p);
   p = nullptr;
+}
+
+static int join_streams(hipStream_t producer, hipStream_t consumer) {
+  if (producer == consumer) return IZH_OK;
+  hipEvent_t ev;
+  IZH_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+  IZH_HIP(hipEventRecord(ev, producer));
+  IZH_HIP(hipStreamWaitEvent(consumer, ev, 0));
+  IZH_HIP(hipEventDestroy(ev));
+  return IZH_OK;
 }
 
 // Moving rows (phase space + original index) for cap particles.
@@ -130,9 +140,9 @@ static int bunch_alloc_live(izh_bunch *b, int64_t cap) {
 }
 
 int bunch_alloc_alt(izh_bunch *b) {
+  if (!b->orig_alt) IZH_CHECK(dmalloc(&b->orig_alt, b->cap));
   IZH_CHECK(dmalloc(&b->r_alt[0], 6 * b->cap));
   for (int r = 1; r < 6; r++) b->r_alt[r] = b->r_alt[0] + r * b->cap;
-  IZH_CHECK(dmalloc(&b->orig_alt, b->cap));
   return IZH_OK;
 }
 
@@ -167,8 +177,9 @@ static int upload_pts(izh_bunch *b, const double *pts9, int64_t n) {
   touch_particles(b);
   if (n > 0xfffffffeLL)
     return fail(IZH_ERR_ARG, "bunch of %lld particles exceeds 2^32-2", (long long)n);
+  // work enqueued on the bunch may still read what is released here
+  IZH_HIP(hipStreamSynchronize(b->stream));
   if (n > b->cap) {
-    IZH_HIP(hipStreamSynchronize(b->stream));
     bunch_free_all(b);
     IZH_CHECK(bunch_alloc_live(b, n));
   }
@@ -307,6 +318,7 @@ int izh_bunch_create(const double *pts9, int64_t n, double current,
     delete b;
     return fail(IZH_ERR_HIP, "izh_bunch_create: stream creation failed");
   }
+  dev_handles(b->device, 1);
   if ((rc = bunch_alloc_live(b, n)) != IZH_OK ||
       (rc = dmalloc(&b->d_part, (int64_t)kMaxRedBlocks * kPartStride)) != IZH_OK ||
       (rc = dmalloc(&b->d_out, (int64_t)kPartStride + 8)) != IZH_OK) {
@@ -351,6 +363,7 @@ int izh_bunch_create_from(const izh_bunch *src, int64_t offset, int64_t n, doubl
     delete b;
     return fail(IZH_ERR_HIP, "izh_bunch_create_from: stream creation failed");
   }
+  dev_handles(b->device, 1);
   if ((rc = bunch_alloc_live(b, n)) != IZH_OK ||
       (rc = dmalloc(&b->d_part, (int64_t)kMaxRedBlocks * kPartStride)) != IZH_OK ||
       (rc = dmalloc(&b->d_out, (int64_t)kPartStride + 8)) != IZH_OK ||
@@ -386,7 +399,9 @@ int izh_bunch_create_from(const izh_bunch *src, int64_t offset, int64_t n, doubl
     izh_bunch_destroy(b);
     return fail(IZH_ERR_HIP, "izh_bunch_create_from: stream join failed");
   }
-  if ((rc = launch_clone(src, b, offset, n, w)) != IZH_OK) {
+  if ((rc = launch_clone(src, b, offset, n, w)) != IZH_OK ||
+      // and its rows stay until they are copied
+      (rc = join_streams(b->stream, src->stream)) != IZH_OK) {
     izh_bunch_destroy(b);
     return rc;
   }
@@ -406,6 +421,7 @@ int izh_bunch_destroy(izh_bunch *b) {
   if (b->h_out) (void)hipHostFree(b->h_out);
   if (b->h_scal) (void)hipHostFree(b->h_scal);
   if (b->stream) (void)hipStreamDestroy(b->stream);
+  dev_handles(b->device, -1);
   delete b;
   return IZH_OK;
 }
@@ -1115,6 +1131,7 @@ int izh_field_create(int nx, int ny, int nz, int precision, izh_field **out) {
     delete f;
     return fail(IZH_ERR_HIP, "izh_field_create: stream creation failed");
   }
+  dev_handles(f->device, 1);
   int rc = field_alloc(f);
   if (rc != IZH_OK) {
     izh_field_destroy(f);
@@ -1130,26 +1147,16 @@ int izh_field_destroy(izh_field *f) {
   void *bufs[] = {f->rho_fx, f->rho,  f->phi,    f->e,    f->spec_a,
                   f->spec_b, f->green, f->green_t, f->corner, f->tw_x,
                   f->tw_y,   f->tw_z, f->d_dom,  f->bin, f->d_wake};
-  for (void *p : bufs)
-    if (p) (void)hipFree(p);
+  for (void *p : bufs) dev_release(p);
   if (f->h_dom) (void)hipHostFree(f->h_dom);
   if (f->stream) (void)hipStreamDestroy(f->stream);
+  dev_handles(f->device, -1);
   delete f;
   return IZH_OK;
 }
 
 // Kernels of a bunch and a field run on their own streams while they share
 // data: the consumer's stream waits for everything queued on the producer's.
-static int join_streams(hipStream_t producer, hipStream_t consumer) {
-  if (producer == consumer) return IZH_OK;
-  hipEvent_t ev;
-  IZH_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-  IZH_HIP(hipEventRecord(ev, producer));
-  IZH_HIP(hipStreamWaitEvent(consumer, ev, 0));
-  IZH_HIP(hipEventDestroy(ev));
-  return IZH_OK;
-}
-
 static int check_dom(const izh_field *f, const izh_compdom *dom, const char *who) {
   if (!dom) return fail(IZH_ERR_ARG, "%s: no domain", who);
   if (dom->nx != f->nx || dom->ny != f->ny || dom->nz != f->nz)

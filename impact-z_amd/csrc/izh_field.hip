@@ -1309,7 +1309,7 @@ int upload_twiddles(izh_field *f) {
   int len[3] = {2 * f->nx, 2 * f->ny, 2 * f->nz};
   for (int a = 0; a < 3; a++) {
     make_twiddles<T>(tw, len[a]);
-    IZH_HIP(hipMalloc(dst[a], tw.size() * sizeof(cx<T>)));
+    IZH_HIP(dev_malloc(dst[a], tw.size() * sizeof(cx<T>)));
     IZH_HIP(hipMemcpy(*dst[a], tw.data(), tw.size() * sizeof(cx<T>),
                       hipMemcpyHostToDevice));
   }
@@ -1336,20 +1336,20 @@ int field_alloc(izh_field *f) {
   // neighbouring x lines, which then start on a line boundary
   const int64_t row = 128 / (2 * (int64_t)es);
   f->ldx = (kx + row - 1) / row * row;
-  IZH_HIP(hipMalloc((void **)&f->rho_fx, g * sizeof(unsigned long long)));
+  IZH_HIP(dev_malloc((void **)&f->rho_fx, g * sizeof(unsigned long long)));
   IZH_HIP(hipMemset(f->rho_fx, 0, g * sizeof(unsigned long long)));
-  IZH_HIP(hipMalloc(&f->rho, g * es));
-  IZH_HIP(hipMalloc(&f->phi, g * es));
-  IZH_HIP(hipMalloc(&f->e, 4 * g * es));
-  IZH_HIP(hipMalloc(&f->spec_a, f->ldx * f->ny * f->nz * 2 * es));
-  IZH_HIP(hipMalloc(&f->spec_b, f->ldx * 2 * f->ny * f->nz * 2 * es));
+  IZH_HIP(dev_malloc(&f->rho, g * es));
+  IZH_HIP(dev_malloc(&f->phi, g * es));
+  IZH_HIP(dev_malloc(&f->e, 4 * g * es));
+  IZH_HIP(dev_malloc(&f->spec_a, f->ldx * f->ny * f->nz * 2 * es));
+  IZH_HIP(dev_malloc(&f->spec_b, f->ldx * 2 * f->ny * f->nz * 2 * es));
   // G^ at x pitch ldx ([j][k][i], written by its z pass; the x pass's
   // output at pitch kx fits as well)
-  IZH_HIP(hipMalloc(&f->green, f->ldx * (f->ny + 1) * (f->nz + 1) * es));
-  IZH_HIP(hipMalloc(&f->green_t, ghalf * es));
-  IZH_HIP(hipMalloc((void **)&f->corner,
+  IZH_HIP(dev_malloc(&f->green, f->ldx * (f->ny + 1) * (f->nz + 1) * es));
+  IZH_HIP(dev_malloc(&f->green_t, ghalf * es));
+  IZH_HIP(dev_malloc((void **)&f->corner,
                     (size_t)(f->nx + 2) * (f->ny + 2) * (f->nz + 2) * sizeof(double)));
-  IZH_HIP(hipMalloc((void **)&f->d_dom, sizeof(DevDom)));
+  IZH_HIP(dev_malloc((void **)&f->d_dom, sizeof(DevDom)));
   IZH_HIP(hipHostMalloc((void **)&f->h_dom, sizeof(DevDom), hipHostMallocDefault));
   IZH_HIP(hipMemset(f->d_dom, 0, sizeof(DevDom)));
   if (f->precision == IZH_FP64) return upload_twiddles<double>(f);
@@ -1426,15 +1426,12 @@ static bool bins_ready(izh_field *f, int64_t n, bool weights, int ntiles) {
   const int64_t rows = weights ? 4 : 3, nch = n / kBinChunk + ntiles + 1;
   if (f->bin && n <= f->bin_cap && rows <= f->bin_rows && ntiles == f->bin_tiles) return true;
   (void)hipStreamSynchronize(f->stream);
-  if (f->bin) (void)hipFree(f->bin);
+  dev_release(f->bin);
   f->bin = nullptr;
   const size_t head = (size_t)2 * ntiles * sizeof(uint32_t) + (size_t)nch * sizeof(Chunk);
   const size_t at_rows = (head + sizeof(int64_t) + 255) / 256 * 256;
-  if (hipMalloc((void **)&f->bin, at_rows + (size_t)rows * n * sizeof(double)) != hipSuccess) {
-    (void)hipGetLastError();
-    f->bin = nullptr;
+  if (dev_malloc((void **)&f->bin, at_rows + (size_t)rows * n * sizeof(double)) != hipSuccess)
     return false;
-  }
   // nchunks, cursors, histogram, chunks, then the rows
   f->bin_cap = n;
   f->bin_rows = (int)rows;

@@ -1246,32 +1246,40 @@ __global__ void k_zero_u32(uint32_t *__restrict__ p, int64_t n) {
 
 int bunch_alloc_fused(izh_bunch *b, int ntiles, int64_t nseg) {
   const size_t ps = b->precision == IZH_FP64 ? sizeof(double) : sizeof(float);
-  if (!b->key) {
-    IZH_HIP(hipMalloc((void **)&b->key, (size_t)b->cap * sizeof(uint32_t)));
-    IZH_HIP(hipMalloc((void **)&b->key_alt, (size_t)b->cap * sizeof(uint32_t)));
-    IZH_HIP(hipMalloc(&b->tpos, (size_t)3 * b->cap * ps));
-    IZH_HIP(hipMalloc(&b->sink, kSinkBytes));
-    IZH_HIP(hipMalloc((void **)&b->d_scal, sizeof(DevScal)));
-  }
+  // each on its own: a call after one that ran out of memory goes on from there
+  const auto need = [](auto **p, size_t bytes) {
+    return *p ? hipSuccess : dev_malloc((void **)p, bytes);
+  };
+  IZH_HIP(need(&b->key, (size_t)b->cap * sizeof(uint32_t)));
+  IZH_HIP(need(&b->key_alt, (size_t)b->cap * sizeof(uint32_t)));
+  IZH_HIP(need(&b->tpos, (size_t)3 * b->cap * ps));
+  IZH_HIP(need(&b->sink, kSinkBytes));
+  IZH_HIP(need(&b->d_scal, sizeof(DevScal)));
   if (!b->r_alt[0]) IZH_CHECK(bunch_alloc_alt(b));
   if (!b->h_scal)
     IZH_HIP(hipHostMalloc((void **)&b->h_scal, sizeof(DevScal), hipHostMallocDefault));
   const int64_t nch = b->cap / chunk_len(b->cap) + ntiles + 1;
   if (ntiles > b->ntiles_cap || nch > b->nchunks_cap) {
+    IZH_HIP(hipStreamSynchronize(b->stream));
+    for (int k = 0; k < 2; k++) dev_release(b->hist[k]);
+    dev_release(b->cursor);
+    dev_release(b->chunks);
+    b->hist[0] = b->hist[1] = b->cursor = nullptr;
+    b->chunks = nullptr;
+    b->ntiles_cap = b->nchunks_cap = 0;
     for (int k = 0; k < 2; k++)
-      if (b->hist[k]) (void)hipFree(b->hist[k]);
-    if (b->cursor) (void)hipFree(b->cursor);
-    if (b->chunks) (void)hipFree(b->chunks);
-    for (int k = 0; k < 2; k++)
-      IZH_HIP(hipMalloc((void **)&b->hist[k], (size_t)ntiles * sizeof(uint32_t)));
-    IZH_HIP(hipMalloc((void **)&b->cursor, (size_t)ntiles * sizeof(uint32_t)));
-    IZH_HIP(hipMalloc((void **)&b->chunks, (size_t)2 * nch * sizeof(Chunk)));
+      IZH_HIP(dev_malloc((void **)&b->hist[k], (size_t)ntiles * sizeof(uint32_t)));
+    IZH_HIP(dev_malloc((void **)&b->cursor, (size_t)ntiles * sizeof(uint32_t)));
+    IZH_HIP(dev_malloc((void **)&b->chunks, (size_t)2 * nch * sizeof(Chunk)));
     b->ntiles_cap = ntiles;
     b->nchunks_cap = nch;
   }
   if (nseg > b->moments_cap) {
-    if (b->d_moments) (void)hipFree(b->d_moments);
-    IZH_HIP(hipMalloc((void **)&b->d_moments, (size_t)nseg * kRunRecord * sizeof(double)));
+    IZH_HIP(hipStreamSynchronize(b->stream));
+    dev_release(b->d_moments);
+    b->d_moments = nullptr;
+    b->moments_cap = 0;
+    IZH_HIP(dev_malloc((void **)&b->d_moments, (size_t)nseg * kRunRecord * sizeof(double)));
     b->moments_cap = nseg;
   }
   return IZH_OK;

@@ -31,6 +31,21 @@ int fail(int code, const char *fmt, ...);
     if (rc_ != IZH_OK) return rc_;   \
   } while (0)
 
+// ------------------------------------------------------ device memory
+// Device memory of the bunches and fields.  dev_release keeps a block for the
+// next dev_malloc on its device instead of returning it (izh_memory.hip says
+// how much and for how long); the caller has waited for the work that uses it.
+hipError_t dev_malloc(void **p, size_t bytes);
+void dev_release(void *p);
+// A bunch or field comes to life (+1) or ends (-1) on a device; with the last
+// one every kept block of the device goes back.
+void dev_handles(int device, int change);
+
+template <typename P>
+hipError_t dev_malloc_n(P **p, size_t count) {
+  return dev_malloc((void **)p, (count > 0 ? count : 1) * sizeof(P));
+}
+
 // ---------------------------------------------------------- constants
 constexpr int kBlock = 256;          // threads per block for particle passes
 constexpr int kMaxRedBlocks = 2048;  // fixed partial count => deterministic sums

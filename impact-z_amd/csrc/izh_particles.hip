@@ -647,7 +647,7 @@ int launch_compact(izh_bunch *b, double xrad, double yrad, int64_t nkeep) {
   const double rad = (xrad + yrad) / 2.0;
   const int64_t nchunks = (b->n + kCompactChunk - 1) / kCompactChunk;
   int64_t *cnt = nullptr;
-  IZH_HIP(hipMalloc((void **)&cnt, (nchunks + 1) * sizeof(int64_t)));
+  IZH_HIP(dev_malloc((void **)&cnt, (nchunks + 1) * sizeof(int64_t)));
   hipLaunchKernelGGL(k_compact_count, dim3(nchunks), dim3(kBlock), 0, b->stream,
                      b->r[0], b->r[1], b->r[2], b->r[3], b->r[5], b->n, gam,
                      rad, cnt);
@@ -663,7 +663,7 @@ int launch_compact(izh_bunch *b, double xrad, double yrad, int64_t nkeep) {
   IZH_HIP(hipMemcpyAsync(&total, cnt + nchunks, sizeof(int64_t),
                          hipMemcpyDeviceToHost, b->stream));
   IZH_HIP(hipStreamSynchronize(b->stream));
-  IZH_HIP(hipFree(cnt));
+  dev_release(cnt);
   if (total != nkeep)
     return fail(IZH_ERR_STATE, "compaction kept %lld particles, conv1st %lld",
                 (long long)total, (long long)nkeep);
@@ -767,7 +767,7 @@ k_chg_count(const uint32_t *__restrict__ orig, const double *__restrict__ qm0, i
 
 int launch_chg_count(izh_bunch *b, const ChgList &cl, int64_t *out) {
   if (!b->d_chg) {
-    IZH_HIP(hipMalloc((void **)&b->d_chg, kMaxChargeStates * sizeof(unsigned long long)));
+    IZH_HIP(dev_malloc((void **)&b->d_chg, kMaxChargeStates * sizeof(unsigned long long)));
     IZH_HIP(hipHostMalloc((void **)&b->h_chg, kMaxChargeStates * sizeof(unsigned long long),
                           hipHostMallocDefault));
   }

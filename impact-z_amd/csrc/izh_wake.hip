@@ -392,7 +392,7 @@ k_wake_add(E4<T> *__restrict__ e, int64_t plane, int nz, const double *__restric
 int wake_alloc(izh_field *f) {
   if (f->d_wake) return IZH_OK;
   const size_t nz = (size_t)f->nz;
-  IZH_HIP(hipMalloc((void **)&f->d_wake, (6 * nz + 3 * (nz + 1)) * sizeof(double)));
+  IZH_HIP(dev_malloc((void **)&f->d_wake, (6 * nz + 3 * (nz + 1)) * sizeof(double)));
   return IZH_OK;
 }
 

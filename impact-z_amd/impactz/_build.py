@@ -19,7 +19,7 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 
 SOURCES = ["izh_api.hip", "izh_particles.hip", "izh_field.hip", "izh_fused.hip",
-           "izh_wake.hip"]
+           "izh_wake.hip", "izh_memory.hip"]
 
 # Packed FP32 instructions are disabled for all device code: they have given
 # intermittently wrong results on this hardware generation's toolchain.
