@@ -1144,9 +1144,9 @@ int izh_field_create(int nx, int ny, int nz, int precision, izh_field **out) {
 int izh_field_destroy(izh_field *f) {
   if (!f) return IZH_OK;
   if (f->stream) (void)hipStreamSynchronize(f->stream);
-  void *bufs[] = {f->rho_fx, f->rho,  f->phi,    f->e,    f->spec_a,
-                  f->spec_b, f->green, f->green_t, f->corner, f->tw_x,
-                  f->tw_y,   f->tw_z, f->d_dom,  f->bin, f->d_wake};
+  void *bufs[] = {f->rho_fx, f->rho,   f->phi,     f->e,      f->spec_a,
+                  f->spec_b, f->green, f->green_t, f->corner, f->igf_box,
+                  f->tables, f->d_dom, f->bin,     f->d_wake};
   for (void *p : bufs) dev_release(p);
   if (f->h_dom) (void)hipHostFree(f->h_dom);
   if (f->stream) (void)hipStreamDestroy(f->stream);

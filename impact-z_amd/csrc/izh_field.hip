@@ -18,8 +18,10 @@
 // decimation in time for the inverse of the fused z pass (bit-reversed in,
 // natural out), so no reorder pass is needed between them.
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstring>
+#include <map>
 #include <vector>
 
 #include "izh_device.hpp"
@@ -70,6 +72,8 @@ struct Lines {
   void *rho;               // kLoadFx: the converted grid
   double fx_inv;           // kLoadFx: grid value of one fixed-point unit
   int tx, ty;              // kLoadIgf: corners per row, rows per plane
+  const void *far;         // kLoadIgf: G away from the origin (T)
+  const IgfBox *box;       // kLoadIgf: where the corners hold
 };
 
 // 8-corner difference of the antiderivative at the cells' corners
@@ -79,6 +83,68 @@ __device__ inline double igf_diff(const double *__restrict__ t, int64_t c, int64
                                   int64_t txy) {
   return t[c + 1 + tx + txy] - t[c + tx + txy] - t[c + 1 + txy] + t[c + txy] -
          t[c + 1 + tx] + t[c + tx] + t[c + 1] - t[c];
+}
+
+// The integrated Green function far from the origin: the mean of 1/r over a
+// cell, as the Taylor series of 1/r averaged over the cell up to eighth order.
+// With a = x^2/r^4 (b, c for y, z) it is a polynomial over r,
+//   g = (1/r) sum of C_ijk a^i b^j c^k, i + j + k <= 4, C_000 = 1,
+// whose coefficients hold the mesh sizes (igf_coefficients).  The 8-corner
+// difference of the antiderivative costs three arctangents and three
+// logarithms per corner and cancels: its relative error grows with r^3, 1e-12
+// at kIgfFar cell half diagonals and 1e-9 at 64 of cells 1:1:4, where the
+// truncated series is off by at most 4e-13 and 3e-16 (against a 20-point
+// Gauss rule in 80 bits, cells from 1:1:0.2 to 1:4:16; at ten half diagonals
+// the two meet for cubes).  So only the box within kIgfFar of the origin
+// keeps the corners.  The deposit's launch, which forms G beside the deposit,
+// fell from 60 to 40 us on 128^3 (150k particles, FP64; 2.2M corners, 27 us of
+// the deposit's own) and from 245 to 199 us on 128x128x256 (10M, mixed).
+constexpr int kIgfOrder = 4;                    // pairs of derivatives
+constexpr int kIgfTerms = 35;
+constexpr double kIgfFar = 12.0;
+// Nodes from which the series is used: below, its preparation takes as long as
+// the corners it saves (deposit's launch and x pass of 64^3: 24.3 us either
+// way; of 64x64x128 42.4 against 45.9).
+constexpr int64_t kIgfSeriesNodes = 400000;
+
+// Place of C_ijk: i outermost, then j, then k.
+__host__ __device__ constexpr int igf_term(int i, int j, int k) {
+  // terms of the i's before: T(4) + T(3) + ..., T(n) = (n+1)(n+2)/2
+  return (i > 0 ? 15 : 0) + (i > 1 ? 10 : 0) + (i > 2 ? 6 : 0) + (i > 3 ? 3 : 0) +
+         j * (kIgfOrder + 1 - i) - j * (j - 1) / 2 + k;
+}
+static_assert(igf_term(kIgfOrder, 0, 0) == kIgfTerms - 1 && igf_term(1, 0, 0) == 15 &&
+              igf_term(0, 0, 4) == 4 && igf_term(0, 1, 0) == 5, "igf_term");
+
+// C: the coefficients, uniform over the wavefront.
+__device__ inline double igf_far(const double (&C)[kIgfTerms], double x2, double y2, double z2) {
+  const double ir = rsqrt(x2 + y2 + z2), ir2 = ir * ir, ir4 = ir2 * ir2;
+  const double a = x2 * ir4, b = y2 * ir4, c = z2 * ir4;
+  double s = 0.0;
+#pragma unroll
+  for (int i = kIgfOrder; i >= 0; i--) {
+    double p = 0.0;
+#pragma unroll
+    for (int j = kIgfOrder - i; j >= 0; j--) {
+      double q = 0.0;
+#pragma unroll
+      for (int k = kIgfOrder - i - j; k >= 0; k--) q = fma(q, c, C[igf_term(i, j, k)]);
+      p = fma(p, b, q);
+    }
+    s = fma(s, a, p);
+  }
+  return s * ir;
+}
+
+// G at node (i, j, k): the corners' difference in the box near the origin,
+// elsewhere the grid the series left (igf_block).
+template <typename T>
+__device__ inline T igf_value(const Lines &p, int i, int j, int k, const int near[3]) {
+  if (i < near[0] && j < near[1] && k < near[2]) {
+    const int64_t txy = (int64_t)p.tx * p.ty;
+    return (T)igf_diff((const double *)p.src, i + j * (int64_t)p.tx + k * txy, p.tx, txy);
+  }
+  return ((const T *)p.far)[i + (p.tx - 1) * (j + (p.ty - 1) * (int64_t)k)];
 }
 
 // Logical block of physical block p of n: the hardware deals blocks to the
@@ -357,9 +423,8 @@ __device__ __attribute__((always_inline)) inline void fft_lines_block(
     // ---- even lines of G: each value is formed once and written to both of
     // its places, m and L-m (thread m = 0 also takes m = L/2)
     static_assert(LOAD != kLoadIgf || PAIR, "even lines travel in pairs");
-    const double *src = (const double *)p.src;
-    const int64_t txy = (int64_t)p.tx * p.ty;
     const int half = L >> 1;
+    const int near[3] = {p.box->near[0], p.box->near[1], p.box->near[2]};
     constexpr int kPer = PTS / 2 / kFftThreads;
 #pragma unroll
     for (int it = 0; it < kPer; it++) {
@@ -370,18 +435,17 @@ __device__ __attribute__((always_inline)) inline void fft_lines_block(
       int j0, k0, j1, k1;
       line_fs(has0 ? l0 : 0, p, j0, k0);
       line_fs(has1 ? l1 : 0, p, j1, k1);
-      const int64_t c0 = j0 * (int64_t)p.tx + k0 * txy, c1 = j1 * (int64_t)p.tx + k1 * txy;
-      const double a = igf_diff(src, c0 + m, p.tx, txy);
-      const double b = igf_diff(src, c1 + m, p.tx, txy);
-      const cx<T> v = {has0 ? (T)a : (T)0, has1 ? (T)b : (T)0};
+      const T a = igf_value<T>(p, m, j0, k0, near);
+      const T b = igf_value<T>(p, m, j1, k1, near);
+      const cx<T> v = {has0 ? a : (T)0, has1 ? b : (T)0};
       cx<T> *row = buf + lb * LP;
       row[lds_pos(m, mask)] = v;
       if (m > 0) {
         row[lds_pos(L - m, mask)] = v;
       } else {
-        const double ah = igf_diff(src, c0 + half, p.tx, txy);
-        const double bh = igf_diff(src, c1 + half, p.tx, txy);
-        row[lds_pos(half, mask)] = {has0 ? (T)ah : (T)0, has1 ? (T)bh : (T)0};
+        const T ah = igf_value<T>(p, half, j0, k0, near);
+        const T bh = igf_value<T>(p, half, j1, k1, near);
+        row[lds_pos(half, mask)] = {has0 ? ah : (T)0, has1 ? bh : (T)0};
       }
     }
 #pragma unroll
@@ -607,34 +671,104 @@ k_fft_two(Lines a, Lines b, int nba, int nbb, const cx<T> *__restrict__ twg) {
 }
 
 // ------------------------------------------------------ Green function
-// IGF antiderivative at cell corners (src/Appl/Field.f90:384-418), FP64,
-// mesh sizes from the device domain; corners first, first + stride, ...
-__device__ inline void igf_corners(double *__restrict__ out, int tx, int ty, int tz,
-                                   const DevDom *__restrict__ dom, int first, int stride) {
+// Block bid of nb of the Green function's values: the corners of the box near
+// the origin, and the series' values on the nodes outside of it (far: the grid
+// of (nx+1)(ny+1)(nz+1) nodes; the x pass reads neither elsewhere).  The first
+// block leaves the box for the x pass.  C: kIgfTerms doubles of LDS.
+template <typename T>
+__device__ inline void igf_block(double *__restrict__ out, T *__restrict__ far, int nx, int ny,
+                                 int nz, const DevDom *__restrict__ dom,
+                                 const double *__restrict__ tab, IgfBox *__restrict__ box,
+                                 double *C, int bid, int nb) {
   const double hx = dom->msize[0], hy = dom->msize[1], hz = dom->msize[2];
-  const double vol = hx * hy * hz;
-  const int n = tx * ty * tz;
-  for (int c = first; c < n; c += stride) {
-    int i = c % tx;
-    int j = (c / tx) % ty;
-    int k = c / (tx * ty);
-    double x = i * hx - hx / 2.0, y = j * hy - hy / 2.0, z = k * hz - hz / 2.0;
-    double rr = sqrt(x * x + y * y + z * z);
-    double aa = -z * z * atan(x * y / (z * rr)) / 2.0;
-    double bb = -y * y * atan(x * z / (y * rr)) / 2.0;
-    double cc = -x * x * atan(y * z / (x * rr)) / 2.0;
-    double dd = y * z * log(x + rr);
-    double ee = x * z * log(y + rr);
-    double ff = x * y * log(z + rr);
-    out[c] = (aa + bb + cc + dd + ee + ff) / vol;
+  const double h2[3] = {hx * hx, hy * hy, hz * hz};
+  const int gx = nx + 1, gy = ny + 1, gz = nz + 1;
+  const bool series = (int64_t)gx * gy * gz > kIgfSeriesNodes;
+  const double reach = kIgfFar * 0.5 * sqrt(h2[0] + h2[1] + h2[2]);
+  const auto edge = [&](int g, double h) {
+    return series ? (int)fmin((double)g, floor(reach / h) + 1.0) : g;
+  };
+  const int near[3] = {edge(gx, hx), edge(gy, hy), edge(gz, hz)};
+  if (bid == 0 && threadIdx.x < 3) box->near[threadIdx.x] = near[threadIdx.x];
+  // corners first (the longer chain), a thread each up to half the blocks;
+  // the rest take the series, or the corners too where there is none
+  const int bx = near[0] + 1, by = near[1] + 1, bz = near[2] + 1;
+  const int ncorners = bx * by * bz;
+  const bool all = near[0] == gx && near[1] == gy && near[2] == gz;
+  const int nbc = all ? nb : min((ncorners + (int)blockDim.x - 1) / (int)blockDim.x, nb / 2);
+  if (bid < nbc) {
+    // IGF antiderivative (src/Appl/Field.f90:384-418)
+    const double vol = hx * hy * hz;
+    const int tx = nx + 2, ty = ny + 2;
+    for (int c = bid * (int)blockDim.x + (int)threadIdx.x; c < ncorners;
+         c += nbc * (int)blockDim.x) {
+      const int k = c / (bx * by), rem = c - k * bx * by, j = rem / bx, i = rem - j * bx;
+      double x = i * hx - hx / 2.0, y = j * hy - hy / 2.0, z = k * hz - hz / 2.0;
+      double rr = sqrt(x * x + y * y + z * z);
+      double aa = -z * z * atan(x * y / (z * rr)) / 2.0;
+      double bb = -y * y * atan(x * z / (y * rr)) / 2.0;
+      double cc = -x * x * atan(y * z / (x * rr)) / 2.0;
+      double dd = y * z * log(x + rr);
+      double ee = x * z * log(y + rr);
+      double ff = x * y * log(z + rr);
+      out[i + tx * (int64_t)(j + ty * k)] = (aa + bb + cc + dd + ee + ff) / vol;
+    }
+    return;
+  }
+  if ((int)threadIdx.x < kIgfTerms) {
+    // term t: its row of the table times the monomials of the squared mesh
+    // sizes (the table is zero between orders)
+    double pw[3][kIgfOrder + 1];
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+      pw[a][0] = 1.0;
+#pragma unroll
+      for (int q = 1; q <= kIgfOrder; q++) pw[a][q] = pw[a][q - 1] * h2[a];
+    }
+    const double *row = tab + (int)threadIdx.x * kIgfTerms;
+    double c = 0.0;
+#pragma unroll
+    for (int i = 0; i <= kIgfOrder; i++)
+#pragma unroll
+      for (int j = 0; i + j <= kIgfOrder; j++)
+#pragma unroll
+        for (int k = 0; i + j + k <= kIgfOrder; k++)
+          c += row[igf_term(i, j, k)] * (pw[0][i] * pw[1][j] * pw[2][k]);
+    C[threadIdx.x] = c;
+  }
+  __syncthreads();
+  // ---- the series.  Its coefficients move to scalar registers, so a node is
+  // its 34 multiply-adds and a reciprocal root; the node's indexes split by
+  // FP64 multiplies (exact: (c + 1/2) / g is at least 1/(2g) from an integer)
+  {
+    double U[kIgfTerms];
+#pragma unroll
+    for (int t = 0; t < kIgfTerms; t++) {
+      const int lo = __builtin_amdgcn_readfirstlane(__double2loint(C[t]));
+      const int hi = __builtin_amdgcn_readfirstlane(__double2hiint(C[t]));
+      U[t] = __hiloint2double(hi, lo);
+    }
+    const int total = gx * gy * gz;
+    const double igx = 1.0 / gx, igy = 1.0 / gy;
+    for (int c = (bid - nbc) * (int)blockDim.x + (int)threadIdx.x; c < total;
+         c += (nb - nbc) * (int)blockDim.x) {
+      const int jk = (int)((c + 0.5) * igx), i = c - jk * gx;
+      const int k = (int)((jk + 0.5) * igy), j = jk - k * gy;
+      if (i < near[0] && j < near[1] && k < near[2]) continue;
+      far[c] = (T)igf_far(U, (double)(i * i) * h2[0], (double)(j * j) * h2[1],
+                          (double)(k * k) * h2[2]);
+    }
   }
 }
 
+constexpr int kIgfBlocks = 768;  // as many as the deposit's LDS lets run at once (2048: 45 us)
+template <typename T>
 __global__ void __launch_bounds__(kBlock)
-k_igf_corner(double *__restrict__ out, int tx, int ty, int tz,
-             const DevDom *__restrict__ dom) {
-  igf_corners(out, tx, ty, tz, dom, blockIdx.x * blockDim.x + threadIdx.x,
-              gridDim.x * blockDim.x);
+k_igf(double *__restrict__ out, T *__restrict__ far, int nx, int ny, int nz,
+      const DevDom *__restrict__ dom, const double *__restrict__ tab,
+      IgfBox *__restrict__ box) {
+  __shared__ double C[kIgfTerms];
+  igf_block<T>(out, far, nx, ny, nz, dom, tab, box, C, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // --------------------------------------------------------------- deposit
@@ -970,14 +1104,15 @@ k_deposit_tiles(const P *__restrict__ X, const P *__restrict__ Y,
                 const KeyGrid *__restrict__ kgrid, const DevDom *__restrict__ dom, int nx,
                 int ny, int nz, int s0, int s1, int s2, int tnx, int tny, double scale,
                 unsigned long long *__restrict__ rho, int64_t *__restrict__ spill,
-                double *__restrict__ corner, int ncorner) {
+                double *__restrict__ corner, P *__restrict__ far,
+                const double *__restrict__ igf_tab, IgfBox *__restrict__ box, int ncorner) {
   __shared__ __align__(16) unsigned long long win[kTileWinCells + 1];
-  // the first ncorner blocks (a multiple of eight) form the corners of the
-  // step's Green function, which needs only the domain: arithmetic beside
-  // the deposit's LDS traffic, and no launch of its own
+  // the first ncorner blocks (a multiple of eight) prepare the step's Green
+  // function, which needs only the domain: arithmetic beside the deposit's
+  // LDS traffic, and no launch of its own
   if ((int)blockIdx.x < ncorner) {
-    igf_corners(corner, nx + 2, ny + 2, nz + 2, dom,
-                (int)blockIdx.x * kDepThreads + (int)threadIdx.x, ncorner * kDepThreads);
+    igf_block<P>(corner, far, nx, ny, nz, dom, igf_tab, box, reinterpret_cast<double *>(win),
+                 (int)blockIdx.x, ncorner);
     return;
   }
   const int bid = (int)blockIdx.x - ncorner;
@@ -1228,10 +1363,11 @@ int convolve_t(izh_field *f) {
   // starts on a 128-byte boundary; lines kx..ld-1 are padding.
   const int64_t ld = f->ldx;
   Lines g{}, p{};
-  // ---- x: lines (j<=ny, k<=nz) of G's corner difference -> green, and
+  // ---- x: lines (j<=ny, k<=nz) of G as they are formed -> green, and
   // rho (nx,ny,nz) real -> A (kx of ld, ny, nz)
   g.src = f->corner; g.dst = f->green;
   g.tx = nx + 2; g.ty = ny + 2;
+  g.far = f->green_t; g.box = f->igf_box;
   g.nf = ny + 1; g.ns = nz + 1;
   g.df = kx; g.ds = (int64_t)kx * (ny + 1); g.de = 1;
   g.L = mx; g.Lin = g.L; g.Lout = nx + 1; g.out_scale = 1.0;
@@ -1294,25 +1430,78 @@ int convolve_t(izh_field *f) {
 }
 
 template <typename T>
-void make_twiddles(std::vector<cx<T>> &tw, int L) {
-  tw.resize(L / 2);
+void make_twiddles(cx<T> *tw, int L) {
   for (int t = 0; t < L / 2; t++) {
     long double a = -2.0L * 3.141592653589793238462643383279502884L * t / L;
     tw[t] = {(T)cosl(a), (T)sinl(a)};
   }
 }
 
+// The series' table: tab[t * kIgfTerms + u] is what the derivative of 1/r of
+// orders (2i, 2j, 2k), u = igf_term(i, j, k), adds to term t per monomial
+// hx^2i hy^2j hz^2k: the derivative's polynomial P / r^(2n+1) by
+// d/dx (P r^-m) = (r^2 dP/dx - m x P) r^-(m+2), times the mean of s^2i / (2i)!
+// over the cell, 1 / (4^i (2i+1)!), and alike for y and z.  P's term
+// x^2p y^2q z^2r / r^(2n) is a^p b^q c^r.
+std::vector<double> igf_table() {
+  using Exps = std::array<int, 3>;
+  std::vector<double> tab((size_t)kIgfTerms * kIgfTerms, 0.0);
+  long double fact[2 * kIgfOrder + 2] = {1.0L};
+  for (int q = 1; q < 2 * kIgfOrder + 2; q++) fact[q] = fact[q - 1] * q;
+  for (int i = 0; i <= kIgfOrder; i++)
+    for (int j = 0; i + j <= kIgfOrder; j++)
+      for (int k = 0; i + j + k <= kIgfOrder; k++) {
+        const int n[3] = {i, j, k}, u = igf_term(i, j, k);
+        std::map<Exps, long double> P{{Exps{0, 0, 0}, 1.0L}};
+        int m = 1;
+        long double w = 1.0L;
+        for (int a = 0; a < 3; a++) {
+          w /= powl(4.0L, n[a]) * fact[2 * n[a] + 1];
+          for (int d = 0; d < 2 * n[a]; d++, m += 2) {
+            std::map<Exps, long double> Q;
+            for (const auto &t : P) {
+              Exps e = t.first;
+              e[a]++;
+              Q[e] -= m * t.second;
+              if (t.first[a] == 0) continue;
+              e = t.first;
+              e[a]--;
+              for (int c = 0; c < 3; c++) {
+                Exps f = e;
+                f[c] += 2;
+                Q[f] += t.first[a] * t.second;
+              }
+            }
+            P = Q;
+          }
+        }
+        for (const auto &t : P)
+          if (t.second != 0.0L)
+            tab[(size_t)igf_term(t.first[0] / 2, t.first[1] / 2, t.first[2] / 2) * kIgfTerms +
+                u] = (double)(w * t.second);
+      }
+  return tab;
+}
+
+// Twiddles of the three line lengths and the series' table, in one buffer.
 template <typename T>
-int upload_twiddles(izh_field *f) {
-  std::vector<cx<T>> tw;
-  void **dst[3] = {&f->tw_x, &f->tw_y, &f->tw_z};
-  int len[3] = {2 * f->nx, 2 * f->ny, 2 * f->nz};
+int upload_tables(izh_field *f) {
+  static const std::vector<double> igf = igf_table();
+  const int len[3] = {2 * f->nx, 2 * f->ny, 2 * f->nz};
+  size_t at[4] = {0, 0, 0, 0}, bytes = igf.size() * sizeof(double);
   for (int a = 0; a < 3; a++) {
-    make_twiddles<T>(tw, len[a]);
-    IZH_HIP(dev_malloc(dst[a], tw.size() * sizeof(cx<T>)));
-    IZH_HIP(hipMemcpy(*dst[a], tw.data(), tw.size() * sizeof(cx<T>),
-                      hipMemcpyHostToDevice));
+    at[a] = bytes;
+    bytes = (bytes + len[a] / 2 * sizeof(cx<T>) + 255) / 256 * 256;
   }
+  std::vector<char> host(bytes);
+  std::memcpy(host.data(), igf.data(), igf.size() * sizeof(double));
+  for (int a = 0; a < 3; a++) make_twiddles<T>((cx<T> *)(host.data() + at[a]), len[a]);
+  IZH_HIP(dev_malloc((void **)&f->tables, bytes));
+  IZH_HIP(hipMemcpy(f->tables, host.data(), bytes, hipMemcpyHostToDevice));
+  f->igf_tab = (const double *)f->tables;
+  f->tw_x = f->tables + at[0];
+  f->tw_y = f->tables + at[1];
+  f->tw_z = f->tables + at[2];
   return IZH_OK;
 }
 
@@ -1352,8 +1541,9 @@ int field_alloc(izh_field *f) {
   IZH_HIP(dev_malloc((void **)&f->d_dom, sizeof(DevDom)));
   IZH_HIP(hipHostMalloc((void **)&f->h_dom, sizeof(DevDom), hipHostMallocDefault));
   IZH_HIP(hipMemset(f->d_dom, 0, sizeof(DevDom)));
-  if (f->precision == IZH_FP64) return upload_twiddles<double>(f);
-  return upload_twiddles<float>(f);
+  IZH_HIP(dev_malloc((void **)&f->igf_box, sizeof(IgfBox)));
+  if (f->precision == IZH_FP64) return upload_tables<double>(f);
+  return upload_tables<float>(f);
 }
 
 int field_set_domain(izh_field *f, const izh_compdom *dom) {
@@ -1396,13 +1586,15 @@ int launch_deposit(izh_bunch *b, izh_field *f, const Chunk *chunks, const KeyGri
   const int tnx = f->nx >> s0, tny = f->ny >> s1;
   int64_t *spill = b->d_scal ? &b->d_scal->overflow : nullptr;
   const int64_t nc = (int64_t)(f->nx + 2) * (f->ny + 2) * (f->nz + 2);
-  const int ncorner = (grid_for(nc, kDepThreads) + 7) & ~7;
+  const int ncorner = std::min((grid_for(nc, kDepThreads) + 7) & ~7, kIgfBlocks);
   const auto go = [&](auto kern, const auto *tp) {
     hipLaunchKernelGGL(kern, dim3((unsigned)(ncorner + max_chunks)), dim3(kDepThreads), 0,
                        f->stream, tp, tp + b->cap, tp + 2 * b->cap, b->orig, b->w0, b->w_value,
                        b->w_uniform, chunks, d_nchunks, kgrid, f->d_dom, f->nx, f->ny, f->nz,
                        s0, s1, s2, tnx, tny, f->fixed_scale, f->rho_fx, spill, f->corner,
-                       ncorner);
+                       const_cast<std::remove_const_t<std::remove_pointer_t<decltype(tp)>> *>(
+                           (decltype(tp))f->green_t),
+                       f->igf_tab, f->igf_box, ncorner);
   };
   if (f->precision == IZH_MIXED) {
     const float *tp = (const float *)b->tpos;
@@ -1526,8 +1718,13 @@ int launch_solve(izh_field *f) {
   {
     ScopedTimer tm_(IZH_T_GREEN, f->stream);
     const int nc = (f->nx + 2) * (f->ny + 2) * (f->nz + 2);
-    hipLaunchKernelGGL(k_igf_corner, dim3(grid_for(nc)), dim3(kBlock), 0, f->stream,
-                       f->corner, f->nx + 2, f->ny + 2, f->nz + 2, f->d_dom);
+    const dim3 g(std::min(grid_for(nc), kIgfBlocks)), t(kBlock);
+    if (f->precision == IZH_FP64)
+      hipLaunchKernelGGL(k_igf<double>, g, t, 0, f->stream, f->corner, (double *)f->green_t,
+                         f->nx, f->ny, f->nz, f->d_dom, f->igf_tab, f->igf_box);
+    else
+      hipLaunchKernelGGL(k_igf<float>, g, t, 0, f->stream, f->corner, (float *)f->green_t,
+                         f->nx, f->ny, f->nz, f->d_dom, f->igf_tab, f->igf_box);
     IZH_HIP(hipGetLastError());
   }
   const int rc = f->precision == IZH_FP64 ? convolve_t<double, false>(f)

@@ -97,6 +97,11 @@ __device__ inline int tile_first_node(int t0, double klo, double kh, double lo,
   return (int)fmin(fmax(u, -1.0e6), 1.0e6);  // callers clamp to the grid
 }
 
+// The box of nodes (from the origin) whose Green function comes from corners.
+struct IgfBox {
+  int near[3];
+};
+
 // Bunch scalars a run of steps keeps on the device.
 struct DevScal {
   double current;     // BeamBunch%Current
@@ -212,7 +217,10 @@ struct izh_field {
   void *green = nullptr;        // T[(ny+1)][(nz+1)][ldx] transformed Green fn
   void *green_t = nullptr;      // T[(nx+1)*(ny+1)*(nz+1)] work
   double *corner = nullptr;     // double[(nx+2)*(ny+2)*(nz+2)] IGF antiderivative
-  void *tw_x = nullptr, *tw_y = nullptr, *tw_z = nullptr;  // twiddles per length
+  izh::IgfBox *igf_box = nullptr;  // where the corners hold, on this domain
+  char *tables = nullptr;       // the series' table and the twiddles per length
+  const double *igf_tab = nullptr;
+  const void *tw_x = nullptr, *tw_y = nullptr, *tw_z = nullptr;
   izh::DevDom *d_dom = nullptr; // domain the kernels read
   izh::DevDom *h_dom = nullptr; // pinned staging for host-set domains
   // izh_charge's bins (launch_deposit_granular), made by its first large bunch
