@@ -433,6 +433,14 @@ int izh_bunch_download(izh_bunch *b, double *pts9, int64_t cap, int64_t *n) {
     return fail(IZH_ERR_ARG, "izh_bunch_download: %lld rows needed, %lld given",
                 (long long)b->n, (long long)cap);
   const int64_t nn = b->n, n0 = b->n0;
+  // packed on the device (300k particles 3.1 -> 1.4 ms with the copy); on the
+  // host where the device has no memory left for it
+  bool no_memory = nn == 0;
+  if (nn > 0) IZH_CHECK(launch_download(b, pts9, &no_memory));
+  if (!no_memory) {
+    *n = nn;
+    return IZH_OK;
+  }
   std::vector<uint32_t> orig((size_t)(nn > 0 ? nn : 1));
   std::vector<double> rows((size_t)(6 * nn > 0 ? 6 * nn : 1));
   std::vector<double> fixed((size_t)(3 * n0 > 0 ? 3 * n0 : 1));

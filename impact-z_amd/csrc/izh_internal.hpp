@@ -508,6 +508,9 @@ int launch_moments_rows(const double *rows, int64_t ld, int64_t n, double *out,
                         hipStream_t st);
 // Looks up the scratch array's address on `device` (current) once.
 int scratch_setup(int device);
+// The live particles as Pts1(9,n), in their original order; *no_memory: there is
+// no device memory to pack them in, and nothing was done.
+int launch_download(izh_bunch *b, double *pts9, bool *no_memory);
 int launch_clone(const izh_bunch *src, izh_bunch *dst, int64_t offset, int64_t n, double w);
 int field_set_domain(izh_field *f, const izh_compdom *dom);
 int launch_deposit(izh_bunch *b, izh_field *f, const Chunk *chunks, const KeyGrid *kgrid,

@@ -5,9 +5,11 @@
 // Reductions (conv1st range, diagnostic moments) go through a fixed number of
 // per-block partials and a single-block tree in LDS: the summation order
 // depends only on N, so results are bitwise reproducible run to run.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <mutex>
+#include <vector>
 
 #include "izh_device.hpp"
 
@@ -292,16 +294,33 @@ k_compact_count(const double *__restrict__ x, const double *__restrict__ px,
   }
 }
 
-__global__ void k_scan_counts(int64_t *__restrict__ cnt, int64_t nchunks) {
-  // one thread: nchunks is N / 2048 and the path runs only after losses
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  int64_t acc = 0;
-  for (int64_t c = 0; c < nchunks; c++) {
-    int64_t v = cnt[c];
+// Exclusive scan of nchunks counts in place, the total behind them: one block,
+// each thread a run of them (one thread alone took 0.3 us a count).
+constexpr int kScanThreads = 1024;
+__global__ void __launch_bounds__(kScanThreads)
+k_scan_counts(int64_t *__restrict__ cnt, int64_t nchunks) {
+  __shared__ long long wsum[kScanThreads / 64];
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int64_t per = (nchunks + kScanThreads - 1) / kScanThreads;
+  const int64_t c0 = min(tid * per, nchunks), c1 = min(c0 + per, nchunks);
+  long long own = 0;
+  for (int64_t c = c0; c < c1; c++) own += cnt[c];
+  long long acc = own;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const long long o = __shfl_up(acc, d, 64);
+    if (lane >= d) acc += o;
+  }
+  if (lane == 63) wsum[wv] = acc;
+  __syncthreads();
+  for (int w = 0; w < wv; w++) acc += wsum[w];
+  if (tid == kScanThreads - 1) cnt[nchunks] = acc;
+  acc -= own;
+  for (int64_t c = c0; c < c1; c++) {
+    const int64_t v = cnt[c];
     cnt[c] = acc;
     acc += v;
   }
-  cnt[nchunks] = acc;
 }
 
 struct Rows7 {
@@ -651,7 +670,7 @@ int launch_compact(izh_bunch *b, double xrad, double yrad, int64_t nkeep) {
   hipLaunchKernelGGL(k_compact_count, dim3(nchunks), dim3(kBlock), 0, b->stream,
                      b->r[0], b->r[1], b->r[2], b->r[3], b->r[5], b->n, gam,
                      rad, cnt);
-  hipLaunchKernelGGL(k_scan_counts, dim3(1), dim3(64), 0, b->stream, cnt, nchunks);
+  hipLaunchKernelGGL(k_scan_counts, dim3(1), dim3(kScanThreads), 0, b->stream, cnt, nchunks);
   Rows7 src, dst;
   for (int r = 0; r < 6; r++) { src.r[r] = b->r[r]; dst.r[r] = b->r_alt[r]; }
   src.orig = b->orig;
@@ -815,6 +834,142 @@ int launch_clone(const izh_bunch *src, izh_bunch *dst, int64_t offset, int64_t n
                      dst->qm0, dst->w0, dst->id0, offset, n, w);
   IZH_HIP(hipGetLastError());
   return IZH_OK;
+}
+
+// --------------------------------------------------------------- download
+// Pts1(9,n) in the original order of the surviving particles (the reference's
+// compaction keeps it, src/Appl/BeamBunch.f90:1290,1345-1347): each original
+// index is marked with its slot, the marks are counted and scanned in chunks
+// of kCompactChunk, and each chunk writes its rows particle-major.
+namespace {
+constexpr uint32_t kNoSlot = 0xffffffffu;
+
+__global__ void __launch_bounds__(kBlock)
+k_pack_clear(uint32_t *__restrict__ mark, int64_t n0, unsigned long long *__restrict__ err) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *err = 0ull;
+  for (int64_t o = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; o < n0;
+       o += (int64_t)gridDim.x * blockDim.x)
+    mark[o] = kNoSlot;
+}
+
+// err counts indexes out of range and indexes two slots claim.
+__global__ void __launch_bounds__(kBlock)
+k_pack_mark(const uint32_t *__restrict__ orig, int64_t n, int64_t n0,
+            uint32_t *__restrict__ mark, unsigned long long *__restrict__ err) {
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
+       i += (int64_t)gridDim.x * blockDim.x) {
+    const uint32_t o = orig[i];
+    if ((int64_t)o >= n0 || atomicExch(&mark[o], (uint32_t)i) != kNoSlot) atomicAdd(err, 1ull);
+  }
+}
+
+__global__ void __launch_bounds__(kBlock)
+k_pack_count(const uint32_t *__restrict__ mark, int64_t n0, int64_t *__restrict__ cnt) {
+  const int64_t base = (int64_t)blockIdx.x * kCompactChunk;
+  int kept = 0;
+  for (int k = 0; k < kCompactChunk / kBlock; k++) {
+    const int64_t o = base + k * kBlock + threadIdx.x;
+    kept += __popcll(__ballot(o < n0 && mark[o] != kNoSlot));
+  }
+  __shared__ int sh[kBlock / 64];
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = kept;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int t = 0;
+    for (int w = 0; w < kBlock / 64; w++) t += sh[w];
+    cnt[blockIdx.x] = t;
+  }
+}
+
+// Chunks chunk0 + blockIdx.x; out starts at the row of chunk0's first survivor.
+__global__ void __launch_bounds__(kBlock)
+k_pack_rows(const uint32_t *__restrict__ mark, int64_t n0, const double *__restrict__ rows,
+            int64_t cap, const double *__restrict__ qm, const double *__restrict__ w,
+            const double *__restrict__ id, const int64_t *__restrict__ offs, int64_t chunk0,
+            double *__restrict__ out) {
+  const int64_t chunk = chunk0 + blockIdx.x, base = chunk * kCompactChunk;
+  int64_t at = offs[chunk] - offs[chunk0];
+  __shared__ int wsum[kBlock / 64];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  for (int k = 0; k < kCompactChunk / kBlock; k++) {
+    const int64_t o = base + k * kBlock + threadIdx.x;
+    const uint32_t slot = o < n0 ? mark[o] : kNoSlot;
+    const unsigned long long live = __ballot(slot != kNoSlot);
+    if (lane == 0) wsum[wv] = __popcll(live);
+    __syncthreads();
+    int before = __popcll(live & ((1ull << lane) - 1ull)), total = 0;
+    for (int v = 0; v < kBlock / 64; v++) {
+      if (v < wv) before += wsum[v];
+      total += wsum[v];
+    }
+    if (slot != kNoSlot) {
+      double *p = out + 9 * (at + before);
+#pragma unroll
+      for (int r = 0; r < 6; r++) p[r] = rows[r * cap + slot];
+      p[6] = qm[o];
+      p[7] = w[o];
+      p[8] = id[o];
+    }
+    at += total;
+    __syncthreads();
+  }
+}
+
+// Rows packed and copied at a time: 144 MB of scratch.
+constexpr int64_t kPackRows = 2000000;
+}  // namespace
+
+int launch_download(izh_bunch *b, double *pts9, bool *no_memory) {
+  *no_memory = false;
+  const int64_t n0 = b->n0, nch = (n0 + kCompactChunk - 1) / kCompactChunk;
+  const int64_t piece = std::min(b->n, kPackRows + kCompactChunk);
+  char *head = nullptr;
+  double *out = nullptr;
+  // the error count, the offsets, the marks
+  const size_t at_mark = (size_t)(nch + 2) * sizeof(int64_t);
+  if (dev_malloc((void **)&head, at_mark + (size_t)n0 * sizeof(uint32_t)) != hipSuccess ||
+      dev_malloc((void **)&out, (size_t)piece * 9 * sizeof(double)) != hipSuccess) {
+    dev_release(head);
+    *no_memory = true;
+    return IZH_OK;
+  }
+  unsigned long long *err = (unsigned long long *)head;
+  int64_t *offs = (int64_t *)head + 1;
+  uint32_t *mark = (uint32_t *)(head + at_mark);
+  const auto work = [&]() -> int {
+    hipLaunchKernelGGL(k_pack_clear, dim3(grid_for(n0)), dim3(kBlock), 0, b->stream, mark, n0,
+                       err);
+    hipLaunchKernelGGL(k_pack_mark, dim3(grid_for(b->n)), dim3(kBlock), 0, b->stream, b->orig,
+                       b->n, n0, mark, err);
+    hipLaunchKernelGGL(k_pack_count, dim3((unsigned)nch), dim3(kBlock), 0, b->stream, mark, n0,
+                       offs);
+    hipLaunchKernelGGL(k_scan_counts, dim3(1), dim3(kScanThreads), 0, b->stream, offs, nch);
+    IZH_HIP(hipGetLastError());
+    std::vector<int64_t> h((size_t)nch + 2);
+    IZH_HIP(hipMemcpyAsync(h.data(), head, h.size() * sizeof(int64_t), hipMemcpyDeviceToHost,
+                           b->stream));
+    IZH_HIP(hipStreamSynchronize(b->stream));
+    const int64_t *off = h.data() + 1;
+    if (h[0] != 0 || off[nch] != b->n)
+      return fail(IZH_ERR_STATE, "izh_bunch_download: corrupt particle index");
+    for (int64_t c0 = 0, c1; c0 < nch; c0 = c1) {
+      for (c1 = c0 + 1; c1 < nch && off[c1 + 1] - off[c0] <= piece; c1++) {}
+      const int64_t rows = off[c1] - off[c0];
+      if (rows == 0) continue;
+      hipLaunchKernelGGL(k_pack_rows, dim3((unsigned)(c1 - c0)), dim3(kBlock), 0, b->stream,
+                         mark, n0, b->r[0], b->cap, b->qm0, b->w0, b->id0, offs, c0, out);
+      IZH_HIP(hipGetLastError());
+      IZH_HIP(hipMemcpyAsync(pts9 + 9 * off[c0], out, (size_t)rows * 9 * sizeof(double),
+                             hipMemcpyDeviceToHost, b->stream));
+    }
+    IZH_HIP(hipStreamSynchronize(b->stream));
+    return IZH_OK;
+  };
+  const int rc = work();
+  if (rc != IZH_OK) (void)hipStreamSynchronize(b->stream);
+  dev_release(head);
+  dev_release(out);
+  return rc;
 }
 
 // ------------------------------------------------ allocation-free moments

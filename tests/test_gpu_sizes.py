@@ -158,3 +158,30 @@ def test_charge_forms(gpu, n, grid, uniform):
     b.close()
     f.close()
     assert err < 1e-13, err
+
+
+@pytest.mark.parametrize("n", [1, 2_047, 2_048, 2_049, 300_007, 4_003_000])
+@pytest.mark.parametrize("lossy", [False, True])
+def test_download_order(gpu, n, lossy):
+    """getpts returns the survivors in their original order: chunk edges of
+    the packing, and more rows than it copies at a time.  The t-frame position
+    is a few FP64 operations (1e-14)."""
+    print(f"download {n} lossy {lossy}", flush=True)
+    from impactz import beam as B
+    bm = B.Beam()
+    pts = B.gaussian_bunch(n, seed=4)
+    b = gpu.BeamBunch.from_beam(pts, bm)
+    rad = 1.5e-3 if lossy else 1.0
+    b.conv1st(0.0, rad, rad)
+    got = b.getpts()
+    rcp = 1.0 / (bm.gamma0 - pts[:, 5])
+    xt = (pts[:, 0] - pts[:, 1] * pts[:, 4] * rcp) * bm.scxl
+    yt = (pts[:, 2] - pts[:, 3] * pts[:, 4] * rcp) * bm.scxl
+    r = np.sqrt(xt * xt + yt * yt)
+    assert np.min(np.abs(r - rad)) > 1e-12     # no particle on the edge
+    keep = r < rad
+    b.close()
+    assert got.shape == (int(keep.sum()), 9)
+    assert np.array_equal(got[:, 6:], pts[keep, 6:])
+    assert np.array_equal(got[:, [1, 3, 5]], pts[keep][:, [1, 3, 5]])
+    assert np.max(np.abs(got[:, 0] - xt[keep]), initial=0.0) < 1e-14
