@@ -1291,8 +1291,12 @@ int run_lines(hipStream_t stream, Lines p, const void *tw, bool inverse) {
   const dim3 g((unsigned)nblk), b(kFftThreads);
   const cx<T> *twc = (const cx<T> *)tw;
   const int inv = inverse ? 1 : 0;
-  // the line lengths of the 64^3 .. 128x128x256 grids as compile-time sizes
+  // the line lengths of the 32^3 .. 128x128x256 grids as compile-time sizes
   switch (p.log2L) {
+    case 6:
+      hipLaunchKernelGGL((k_fft_lines<T, LOAD, STORE, CONV, PAIR, pts, 6>), g, b, tw_bytes,
+                         stream, p, twc, inv);
+      break;
     case 7:
       hipLaunchKernelGGL((k_fft_lines<T, LOAD, STORE, CONV, PAIR, pts, 7>), g, b, tw_bytes,
                          stream, p, twc, inv);
@@ -1327,6 +1331,10 @@ int run_two(hipStream_t stream, Lines ga, Lines cb, const void *tw) {
   const cx<T> *twc = (const cx<T> *)tw;
   const int na = (int)nba, nb = (int)nbb;
   switch (ga.log2L) {
+    case 6:
+      hipLaunchKernelGGL((k_fft_two<T, LOADA, LOADB, STOREB, PAIRB, 6>), g, b, tw_bytes,
+                         stream, ga, cb, na, nb, twc);
+      break;
     case 7:
       hipLaunchKernelGGL((k_fft_two<T, LOADA, LOADB, STOREB, PAIRB, 7>), g, b, tw_bytes,
                          stream, ga, cb, na, nb, twc);

@@ -70,7 +70,9 @@ struct PassCfg {
   uint32_t *cursor;         // kPassScatter: scatter cursor per tile of the input keys
   uint32_t *hist_new;       // kPassKeys: histogram of the output keys
   const DevDom *dom;        // domain of step s-1: gather and key geometry
-  const void *e;            // E4<T> of step s-1
+  const void *e;            // E4<T> of step s-1 (a pass with gather boxes)
+  const void *phi;          // T, its potential (a pass without)
+  int box;                  // which of the two
   const DevScal *scal;      // current and kick constants of step s-1
   DevScal *err;             // the same record, for the slot-overflow flag
   int nx, ny, nz;
@@ -344,6 +346,89 @@ __device__ inline void block_range(int64_t n, int64_t &lo, int64_t &hi) {
   hi = lo + per < n ? lo + per : n;
 }
 
+// Whether the passes of a run take gather boxes.  Where a block has few slots
+// its chain of chunk search, box and barriers is longer than the scattered
+// loads it saves, and where a tile has few particles a box is read by few.  A
+// pass without reads the potential itself, whose 32 values around a cell are
+// as many bytes as E on its eight nodes, so the step needs no E grid either.
+// Pass + E kernel with a box / pass without (us, 512 blocks unless said):
+//   slots a block <= 1024   100k on 32^3 (FP64) 16.2 + 3.3 / 14.2, 524k 33.0 +
+//                           3.5 / 30.2, 137k on 64^3 (mixed) 21.0 + 4.0 / 18.4
+//   2560, 4 slots a node    1M on 64^3 (mixed) 43.7 + 5.5 / 45.3, 1.2M on
+//                           64x64x128 52.5 + 6.0 / 53.8
+//   3/2 slots a node        2M on 128^3 (FP64, 1024 blocks) 130 + 20 / 137, 5M
+//                           on 128x128x256 (2048 blocks) 312 + 43 / 328
+// and past the lines 2M on 64^3 (FP64) 77 + 5.6 / 85, 10M on 128x128x256
+// (mixed) 378 + 19 / 488.
+inline bool pass_boxes(int64_t n, int nb, int64_t nodes) {
+  const int64_t slots = (n + nb - 1) / nb;
+  return !(slots <= 1024 || n <= nodes + nodes / 2 || (slots <= 2560 && n <= 4 * nodes));
+}
+
+// The field of step s-1 at a particle from the potential: E on the eight nodes
+// as k_efield forms it (central differences, one-sided at the edges), summed
+// in cic8's order.
+template <typename T>
+__device__ inline void gather_phi(const T *__restrict__ phi, int i, int j, int k, int nx, int ny,
+                                  int nz, const double *hinv, T ab, T cd, T ef, T &gx, T &gy,
+                                  T &gz) {
+  struct Pair { T a, b; };   // two neighbours along x
+  const int sy = nx, sz = nx * ny;
+  const T one = (T)1;
+  // neighbours of the cell's lower and upper node, the node itself at an edge
+  const int im = max(i - 1, 0), ip = min(i + 2, nx - 1);
+  const int jm = max(j - 1, 0), jp = min(j + 2, ny - 1);
+  const int km = max(k - 1, 0), kp = min(k + 2, nz - 1);
+  const auto at = [&](int a, int b, int c) { return (int64_t)a + (int64_t)sy * b + (int64_t)sz * c; };
+  const auto pair = [&](int b, int c) {
+    const T *q = phi + at(i, b, c);
+    return Pair{q[0], q[1]};
+  };
+  Pair in[2][2], yl[2], yu[2], zl[2], zu[2];
+  T xl[2][2], xu[2][2];
+#pragma unroll
+  for (int c = 0; c < 2; c++) {
+#pragma unroll
+    for (int b = 0; b < 2; b++) {
+      in[b][c] = pair(j + b, k + c);
+      xl[b][c] = phi[at(im, j + b, k + c)];
+      xu[b][c] = phi[at(ip, j + b, k + c)];
+    }
+    yl[c] = pair(jm, k + c);
+    yu[c] = pair(jp, k + c);
+  }
+#pragma unroll
+  for (int b = 0; b < 2; b++) {
+    zl[b] = pair(j + b, km);
+    zu[b] = pair(j + b, kp);
+  }
+  const T hx = (T)hinv[0], hy = (T)hinv[1], hz = (T)hinv[2];
+  const T hx2 = (T)(0.5 * hinv[0]), hy2 = (T)(0.5 * hinv[1]), hz2 = (T)(0.5 * hinv[2]);
+  const T fx[2] = {i == 0 ? hx : hx2, i + 1 == nx - 1 ? hx : hx2};
+  const T fy[2] = {j == 0 ? hy : hy2, j + 1 == ny - 1 ? hy : hy2};
+  const T fz[2] = {k == 0 ? hz : hz2, k + 1 == nz - 1 ? hz : hz2};
+  // nodes in cic8's order: (x, y, z) offsets of its index list
+  constexpr int da[8] = {0, 0, 0, 0, 1, 1, 1, 1}, db[8] = {0, 1, 1, 0, 0, 1, 1, 0},
+                dc[8] = {0, 0, 1, 1, 1, 1, 0, 0};
+  T sx = (T)0, syy = (T)0, szz = (T)0;
+#pragma unroll
+  for (int q = 0; q < 8; q++) {
+    const int a = da[q], b = db[q], c = dc[q];
+    const T w = (a ? one - ab : ab) * (b ? one - cd : cd) * (c ? one - ef : ef);
+    const auto of = [&](const Pair &p) { return a ? p.b : p.a; };
+    // lower minus upper neighbour
+    const T vx = fx[a] * ((a ? in[b][c].a : xl[b][c]) - (a ? xu[b][c] : in[b][c].b));
+    const T vy = fy[b] * ((b ? of(in[0][c]) : of(yl[c])) - (b ? of(yu[c]) : of(in[1][c])));
+    const T vz = fz[c] * ((c ? of(in[b][0]) : of(zl[b])) - (c ? of(zu[b]) : of(in[b][1])));
+    sx += vx * w;
+    syy += vy * w;
+    szz += vz * w;
+  }
+  gx = sx;
+  gy = syy;
+  gz = szz;
+}
+
 // Last of nch chunks that starts at or before slot lo (0 if none does), by
 // the whole block: each round cuts the candidates into kBlock steps and
 // counts the steps that start at or before lo, so two dependent loads cover
@@ -387,28 +472,28 @@ constexpr int kWalk = 8;      // chunk starts read at a time across sparse tiles
 // instead of four (2M on 64^3: 95 -> 91 us a pass).
 constexpr int kBoxBatch = 4;
 
-template <typename T> struct GatherLds;
-template <> struct GatherLds<double> {
+template <typename T, bool ON> struct GatherLds {};
+template <> struct GatherLds<double, true> {
   double2 xy[kGBoxCells];
   double z[kGBoxCells];
 };
-template <> struct GatherLds<float> {
+template <> struct GatherLds<float, true> {
   float4 e[kGBoxCells];
 };
 
-__device__ inline void box_store(GatherLds<double> &g, int q, const E4<double> &v) {
+__device__ inline void box_store(GatherLds<double, true> &g, int q, const E4<double> &v) {
   g.xy[q] = make_double2(v.x, v.y);
   g.z[q] = v.z;
 }
-__device__ inline void box_store(GatherLds<float> &g, int q, const E4<float> &v) {
+__device__ inline void box_store(GatherLds<float, true> &g, int q, const E4<float> &v) {
   g.e[q] = make_float4(v.x, v.y, v.z, 0.0f);
 }
-__device__ inline void box_load(const GatherLds<double> &g, int64_t q, double &x,
+__device__ inline void box_load(const GatherLds<double, true> &g, int64_t q, double &x,
                                 double &y, double &z) {
   const double2 v = g.xy[q];
   x = v.x; y = v.y; z = g.z[q];
 }
-__device__ inline void box_load(const GatherLds<float> &g, int64_t q, float &x,
+__device__ inline void box_load(const GatherLds<float, true> &g, int64_t q, float &x,
                                 float &y, float &z) {
   const float4 v = g.e[q];
   x = v.x; y = v.y; z = v.z;
@@ -467,18 +552,18 @@ __device__ inline void gather_batched(Load ld, int64_t o, int64_t sy, int64_t sz
 // a set of PassMode bits.  The slot loop is unrolled by two over two
 // register sets, so the loads of the next slot group land in the set not
 // being worked on.
-// Two blocks (wavefronts) per SIMD; three for an in-place pass with an FP32
-// grid and compile-time push kinds, which then spills at most 4 VGPRs and
+// Two blocks (wavefronts) per SIMD (a pass without gather boxes has no more
+// than that to run); three for an in-place pass with a box, an FP32 grid and compile-time push kinds, which then spills at most 4 VGPRs and
 // gains from the extra wavefront (measured: 3%).  FP64 would spill 70 VGPRs
 // to scratch at three (32% slower); a scatter pass's LDS (70 KB) allows two.
-template <typename T, int MODE, int KB>
+template <typename T, int MODE, int KB, bool BOX>
 constexpr int pass_blocks_per_cu(int ka) {
-  return ((MODE & kPassScatter) == 0 && sizeof(T) == 4 && KB != kPushAnyKind &&
+  return (BOX && (MODE & kPassScatter) == 0 && sizeof(T) == 4 && KB != kPushAnyKind &&
           ka != kPushAnyKind) ? 3 : 2;
 }
 
-template <typename T, int MODE, int KB, int KA>
-__global__ void __launch_bounds__(kBlock, (pass_blocks_per_cu<T, MODE, KB>(KA))) k_pass(PassCfg c) {
+template <typename T, int MODE, int KB, int KA, bool BOX>
+__global__ void __launch_bounds__(kBlock, (pass_blocks_per_cu<T, MODE, KB, BOX>(KA))) k_pass(PassCfg c) {
   constexpr bool kScatter = (MODE & kPassScatter) != 0, kKeys = (MODE & kPassKeys) != 0;
   const bool has_kick = KB == kPushAnyKind ? c.kb != kPushNone : KB != kPushNone;
   const bool has_conv = KA == kPushAnyKind ? c.ka != kPushNone : KA != kPushNone;
@@ -496,7 +581,7 @@ __global__ void __launch_bounds__(kBlock, (pass_blocks_per_cu<T, MODE, KB>(KA)))
   const int sy = c.nx, sz = c.nx * c.ny;
   const E4<T> *E = (const E4<T> *)c.e;
   T *tpx = (T *)c.tpos;
-  __shared__ GatherLds<T> gbox;
+  __shared__ GatherLds<T, BOX> gbox;
   constexpr bool kStage = kScatter && kStagedScatter;
   __shared__ ScatterStage<T, kStage> sg;
   __shared__ uint32_t key_hist[kKeys ? kPassLdsTiles : 1];
@@ -552,7 +637,7 @@ __global__ void __launch_bounds__(kBlock, (pass_blocks_per_cu<T, MODE, KB>(KA)))
   };
   auto load = [&](int64_t base, SlotIn &sl) {
     uint32_t k0 = kDeadKey;
-    if (has_kick && base < hi) {
+    if (BOX && has_kick && base < hi) {
       // the next chunk's start is held, so only a crossing loads; between
       // sparse tiles a group crosses many chunks, eight starts at a time
       if (nxt_start <= base) {
@@ -640,7 +725,7 @@ __global__ void __launch_bounds__(kBlock, (pass_blocks_per_cu<T, MODE, KB>(KA)))
     const double qm = c.need_orig ? c.qm0[sl.orig] : c.qm_value;
     if (has_kick) {
       // restage the gather box when the slot group starts another tile
-      if (kick && k0 != kDeadKey && k0 != box_key) {
+      if constexpr (BOX) if (kick && k0 != kDeadKey && k0 != box_key) {
         const uint32_t txy = (uint32_t)c.tnx * (uint32_t)c.tny;
         const int tz = (int)(k0 / txy), rem = (int)(k0 % txy);
         const int ty = rem / c.tnx, tx = rem % c.tnx;
@@ -691,22 +776,27 @@ __global__ void __launch_bounds__(kBlock, (pass_blocks_per_cu<T, MODE, KB>(KA)))
         jx = min(max(jx, 1), c.ny - 1);
         kx = min(max(kx, 1), c.nz - 1);
         T gx = (T)0, gy = (T)0, gz = (T)0;
-        const int li = ix - 1 - ox, lj = jx - 1 - oy, lk = kx - 1 - oz;
-        const bool inbox = box_key != kDeadKey && li >= 0 && li + 1 < bdx && lj >= 0 &&
-                           lj + 1 < bdy && lk >= 0 && lk + 1 < bdz;
-        if (valid && inbox) {
-          gather_batched<T>(
-              [](int64_t q, T &ex, T &ey, T &ez) { box_load(gbox, q, ex, ey, ez); },
-              (int64_t)li + (int64_t)bdx * (lj + bdy * lk), bdx, bdx * bdy, (T)ab, (T)cd,
-              (T)ef, gx, gy, gz);
+        if constexpr (BOX) {
+          const int li = ix - 1 - ox, lj = jx - 1 - oy, lk = kx - 1 - oz;
+          const bool inbox = box_key != kDeadKey && li >= 0 && li + 1 < bdx && lj >= 0 &&
+                             lj + 1 < bdy && lk >= 0 && lk + 1 < bdz;
+          if (valid && inbox) {
+            gather_batched<T>(
+                [](int64_t q, T &ex, T &ey, T &ez) { box_load(gbox, q, ex, ey, ez); },
+                (int64_t)li + (int64_t)bdx * (lj + bdy * lk), bdx, bdx * bdy, (T)ab, (T)cd,
+                (T)ef, gx, gy, gz);
+          } else if (valid) {
+            const int64_t o = (int64_t)(ix - 1) + (int64_t)sy * (jx - 1) + (int64_t)sz * (kx - 1);
+            gather_batched<T>(
+                [E](int64_t q, T &ex, T &ey, T &ez) {
+                  const E4<T> v = E[q];
+                  ex = v.x; ey = v.y; ez = v.z;
+                },
+                o, sy, sz, (T)ab, (T)cd, (T)ef, gx, gy, gz);
+          }
         } else if (valid) {
-          const int64_t o = (int64_t)(ix - 1) + (int64_t)sy * (jx - 1) + (int64_t)sz * (kx - 1);
-          gather_batched<T>(
-              [E](int64_t q, T &ex, T &ey, T &ez) {
-                const E4<T> v = E[q];
-                ex = v.x; ey = v.y; ez = v.z;
-              },
-              o, sy, sz, (T)ab, (T)cd, (T)ef, gx, gy, gz);
+          gather_phi<T>((const T *)c.phi, ix - 1, jx - 1, kx - 1, c.nx, c.ny, c.nz, c.dom->hinv,
+                        (T)ab, (T)cd, (T)ef, gx, gy, gz);
         }
         const double exn = (double)gx * c.gam_k, eyn = (double)gy * c.gam_k, ezn = (double)gz;
         if (valid) {
@@ -867,7 +957,7 @@ __global__ void __launch_bounds__(kBlock, (pass_blocks_per_cu<T, MODE, KB>(KA)))
   if (lo < hi) {
     // the first group's rows are on their way while the block finds its chunk
     load_rows(lo, sa);
-    if (has_kick) {
+    if (BOX && has_kick) {
       __shared__ int red[kBlock / 64];
       nch = (int)*(__attribute__((address_space(4))) const int64_t *)c.in_nchunks;
       if (nch > 0) {
@@ -876,7 +966,7 @@ __global__ void __launch_bounds__(kBlock, (pass_blocks_per_cu<T, MODE, KB>(KA)))
         nxt_start = ci + 1 < nch ? (int64_t)chs[ci + 1].start : INT64_MAX;
       }
     }
-    sa.k0 = nxt_start - lo >= kStageMin ? cur_tile : kDeadKey;
+    sa.k0 = cur_tile != kDeadKey && nxt_start - lo >= kStageMin ? cur_tile : kDeadKey;
     step(sa, (uint32_t)__builtin_amdgcn_readfirstlane((int)sa.k0), lo, 0,
          [&] { load(lo + kBlock, sb); });
     for (int64_t base = lo + kBlock; base < hi; base += 2 * kBlock) {
@@ -922,21 +1012,29 @@ __global__ void __launch_bounds__(kBlock, (pass_blocks_per_cu<T, MODE, KB>(KA)))
   }
 }
 
-template <typename T, int KB, int KA>
-void launch_pass_kinds(int mode, int nb, hipStream_t st, const PassCfg &pc) {
+template <typename T, int KB, int KA, bool BOX>
+void launch_pass_mode(int mode, int nb, hipStream_t st, const PassCfg &pc) {
   const dim3 g(nb), b(kBlock);
   switch (mode) {
     case kPassInPlace:
-      hipLaunchKernelGGL((k_pass<T, kPassInPlace, KB, KA>), g, b, 0, st, pc);
+      hipLaunchKernelGGL((k_pass<T, kPassInPlace, KB, KA, BOX>), g, b, 0, st, pc);
       break;
-    case kPassKeys: hipLaunchKernelGGL((k_pass<T, kPassKeys, KB, KA>), g, b, 0, st, pc); break;
+    case kPassKeys:
+      hipLaunchKernelGGL((k_pass<T, kPassKeys, KB, KA, BOX>), g, b, 0, st, pc);
+      break;
     case kPassScatter:
-      hipLaunchKernelGGL((k_pass<T, kPassScatter, KB, KA>), g, b, 0, st, pc);
+      hipLaunchKernelGGL((k_pass<T, kPassScatter, KB, KA, BOX>), g, b, 0, st, pc);
       break;
     default:
-      hipLaunchKernelGGL((k_pass<T, kPassScatter | kPassKeys, KB, KA>), g, b, 0, st, pc);
+      hipLaunchKernelGGL((k_pass<T, kPassScatter | kPassKeys, KB, KA, BOX>), g, b, 0, st, pc);
       break;
   }
+}
+
+template <typename T, int KB, int KA>
+void launch_pass_kinds(int mode, int nb, hipStream_t st, const PassCfg &pc) {
+  if (pc.box) launch_pass_mode<T, KB, KA, true>(mode, nb, st, pc);
+  else launch_pass_mode<T, KB, KA, false>(mode, nb, st, pc);
 }
 
 // Drift, map and none as compile-time kinds (3 x 3); the run-time form
@@ -1362,6 +1460,8 @@ struct Runner {
   hipStream_t st = nullptr, fstream = nullptr;
   int nx = 0, ny = 0, nz = 0, s0 = 0, s1 = 0, s2 = 0, tnx = 0, tny = 0, ntiles = 0;
   int nb = 0, period = 1;
+  bool boxes = true;   // the passes gather E through boxes (else from phi)
+  bool e_made = false; // the last step launched left E (else phi alone)
   int g_cur = 1, g_next = 0;
   int64_t total = 0;   // steps of the run
   int64_t s = 0;       // index of the next pass
@@ -1403,6 +1503,7 @@ struct Runner {
     const double wsum = b->wabs_sum > 0 ? b->wabs_sum : 1.0;
     const double rho_scale = f->precision == IZH_FP64 ? 1.0 : 1.0 / wsum;
     nb = pass_blocks(b->n, ntiles);
+    boxes = pass_boxes(b->n, nb, (int64_t)nx * ny * nz);
     period = b->resort_period > 0 ? b->resort_period : kDefaultResortPeriod;
     refpt_after.assign(2 * (size_t)total, 0.0);
     // Two chunk lists (with their key grids and counts) describe groupings
@@ -1481,6 +1582,7 @@ struct Runner {
     pc.hist_new = hist;
     pc.dom = f->d_dom;
     pc.e = f->e;
+    pc.phi = f->phi;
     pc.scal = b->d_scal;
     pc.err = b->d_scal;
     pc.nx = nx; pc.ny = ny; pc.nz = nz;
@@ -1532,6 +1634,7 @@ struct Runner {
     pc.in_chunks = b->chunks + g_cur * b->nchunks_cap;
     pc.in_nchunks = &b->d_scal->nchunks[g_cur];
     pc.kgrid = &f->d_dom->kgrid[g_cur];
+    pc.box = e_made ? 1 : 0;  // E of step s-1, or its potential
     pc.kb = kb_prev;
     pc.ka = ka;
     pc.pb = pb_prev;
@@ -1572,13 +1675,16 @@ struct Runner {
     s++;
     if (last) return IZH_OK;
     const int64_t step = s - 1;
+    // a wake adds to E, and the last step leaves E for the caller
+    const bool makes_e = boxes || step == total - 1 || (seg->wake && seg->wake->kind != 0);
+    e_made = makes_e;
     if (!dry) {
       // charge, update3O and the E field of step s on the grouping the slots are in
       const Chunk *dch = b->chunks + g_cur * b->nchunks_cap;
       IZH_CHECK(launch_deposit(b, f, dch, &f->d_dom->kgrid[g_cur],
                                &b->d_scal->nchunks[g_cur], b->nchunks_cap));
       IZH_CHECK(launch_convolve_fx(f));
-      IZH_CHECK(launch_efield(f));
+      if (makes_e) IZH_CHECK(launch_efield(f));
       // the step's wakefield (src/Contrl/AccSimulator.f90:1272-1338) from the
       // same t positions, into E before the next pass kicks
       if (seg->wake && seg->wake->kind != 0) {

@@ -108,6 +108,11 @@ def test_solve_line_lengths(gpu, grid):
     (257, (16, 16, 16), 2),          # two blocks, one of a single slot
     (3_000, (128, 128, 128), 2),     # a group crosses hundreds of tiles
     (131_073, (64, 64, 128), 3),     # the first bunch of two groups a block
+    (524_288, (32, 32, 32), 2),      # the last pass that kicks from phi
+    (524_289, (32, 32, 32), 2),      # the first that gathers E through a box
+    (70_000, (4, 4, 4), 2),          # from phi, every cell at an edge
+    (786_432, (64, 64, 128), 2),     # 3/2 of the nodes
+    (1_048_577, (64, 64, 64), 2),    # past four times the nodes
     (1_500_001, (64, 64, 128), 2),   # the first pass of 1024 blocks
     (4_000_001, (64, 64, 128), 2),   # and of 2048
 ])
