@@ -773,7 +773,9 @@ k_igf(double *__restrict__ out, T *__restrict__ far, int nx, int ny, int nz,
 
 // --------------------------------------------------------------- deposit
 // Lower-node cell (0-based) and CIC weights of deposit_BeamBunch
-// (src/Appl/BeamBunch.f90:3737-3744) in the position type P.
+// (src/Appl/BeamBunch.f90:3737-3744) in the position type P.  The multiply and
+// the add are fused by name, as the compiler fuses them: the kernels of one
+// binned deposit then agree on every particle's cell by construction.
 template <typename P>
 struct Cic {
   int i, j, k;
@@ -784,11 +786,11 @@ template <typename P>
 __device__ inline Cic<P> cic_of(P x, P y, P z, P xmin, P ymin, P zmin, P hx, P hy,
                                 P hz, P hxi, P hyi, P hzi) {
   Cic<P> c;
-  int ix = (int)((x - xmin) * hxi + (P)1);
+  int ix = (int)fma(x - xmin, hxi, (P)1);
   c.ab = ((xmin - x) + ix * hx) * hxi;
-  int jx = (int)((y - ymin) * hyi + (P)1);
+  int jx = (int)fma(y - ymin, hyi, (P)1);
   c.cd = ((ymin - y) + jx * hy) * hyi;
-  int kx = (int)((z - zmin) * hzi + (P)1);
+  int kx = (int)fma(z - zmin, hzi, (P)1);
   c.ef = ((zmin - z) + kx * hz) * hzi;
   c.i = ix - 1;
   c.j = jx - 1;
