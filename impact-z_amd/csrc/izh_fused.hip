@@ -9,7 +9,7 @@
 // grouped by the tile key computed one step earlier (a counting sort whose
 // histogram and scan were done by the previous k_finalize): neighbours in
 // memory stay neighbours in space, so the gather hits cache and the deposit
-// (izh_field.hip, k_deposit_chunks) accumulates each chunk in LDS.
+// (izh_field.hip, k_deposit_tiles) accumulates each chunk in LDS.
 // k_finalize (one block) then reduces the pass's partials into the step's
 // moments, the new domain (update_CompDom), particle count, Current rescale
 // and kick constants, scans the new tile histogram into scatter cursors and
@@ -57,6 +57,11 @@ enum PushKind : int {
 // histogram, for a scatter in the next pass.
 enum PassMode : int { kPassInPlace = 0, kPassScatter = 1, kPassKeys = 2 };
 
+// Where a pass takes the field from, and how it reads and writes the rows.
+// kFormPhi: from the potential, 32 values a particle.  kFormBox: from E through
+// gather boxes.  kFormStream: with boxes, and the rows past the caches.
+enum PassForm : int { kFormPhi = 0, kFormBox = 1, kFormStream = 2 };
+
 struct PassCfg {
   const double *in;         // six rows of cap doubles, row k at in + k*cap
   double *out;              // (== in for a pass without kPassScatter)
@@ -72,7 +77,7 @@ struct PassCfg {
   const DevDom *dom;        // domain of step s-1: gather and key geometry
   const void *e;            // E4<T> of step s-1 (a pass with gather boxes)
   const void *phi;          // T, its potential (a pass without)
-  int box;                  // which of the two
+  int form;                 // PassForm
   const DevScal *scal;      // current and kick constants of step s-1
   DevScal *err;             // the same record, for the slot-overflow flag
   int nx, ny, nz;
@@ -365,6 +370,20 @@ inline bool pass_boxes(int64_t n, int nb, int64_t nodes) {
   return !(slots <= 1024 || n <= nodes + nodes / 2 || (slots <= 2560 && n <= 4 * nodes));
 }
 
+// Whether the passes read the rows (and in place write them) by non-temporal
+// accesses: once the six rows outgrow the 256 MB last-level cache the next
+// pass finds nothing of them there, and what they push out (the field, the t
+// positions the deposit reads next, the lines a scatter is still filling) is
+// missed.  16 steps by ordinary accesses / so (ms): 7M on 64x64x128 (mixed)
+// 8.57 / 8.15, 7M on 128^3 (FP64) 14.04 / 13.74, 10M on 64^3 (FP64) 11.35 /
+// 10.56, 10M on 128x128x256 (mixed) 18.85 / 18.34, 50M (FP64) 63.1 / 61.9;
+// below the line either sign: 2.5M on 64x64x128 (mixed) 4.40 / 4.46, 4M 6.05 /
+// 5.88, 5M on 128^3 (FP64) 11.90 / 11.87.  A scatter's stores stay ordinary
+// (their lines fill over several groups), and so do the t positions' (10M on
+// 64^3 10.62 with them, 50M 61.5).
+constexpr int64_t kCacheBytes = (int64_t)256 << 20;
+inline bool pass_streams(int64_t n) { return 6 * (int64_t)sizeof(double) * n > kCacheBytes; }
+
 // The field of step s-1 at a particle from the potential: E on the eight nodes
 // as k_efield forms it (central differences, one-sided at the edges), summed
 // in cic8's order.
@@ -499,6 +518,18 @@ __device__ inline void box_load(const GatherLds<float, true> &g, int64_t q, floa
   x = v.x; y = v.y; z = v.z;
 }
 
+// A row's value, past the caches (PAST: the non-temporal forms) or not.
+template <bool PAST>
+__device__ inline double load_row(const double *p) {
+  if constexpr (PAST) return __builtin_nontemporal_load(p);
+  else return *p;
+}
+template <bool PAST>
+__device__ inline void store_row(double *p, double v) {
+  if constexpr (PAST) __builtin_nontemporal_store(v, p);
+  else *p = v;
+}
+
 // One slot of the pass's input, read an iteration before it is processed.
 // The loaded values are kept as loaded (a lane past the range holds its
 // block's last slot): nothing between the loads and the next group's first
@@ -556,14 +587,16 @@ __device__ inline void gather_batched(Load ld, int64_t o, int64_t sy, int64_t sz
 // than that to run); three for an in-place pass with a box, an FP32 grid and compile-time push kinds, which then spills at most 4 VGPRs and
 // gains from the extra wavefront (measured: 3%).  FP64 would spill 70 VGPRs
 // to scratch at three (32% slower); a scatter pass's LDS (70 KB) allows two.
-template <typename T, int MODE, int KB, bool BOX>
+template <typename T, int MODE, int KB, int FORM>
 constexpr int pass_blocks_per_cu(int ka) {
-  return (BOX && (MODE & kPassScatter) == 0 && sizeof(T) == 4 && KB != kPushAnyKind &&
+  return (FORM != kFormPhi && (MODE & kPassScatter) == 0 && sizeof(T) == 4 && KB != kPushAnyKind &&
           ka != kPushAnyKind) ? 3 : 2;
 }
 
-template <typename T, int MODE, int KB, int KA, bool BOX>
-__global__ void __launch_bounds__(kBlock, (pass_blocks_per_cu<T, MODE, KB, BOX>(KA))) k_pass(PassCfg c) {
+template <typename T, int MODE, int KB, int KA, int FORM>
+__global__ void __launch_bounds__(kBlock, (pass_blocks_per_cu<T, MODE, KB, FORM>(KA))) k_pass(PassCfg c) {
+  constexpr bool BOX = FORM != kFormPhi;
+  constexpr bool kPast = FORM == kFormStream;
   constexpr bool kScatter = (MODE & kPassScatter) != 0, kKeys = (MODE & kPassKeys) != 0;
   const bool has_kick = KB == kPushAnyKind ? c.kb != kPushNone : KB != kPushNone;
   const bool has_conv = KA == kPushAnyKind ? c.ka != kPushNone : KA != kPushNone;
@@ -630,7 +663,7 @@ __global__ void __launch_bounds__(kBlock, (pass_blocks_per_cu<T, MODE, KB, BOX>(
       if (c.need_orig) og = c.in_orig[jj];
     }
 #pragma unroll
-    for (int k = 0; k < 6; k++) sl.r[k] = c.in[k * cap + jj];
+    for (int k = 0; k < 6; k++) sl.r[k] = load_row<kPast>(c.in + k * cap + jj);
     sl.in = j < hi;
     sl.key = key;
     sl.orig = og;
@@ -929,12 +962,12 @@ __global__ void __launch_bounds__(kBlock, (pass_blocks_per_cu<T, MODE, KB, BOX>(
     double *sd = (double *)c.sink + lane;
     uint32_t *su = (uint32_t *)((double *)c.sink + 8 * 64) + lane;
     T *st = (T *)((double *)c.sink + 10 * 64) + lane;
-    (ok ? c.out[slot] : sd[0]) = x;
-    (ok ? c.out[cap + slot] : sd[64]) = px;
-    (ok ? c.out[2 * cap + slot] : sd[128]) = y;
-    (ok ? c.out[3 * cap + slot] : sd[192]) = py;
-    (ok ? c.out[4 * cap + slot] : sd[256]) = ph;
-    (ok ? c.out[5 * cap + slot] : sd[320]) = pt;
+    store_row<kPast && !kScatter>(ok ? &c.out[slot] : sd + 0, x);
+    store_row<kPast && !kScatter>(ok ? &c.out[cap + slot] : sd + 64, px);
+    store_row<kPast && !kScatter>(ok ? &c.out[2 * cap + slot] : sd + 128, y);
+    store_row<kPast && !kScatter>(ok ? &c.out[3 * cap + slot] : sd + 192, py);
+    store_row<kPast && !kScatter>(ok ? &c.out[4 * cap + slot] : sd + 256, ph);
+    store_row<kPast && !kScatter>(ok ? &c.out[5 * cap + slot] : sd + 320, pt);
     if constexpr (kScatter) (ok ? c.out_orig[slot] : su[0]) = sl.orig;
     // In place, the key of EVERY slot of the block's range is rewritten: the
     // slot of a particle lost before this pass takes kDeadKey, so the next
@@ -1012,29 +1045,37 @@ __global__ void __launch_bounds__(kBlock, (pass_blocks_per_cu<T, MODE, KB, BOX>(
   }
 }
 
-template <typename T, int KB, int KA, bool BOX>
+template <typename T, int KB, int KA, int FORM>
 void launch_pass_mode(int mode, int nb, hipStream_t st, const PassCfg &pc) {
   const dim3 g(nb), b(kBlock);
   switch (mode) {
     case kPassInPlace:
-      hipLaunchKernelGGL((k_pass<T, kPassInPlace, KB, KA, BOX>), g, b, 0, st, pc);
+      hipLaunchKernelGGL((k_pass<T, kPassInPlace, KB, KA, FORM>), g, b, 0, st, pc);
       break;
     case kPassKeys:
-      hipLaunchKernelGGL((k_pass<T, kPassKeys, KB, KA, BOX>), g, b, 0, st, pc);
+      hipLaunchKernelGGL((k_pass<T, kPassKeys, KB, KA, FORM>), g, b, 0, st, pc);
       break;
     case kPassScatter:
-      hipLaunchKernelGGL((k_pass<T, kPassScatter, KB, KA, BOX>), g, b, 0, st, pc);
+      hipLaunchKernelGGL((k_pass<T, kPassScatter, KB, KA, FORM>), g, b, 0, st, pc);
       break;
     default:
-      hipLaunchKernelGGL((k_pass<T, kPassScatter | kPassKeys, KB, KA, BOX>), g, b, 0, st, pc);
+      hipLaunchKernelGGL((k_pass<T, kPassScatter | kPassKeys, KB, KA, FORM>), g, b, 0, st, pc);
       break;
   }
 }
 
 template <typename T, int KB, int KA>
 void launch_pass_kinds(int mode, int nb, hipStream_t st, const PassCfg &pc) {
-  if (pc.box) launch_pass_mode<T, KB, KA, true>(mode, nb, st, pc);
-  else launch_pass_mode<T, KB, KA, false>(mode, nb, st, pc);
+  // without a kick there is no field to take
+  if constexpr (KB == kPushNone) {
+    launch_pass_mode<T, KB, KA, kFormPhi>(mode, nb, st, pc);
+  } else if (pc.form == kFormStream) {
+    launch_pass_mode<T, KB, KA, kFormStream>(mode, nb, st, pc);
+  } else if (pc.form == kFormBox) {
+    launch_pass_mode<T, KB, KA, kFormBox>(mode, nb, st, pc);
+  } else {
+    launch_pass_mode<T, KB, KA, kFormPhi>(mode, nb, st, pc);
+  }
 }
 
 // Drift, map and none as compile-time kinds (3 x 3); the run-time form
@@ -1461,6 +1502,7 @@ struct Runner {
   int nx = 0, ny = 0, nz = 0, s0 = 0, s1 = 0, s2 = 0, tnx = 0, tny = 0, ntiles = 0;
   int nb = 0, period = 1;
   bool boxes = true;   // the passes gather E through boxes (else from phi)
+  bool past = false;   // and take the rows past the caches
   bool e_made = false; // the last step launched left E (else phi alone)
   int g_cur = 1, g_next = 0;
   int64_t total = 0;   // steps of the run
@@ -1504,6 +1546,7 @@ struct Runner {
     const double rho_scale = f->precision == IZH_FP64 ? 1.0 : 1.0 / wsum;
     nb = pass_blocks(b->n, ntiles);
     boxes = pass_boxes(b->n, nb, (int64_t)nx * ny * nz);
+    past = pass_streams(b->n);
     period = b->resort_period > 0 ? b->resort_period : kDefaultResortPeriod;
     refpt_after.assign(2 * (size_t)total, 0.0);
     // Two chunk lists (with their key grids and counts) describe groupings
@@ -1634,7 +1677,7 @@ struct Runner {
     pc.in_chunks = b->chunks + g_cur * b->nchunks_cap;
     pc.in_nchunks = &b->d_scal->nchunks[g_cur];
     pc.kgrid = &f->d_dom->kgrid[g_cur];
-    pc.box = e_made ? 1 : 0;  // E of step s-1, or its potential
+    pc.form = !e_made ? kFormPhi : (past ? kFormStream : kFormBox);
     pc.kb = kb_prev;
     pc.ka = ka;
     pc.pb = pb_prev;

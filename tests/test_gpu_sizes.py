@@ -190,3 +190,12 @@ def test_download_order(gpu, n, lossy):
     assert np.array_equal(got[:, 6:], pts[keep, 6:])
     assert np.array_equal(got[:, [1, 3, 5]], pts[keep][:, [1, 3, 5]])
     assert np.max(np.abs(got[:, 0] - xt[keep]), initial=0.0) < 1e-14
+
+
+@pytest.mark.parametrize("n,grid,period", [
+    (5_592_405, (64, 64, 64), 2),    # rows of the cache's 256 MB: the last ordinary ones
+    (5_592_406, (64, 64, 64), 2),    # the first read past it
+    (5_592_999, (64, 64, 64), 1),    # scatters only, a ragged last block
+])
+def test_streamed_rows(gpu, n, grid, period):
+    run_against_step(gpu, n, grid, period, steps=4)
