@@ -380,7 +380,9 @@ inline bool pass_boxes(int64_t n, int nb, int64_t nodes) {
 // below the line either sign: 2.5M on 64x64x128 (mixed) 4.40 / 4.46, 4M 6.05 /
 // 5.88, 5M on 128^3 (FP64) 11.90 / 11.87.  A scatter's stores stay ordinary
 // (their lines fill over several groups), and so do the t positions' (10M on
-// 64^3 10.62 with them, 50M 61.5).
+// 64^3 10.62 with them, 50M 61.5).  The first pass, which scatters unsorted rows, has
+// its open lines displaced most: with it 50M 61.7 -> 61.4, 10M on 128x128x256
+// 18.36 -> 18.24.
 constexpr int64_t kCacheBytes = (int64_t)256 << 20;
 inline bool pass_streams(int64_t n) { return 6 * (int64_t)sizeof(double) * n > kCacheBytes; }
 
@@ -519,13 +521,13 @@ __device__ inline void box_load(const GatherLds<float, true> &g, int64_t q, floa
 }
 
 // A row's value, past the caches (PAST: the non-temporal forms) or not.
-template <bool PAST>
-__device__ inline double load_row(const double *p) {
+template <bool PAST, typename T>
+__device__ inline T load_row(const T *p) {
   if constexpr (PAST) return __builtin_nontemporal_load(p);
   else return *p;
 }
-template <bool PAST>
-__device__ inline void store_row(double *p, double v) {
+template <bool PAST, typename T>
+__device__ inline void store_row(T *p, T v) {
   if constexpr (PAST) __builtin_nontemporal_store(v, p);
   else *p = v;
 }
@@ -657,8 +659,8 @@ __global__ void __launch_bounds__(kBlock, (pass_blocks_per_cu<T, MODE, KB, FORM>
     const int64_t jj = j < hi ? j : hi - 1;
     uint32_t key = 0u, og = 0u;
     if constexpr (kScatter) {
-      key = c.in_key[jj];
-      og = c.in_orig[jj];
+      key = load_row<kPast>(c.in_key + jj);
+      og = load_row<kPast>(c.in_orig + jj);
     } else {
       if (c.need_orig) og = c.in_orig[jj];
     }
@@ -1066,16 +1068,20 @@ void launch_pass_mode(int mode, int nb, hipStream_t st, const PassCfg &pc) {
 
 template <typename T, int KB, int KA>
 void launch_pass_kinds(int mode, int nb, hipStream_t st, const PassCfg &pc) {
-  // without a kick there is no field to take
-  if constexpr (KB == kPushNone) {
-    launch_pass_mode<T, KB, KA, kFormPhi>(mode, nb, st, pc);
-  } else if (pc.form == kFormStream) {
+  // without a kick there is no field to take: no box, which a run-time kind
+  // would carry for nothing
+  const bool no_box = KB == kPushAnyKind && pc.kb == kPushNone;
+  if (pc.form == kFormStream && !no_box) {
     launch_pass_mode<T, KB, KA, kFormStream>(mode, nb, st, pc);
-  } else if (pc.form == kFormBox) {
-    launch_pass_mode<T, KB, KA, kFormBox>(mode, nb, st, pc);
-  } else {
-    launch_pass_mode<T, KB, KA, kFormPhi>(mode, nb, st, pc);
+    return;
   }
+  if constexpr (KB != kPushNone) {
+    if (pc.form == kFormBox && !no_box) {
+      launch_pass_mode<T, KB, KA, kFormBox>(mode, nb, st, pc);
+      return;
+    }
+  }
+  launch_pass_mode<T, KB, KA, kFormPhi>(mode, nb, st, pc);
 }
 
 // Drift, map and none as compile-time kinds (3 x 3); the run-time form
@@ -1677,7 +1683,8 @@ struct Runner {
     pc.in_chunks = b->chunks + g_cur * b->nchunks_cap;
     pc.in_nchunks = &b->d_scal->nchunks[g_cur];
     pc.kgrid = &f->d_dom->kgrid[g_cur];
-    pc.form = !e_made ? kFormPhi : (past ? kFormStream : kFormBox);
+    // (the first pass kicks nothing: only how it reads the rows counts)
+    pc.form = past && (e_made || s == 0) ? kFormStream : (e_made ? kFormBox : kFormPhi);
     pc.kb = kb_prev;
     pc.ka = ka;
     pc.pb = pb_prev;
