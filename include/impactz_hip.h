@@ -455,9 +455,11 @@ int izh_probe_copy(int64_t nbytes, double *ms);
  * of timed launches (both IZH_T_COUNT long) and optionally resets them. */
 #define IZH_T_PUSH 0       /* drift1 / map apply */
 #define IZH_T_CONV1ST 1    /* conv1st + range reduction */
-#define IZH_T_DEPOSIT 2    /* CIC deposition (charge_BeamBunch) */
-#define IZH_T_GREEN 3      /* integrated Green function + its transform */
-#define IZH_T_FFT 4        /* rho -> phi convolution passes */
+#define IZH_T_DEPOSIT 2    /* CIC deposition (charge_BeamBunch); in izh_run with
+                              the Green function's values, formed beside it */
+#define IZH_T_GREEN 3      /* integrated Green function's values (izh_update3O) */
+#define IZH_T_FFT 4        /* rho -> phi: transforms of the Green function and
+                              of the charge, convolution */
 #define IZH_T_EFIELD 5     /* E = -grad phi */
 #define IZH_T_KICK 6       /* gather + kick + back transform (scatter1) */
 #define IZH_T_CVBK 7       /* cvbkforth1st */
