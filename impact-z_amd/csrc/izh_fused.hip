@@ -370,19 +370,20 @@ inline bool pass_boxes(int64_t n, int nb, int64_t nodes) {
   return !(slots <= 1024 || n <= nodes + nodes / 2 || (slots <= 2560 && n <= 4 * nodes));
 }
 
-// Whether the passes read the rows (and in place write them) by non-temporal
-// accesses: once the six rows outgrow the 256 MB last-level cache the next
-// pass finds nothing of them there, and what they push out (the field, the t
-// positions the deposit reads next, the lines a scatter is still filling) is
-// missed.  16 steps by ordinary accesses / so (ms): 7M on 64x64x128 (mixed)
+// Whether the passes read and write the rows by non-temporal accesses: once
+// the six rows outgrow the 256 MB last-level cache the next pass finds nothing
+// of them there, and what they push out (the field, the t positions the deposit
+// reads next, the lines a scatter is still filling) is missed.  16 steps by ordinary accesses / so (ms): 7M on 64x64x128 (mixed)
 // 8.57 / 8.15, 7M on 128^3 (FP64) 14.04 / 13.74, 10M on 64^3 (FP64) 11.35 /
 // 10.56, 10M on 128x128x256 (mixed) 18.85 / 18.34, 50M (FP64) 63.1 / 61.9;
 // below the line either sign: 2.5M on 64x64x128 (mixed) 4.40 / 4.46, 4M 6.05 /
-// 5.88, 5M on 128^3 (FP64) 11.90 / 11.87.  A scatter's stores stay ordinary
-// (their lines fill over several groups), and so do the t positions' (10M on
-// 64^3 10.62 with them, 50M 61.5).  The first pass, which scatters unsorted rows, has
-// its open lines displaced most: with it 50M 61.7 -> 61.4, 10M on 128x128x256
-// 18.36 -> 18.24.
+// 5.88, 5M on 128^3 (FP64) 11.90 / 11.87.  The first pass, which scatters
+// unsorted rows, has its open lines displaced most: with it 50M 61.7 -> 61.4,
+// 10M on 128x128x256 18.36 -> 18.24.  It stores by ordinary accesses (its lines
+// fill over many groups); the later scatters, whose runs of a tile are long, go
+// past the caches too: 10M on 128x128x256 16.76 -> 16.44, 7M on 128^3 13.35 ->
+// 13.08, 10M on 128^3 16.56 -> 16.25, on 64^3 and 64x64x128 the same within 1%.
+// The t positions are read next and stay ordinary (10M on 64^3 10.56 -> 10.62).
 constexpr int64_t kCacheBytes = (int64_t)256 << 20;
 inline bool pass_streams(int64_t n) { return 6 * (int64_t)sizeof(double) * n > kCacheBytes; }
 
@@ -939,7 +940,8 @@ __global__ void __launch_bounds__(kBlock, (pass_blocks_per_cu<T, MODE, KB, FORM>
       uint32_t *su = (uint32_t *)((double *)c.sink + 8 * 64) + lane;
       T *stt = (T *)((double *)c.sink + 10 * 64) + lane;
 #pragma unroll
-      for (int k = 0; k < 6; k++) (ok ? c.out[k * cap + q] : sd[64 * k]) = sg.row[k][t];
+      for (int k = 0; k < 6; k++)
+        store_row<kPast && KB != kPushNone>(ok ? c.out + k * cap + q : sd + 64 * k, sg.row[k][t]);
       (ok ? c.out_orig[q] : su[0]) = sg.orig[t];
       if constexpr (kKeys) (ok ? c.out_key[q] : su[64]) = sg.nkey[t];
       if (has_conv) {
