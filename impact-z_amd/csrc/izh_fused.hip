@@ -1755,15 +1755,24 @@ struct Runner {
     return IZH_OK;
   }
 
-  // Give the field its own stream back (after an error too).
+  // Give the field its own stream back.  Everything of the run is queued on the
+  // bunch's, so it ends first: whoever waits for the field's stream alone (its
+  // destroy call, which passes its buffers on) would not see it.
   void release() {
-    if (began) f->stream = fstream;
+    if (!began) return;
+    (void)hipStreamSynchronize(st);
+    f->stream = fstream;
     began = false;
   }
 
-  // After the last pass: wait for the stream and take the results.
+  // After the last pass: take the results.
   int end(izh_compdom *dom, double *moments) {
+    const int rc = results(dom, moments);
     release();
+    return rc;
+  }
+
+  int results(izh_compdom *dom, double *moments) {
     IZH_HIP(hipMemcpyAsync(b->h_scal, b->d_scal, sizeof(DevScal), hipMemcpyDeviceToHost,
                            st));
     IZH_HIP(hipMemcpyAsync(f->h_dom, f->d_dom, sizeof(DevDom), hipMemcpyDeviceToHost, st));
@@ -2022,11 +2031,7 @@ int izh_job_info(const izh_job *j, int64_t info[4]) {
 
 int izh_job_destroy(izh_job *j) {
   if (!j) return IZH_OK;
-  if (!j->finished) {
-    // stop the run where it is: wait for what was enqueued
-    (void)hipStreamSynchronize(j->b->stream);
-    j->r.release();
-  }
+  j->r.release();   // a run that did not finish stops where it is
   if (j->exec) (void)hipGraphExecDestroy(j->exec);
   if (j->graph) (void)hipGraphDestroy(j->graph);
   if (j->done_ev) (void)hipEventDestroy(j->done_ev);

@@ -1,0 +1,96 @@
+"""The library's host side on the CPU, over a HIP runtime that queues work and
+launches nothing (fake_hip.cpp): what is still queued when a failed call
+returns, what is launched and allocated, and what becomes of device memory."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+from conftest import ROOT
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+PREAMBLE = """
+import ctypes as C, sys, threading
+sys.path.insert(0, {pkg!r})
+fake = C.CDLL({fake!r}, mode=C.RTLD_GLOBAL)
+fake.fake_pending.restype = fake.fake_launches.restype = C.c_int64
+fake.fake_held.restype = fake.fake_peak.restype = C.c_size_t
+fake.fake_capacity.argtypes = fake.fake_fail_alloc.argtypes = [C.c_size_t]
+fake.fake_poke.argtypes = [C.c_size_t, C.c_size_t, C.c_int64]
+from impactz import beam as B, hip
+import numpy as np
+hip.init(0)
+BEAM = B.Beam()
+
+def bunch(n, precision=hip.FP64):
+    return hip.BeamBunch.from_beam(B.gaussian_bunch(n, seed=1), BEAM, precision)
+
+def drift():
+    return hip.segment(0.05, 0, 0.0, 10, 1.0, 1.0, 0.1, 0.0)
+
+def refused(call, text=''):
+    try:
+        call()
+    except hip.IZHError as e:
+        assert text in str(e), str(e)
+        return
+    raise AssertionError('accepted')
+
+def answered(steps):
+    # a run's results come as one copy of the 11 words it keeps on the device
+    fake.fake_poke(88, 80, steps)
+"""
+
+
+@pytest.fixture(scope="session")
+def fake_hip(tmp_path_factory):
+    lib = str(tmp_path_factory.mktemp("fake") / "libfake_hip.so")
+    subprocess.check_call(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-pthread",
+                           os.path.join(HERE, "fake_hip.cpp"), "-o", lib])
+
+    def run(script):
+        head = PREAMBLE.format(pkg=os.path.join(ROOT, "impact-z_amd"), fake=lib)
+        r = subprocess.run([sys.executable, "-c", head + script], capture_output=True, text=True,
+                           timeout=120)
+        assert r.returncode == 0, r.stdout + r.stderr
+
+    return run
+
+
+@pytest.mark.parametrize("kernel", ["k_pass", "k_finalize", "k_deposit_tiles", "k_fft_two",
+                                    "k_efield"])
+def test_failed_run_leaves_nothing_queued(fake_hip, kernel):
+    """After a run that fails on the way, the field's stream is its own again:
+    nothing may be queued on the bunch's by then, or the field's buffers could
+    pass to another owner while kernels still use them."""
+    fake_hip(f"""
+b = bunch(600_000)          # gathers E through a box, so every step has its E kernel
+f, d = hip.FieldQuant(32, 32, 32), hip.CompDom(32, 32, 32)
+fake.fake_fail_kernel({kernel.encode()!r})
+refused(lambda: b.run(f, d, 0.0, [drift()] * 4, BEAM.current), 'injected')
+assert fake.fake_launches({kernel.encode()!r}) == 1
+assert fake.fake_pending() == 0, fake.fake_pending()
+f.close()
+b.close()
+""")
+
+
+@pytest.mark.parametrize("kernel", ["k_prologue_keys", "k_pass", "k_fft_two"])
+def test_failed_job_leaves_nothing_queued(fake_hip, kernel):
+    fake_hip(f"""
+b = bunch(5_000)
+f, d = hip.FieldQuant(16, 16, 16), hip.CompDom(16, 16, 16)
+fake.fake_fail_kernel({kernel.encode()!r})
+refused(lambda: hip.Job(b, f, d, 0.0, [drift()], 8, BEAM.current), 'injected')
+assert fake.fake_pending() == 0, fake.fake_pending()
+job = hip.Job(b, f, d, 0.0, [drift()], 8, BEAM.current, False)
+job.advance(3)
+fake.fake_fail_kernel(b'k_deposit_tiles')
+refused(lambda: job.advance(3), 'injected')
+job.close()
+assert fake.fake_pending() == 0, fake.fake_pending()
+f.close()
+b.close()
+""")
