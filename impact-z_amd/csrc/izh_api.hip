@@ -1701,6 +1701,11 @@ int izh_run(izh_bunch *b, izh_field *f, izh_compdom *dom, double *z,
                   sg.e.bitype, why);
     if (!(sg.tau1 >= 0) || (kind == kMap1Linear && sg.e.mapstp < 1))
       return fail(IZH_ERR_ARG, "izh_run: segment %lld: bad step or map steps", (long long)s);
+    // what its map needs too (an RF cavity's field), before anything is queued
+    LinearElement le;
+    if (kind == kMap1Linear && (why = linear_element(&b->c, sg.e, le)) != nullptr)
+      return fail(IZH_ERR_ARG, "izh_run: segment %lld: bitype %d: %s", (long long)s,
+                  sg.e.bitype, why);
     if (needs_wake(sg.e) && !sg.wake)
       return fail(IZH_ERR_ARG, "izh_run: segment %lld: bitype %d with a wake length "
                   "(Param(15) > 0) needs its izh_wake", (long long)s, sg.e.bitype);

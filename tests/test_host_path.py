@@ -94,3 +94,27 @@ assert fake.fake_pending() == 0, fake.fake_pending()
 f.close()
 b.close()
 """)
+
+
+@pytest.mark.parametrize("cavity,why", [
+    ("hip.segment(0.05, 103, [1e6, 324e6, 0, 1, 1], 10, 1.0, 1.0, 0.1, 0.0)", "needs its field"),
+    ("hip.segment(0.05, 105, [1e6, 324e6, 0, 1, 1], 10, 1.0, 1.0, 0.1, 0.0, TABLE)", "Fourier"),
+    ("hip.segment(0.05, 101, [1e6, 324e6, 0, 1, 1], 10, 1.0, 1.0, 0.1, 0.0, SERIES)", "table"),
+    ("hip.segment(0.05, 102, [1e6, 0.0, 0, 1, 1], 10, 1.0, 1.0, 0.1, 0.0, TABLE)", "frequency"),
+])
+def test_run_refuses_a_cavity_before_it_starts(fake_hip, cavity, why):
+    """A cavity in mid-lattice that has no usable field is refused with the
+    bunch as it was, not after the steps before it."""
+    fake_hip(f"""
+TABLE = hip.RFData(np.array([[0.0, 1.0, 0.0, 0.0], [1.0, 1.0, 0.0, 0.0]]), fourier=False)
+SERIES = hip.RFData(np.array([5.0, 0.0, 1.0, 1.0, 0.5, 0.2, 0.1, 0.1, 0.1]), fourier=True)
+b = bunch(2_000)
+f, d = hip.FieldQuant(16, 16, 16), hip.CompDom(16, 16, 16)
+before = list(b.info().refpt)
+fake.fake_forget_launches()
+for current in (BEAM.current, 0.0):
+    refused(lambda: b.run(f, d, 0.0, [drift(), drift(), {cavity}], current), {why!r})
+assert fake.fake_launches(b'') == 0 and list(b.info().refpt) == before
+f.close()
+b.close()
+""")
