@@ -128,6 +128,21 @@ static int join_streams(hipStream_t producer, hipStream_t consumer) {
   return IZH_OK;
 }
 
+// Kernels of a bunch and a field run on their own streams while they share
+// data: the consumer's stream waits for everything queued on the producer's.
+// work() queues kernels on `on` that use what belongs to `of`: they follow the
+// work of `of`, whose later work (and its owner's destroy call) follows them.
+// A call that fails in between waits, so that nothing it queued is left behind
+// that nobody follows.
+template <typename F>
+static int queue_on(hipStream_t on, hipStream_t of, F work) {
+  int rc = join_streams(of, on);
+  if (rc == IZH_OK) rc = work();
+  if (rc == IZH_OK) rc = join_streams(on, of);
+  if (rc != IZH_OK) (void)hipStreamSynchronize(on);
+  return rc;
+}
+
 // Moving rows (phase space + original index) for cap particles.
 // The six rows share one allocation, row k at r[0] + k*cap, so a kernel can
 // address them from one base pointer.
@@ -1163,8 +1178,6 @@ int izh_field_destroy(izh_field *f) {
   return IZH_OK;
 }
 
-// Kernels of a bunch and a field run on their own streams while they share
-// data: the consumer's stream waits for everything queued on the producer's.
 static int check_dom(const izh_field *f, const izh_compdom *dom, const char *who) {
   if (!dom) return fail(IZH_ERR_ARG, "%s: no domain", who);
   if (dom->nx != f->nx || dom->ny != f->ny || dom->nz != f->nz)
@@ -1184,10 +1197,7 @@ int izh_charge(izh_bunch *b, const izh_compdom *dom, izh_field *f) {
   if (b->precision != f->precision)
     return fail(IZH_ERR_ARG, "izh_charge: bunch and field precision differ");
   IZH_CHECK(field_set_domain(f, dom));
-  IZH_CHECK(join_streams(b->stream, f->stream));
-  IZH_CHECK(launch_deposit_granular(b, f));
-  IZH_CHECK(join_streams(f->stream, b->stream));
-  return IZH_OK;
+  return queue_on(f->stream, b->stream, [&] { return launch_deposit_granular(b, f); });
 }
 
 int izh_update3O(izh_field *f, const izh_compdom *dom) {
@@ -1225,11 +1235,10 @@ int izh_kick1(izh_bunch *b, double tau, izh_field *f, const izh_compdom *dom,
     return fail(IZH_ERR_ARG, "izh_kick1: bunch and field precision differ");
   IZH_CHECK(field_set_domain(f, dom));
   IZH_CHECK(launch_efield(f));
-  IZH_CHECK(join_streams(f->stream, b->stream));
   double xycon, tcon;
   sc_constants(b, &xycon, &tcon);
-  IZH_CHECK(launch_gather_kick(b, f, tau, xycon, tcon));
-  IZH_CHECK(join_streams(b->stream, f->stream));
+  IZH_CHECK(queue_on(b->stream, f->stream,
+                     [&] { return launch_gather_kick(b, f, tau, xycon, tcon); }));
   b->frame = kFrameZ;
   return IZH_OK;
 }
@@ -1391,12 +1400,10 @@ static int kick2_impl(izh_bunch *b, double z, double tau, const izh_element *e,
     }
     IZH_CHECK(field_set_domain(f, dom));
     IZH_CHECK(launch_efield(f));
-    IZH_CHECK(join_streams(f->stream, b->stream));
     // Clight^2 * 1e-7 (REAL(4)) is 1/(4 pi eps0); the grid holds charge * rho_scale
     k.tmpscale = b->c.clight * b->c.clight * (double)1.0e-7f / f->rho_scale;
     // -beta0/Clight*tmpscale*eyn: the scaled factor enters through tmpscale
-    IZH_CHECK(launch_kick2(b, f, k, true));
-    IZH_CHECK(join_streams(b->stream, f->stream));
+    IZH_CHECK(queue_on(b->stream, f->stream, [&] { return launch_kick2(b, f, k, true); }));
   } else {
     IZH_CHECK(launch_kick2(b, f, k, false));
   }
@@ -1604,10 +1611,8 @@ int izh_wakefield(izh_bunch *b, izh_field *f, const izh_compdom *dom, const izh_
   WakeParams p;
   IZH_CHECK(wake_params_of(b, f, w, &p));
   IZH_CHECK(field_set_domain(f, dom));
-  IZH_CHECK(join_streams(b->stream, f->stream));
-  IZH_CHECK(launch_wake(b, f, p, nullptr, nullptr, nullptr, 0));
-  IZH_CHECK(join_streams(f->stream, b->stream));
-  return IZH_OK;
+  return queue_on(f->stream, b->stream,
+                  [&] { return launch_wake(b, f, p, nullptr, nullptr, nullptr, 0); });
 }
 
 int izh_kick1wake(izh_bunch *b, double tau, izh_field *f, const izh_compdom *dom,
@@ -1628,11 +1633,10 @@ int izh_kick1wake(izh_bunch *b, double tau, izh_field *f, const izh_compdom *dom
   IZH_CHECK(field_set_domain(f, dom));
   IZH_CHECK(launch_efield(f));
   IZH_CHECK(launch_wake_add(f));
-  IZH_CHECK(join_streams(f->stream, b->stream));
   double xycon, tcon;
   sc_constants(b, &xycon, &tcon);
-  IZH_CHECK(launch_gather_kick(b, f, tau, xycon, tcon));
-  IZH_CHECK(join_streams(b->stream, f->stream));
+  IZH_CHECK(queue_on(b->stream, f->stream,
+                     [&] { return launch_gather_kick(b, f, tau, xycon, tcon); }));
   b->frame = kFrameZ;
   return IZH_OK;
 }

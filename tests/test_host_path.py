@@ -118,3 +118,48 @@ assert fake.fake_launches(b'') == 0 and list(b.info().refpt) == before
 f.close()
 b.close()
 """)
+
+
+@pytest.mark.parametrize("n,kernel", [(100, "k_deposit_direct"), (5_000, "k_deposit_small"),
+                                      (5_000, "k_fx_to_grid"), (5_000, "k_wake_field")])
+def test_failed_call_on_the_field_leaves_the_bunch_free(fake_hip, n, kernel):
+    """Kernels on the field's stream read the bunch's rows: after a call that
+    fails, ending the bunch alone must find them done."""
+    fake_hip(f"""
+b = bunch({n})
+f, d = hip.FieldQuant(16, 16, 16), hip.CompDom(16, 16, 16)
+b.conv1st(0.05, 1.0, 1.0)
+d.set([0, 1, 0, 1, 0, 1], [1 / 15] * 3)
+w = hip.wake(1, 0.01, 0.02, 0.03)
+fake.fake_fail_kernel({kernel.encode()!r})
+
+def calls():
+    b.wakefield(f, d, w)
+    b.charge(d, f)
+refused(calls, 'injected')
+b.close()
+assert fake.fake_pending() == 0, fake.fake_pending()
+f.close()
+""")
+
+
+@pytest.mark.parametrize("kernel", ["k_gather_kick", "k_kick2"])
+def test_failed_kick_leaves_the_field_free(fake_hip, kernel):
+    """And kernels on the bunch's stream read the field's E."""
+    fake_hip(f"""
+b = bunch(5_000)
+f, d = hip.FieldQuant(16, 16, 16), hip.CompDom(16, 16, 16)
+b.conv1st(0.05, 1.0, 1.0)
+d.set([0, 1, 0, 1, 0, 1], [1 / 15] * 3)
+b.charge(d, f)
+f.update3O(d)
+b.cvbkforth1st()
+fake.fake_fail_kernel({kernel.encode()!r})
+if {kernel!r} == 'k_kick2':
+    refused(lambda: b.kick2(0.0, 0.05, hip.element(0, 0.0, 0.1), f, d), 'injected')
+else:
+    refused(lambda: b.kick1(0.05, f, d), 'injected')
+f.close()
+assert fake.fake_pending() == 0, fake.fake_pending()
+b.close()
+""")
