@@ -1584,6 +1584,15 @@ static void deposit_scales(const izh_bunch *b, izh_field *f) {
   f->rho_scale = f->precision == IZH_FP64 ? 1.0 : 1.0 / wsum;
 }
 
+// Whatever reads the accumulator clears it for the next deposit, unless the call
+// failed in between: then this deposit clears it first.
+static void begin_deposit(izh_field *f) {
+  if (f->fx_dirty)
+    hipLaunchKernelGGL(k_fill_u32, dim3(grid_for(2 * f->g)), dim3(kBlock), 0, f->stream,
+                       (uint32_t *)f->rho_fx, 2 * f->g, 0u);
+  f->fx_dirty = 1;
+}
+
 // The fused run's deposit: the t positions (T) of the tile-sorted bunch, by
 // its chunk list, into the (cleared) fixed-point accumulator, and in the same
 // launch the corners of the step's Green function; launch_convolve_fx
@@ -1593,6 +1602,7 @@ int launch_deposit(izh_bunch *b, izh_field *f, const Chunk *chunks, const KeyGri
   if (!chunks || !kgrid || max_chunks < 1)
     return fail(IZH_ERR_ARG, "deposit: no chunk list or key grid");
   deposit_scales(b, f);
+  begin_deposit(f);
   // every contribution is at most |w| * scale: below 2^50 the fused
   // deposit rounds with the short form
   const bool fast = b->wabs_max * f->fixed_scale < 0x1p50;
@@ -1655,6 +1665,7 @@ static bool bins_ready(izh_field *f, int64_t n, bool weights, int ntiles) {
 constexpr int64_t kDirect = 4096;
 int launch_deposit_granular(izh_bunch *b, izh_field *f) {
   deposit_scales(b, f);
+  begin_deposit(f);
   const DepRows d{b->r[0], b->r[2], b->r[4], b->orig, b->w0, b->w_value, b->w_uniform, b->n,
                   f->d_dom, f->nx, f->ny, f->nz, f->fixed_scale};
   if (b->n > 0) {
@@ -1717,6 +1728,7 @@ int launch_deposit_granular(izh_bunch *b, izh_field *f) {
     hipLaunchKernelGGL(k_fx_to_grid<float>, dim3(grid_for(f->g)), dim3(kBlock), 0,
                        f->stream, f->rho_fx, (float *)f->rho, f->g, inv);
   IZH_HIP(hipGetLastError());
+  f->fx_dirty = 0;
   f->have_rho = 1;
   f->have_phi = 0;
   return IZH_OK;
@@ -1725,7 +1737,10 @@ int launch_deposit_granular(izh_bunch *b, izh_field *f) {
 int launch_convolve_fx(izh_field *f) {
   const int rc = f->precision == IZH_FP64 ? convolve_t<double, true>(f)
                                           : convolve_t<float, true>(f);
-  if (rc == IZH_OK) f->have_rho = f->have_phi = 1;
+  if (rc == IZH_OK) {
+    f->fx_dirty = 0;
+    f->have_rho = f->have_phi = 1;
+  }
   return rc;
 }
 

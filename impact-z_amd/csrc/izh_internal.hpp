@@ -207,6 +207,7 @@ struct izh_field {
   int nx = 0, ny = 0, nz = 0;
   int64_t g = 0;                // nx*ny*nz
   unsigned long long *rho_fx = nullptr;  // fixed-point deposit accumulator
+  int fx_dirty = 0;             // a deposit began and nothing has read and cleared it
   void *rho = nullptr;          // T[g]   charge density (T = double or float)
   void *phi = nullptr;          // T[g]   potential
   void *e = nullptr;            // T4[g]  (Ex, Ey, Ez, 0) interleaved

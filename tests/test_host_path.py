@@ -163,3 +163,38 @@ f.close()
 assert fake.fake_pending() == 0, fake.fake_pending()
 b.close()
 """)
+
+
+@pytest.mark.parametrize("kernel", ["k_deposit_small", "k_fx_to_grid"])
+def test_charge_after_a_failed_one_starts_clean(fake_hip, kernel):
+    """The accumulator is cleared by whatever reads it; a deposit that no call
+    read must not add to the next one."""
+    fake_hip(f"""
+b = bunch(5_000)
+f, d = hip.FieldQuant(16, 16, 16), hip.CompDom(16, 16, 16)
+b.conv1st(0.05, 1.0, 1.0)
+d.set([0, 1, 0, 1, 0, 1], [1 / 15] * 3)
+b.charge(d, f)
+assert fake.fake_launches(b'k_fill_u32') == 0
+fake.fake_fail_kernel({kernel.encode()!r})
+refused(lambda: b.charge(d, f), 'injected')
+b.charge(d, f)
+b.charge(d, f)
+assert fake.fake_launches(b'k_fill_u32') == 1
+""")
+
+
+@pytest.mark.parametrize("kernel", ["k_deposit_tiles", "k_fft_two"])
+def test_deposit_after_a_failed_run_starts_clean(fake_hip, kernel):
+    fake_hip(f"""
+b = bunch(5_000)
+f, d = hip.FieldQuant(16, 16, 16), hip.CompDom(16, 16, 16)
+fake.fake_fail_kernel({kernel.encode()!r})
+refused(lambda: b.run(f, d, 0.0, [drift()] * 3, BEAM.current), 'injected')
+assert fake.fake_launches(b'k_fill_u32') == 0
+answered(3)
+b.run(f, d, 0.0, [drift()] * 3, BEAM.current)
+assert fake.fake_launches(b'k_fill_u32') == 1
+b.run(f, d, 0.0, [drift()] * 3, BEAM.current)
+assert fake.fake_launches(b'k_fill_u32') == 1
+""")
