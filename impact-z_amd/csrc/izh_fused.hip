@@ -1408,6 +1408,8 @@ int bunch_alloc_fused(izh_bunch *b, int ntiles, int64_t nseg) {
   const int64_t nch = b->cap / chunk_len(b->cap) + ntiles + 1;
   if (ntiles > b->ntiles_cap || nch > b->nchunks_cap) {
     IZH_HIP(hipStreamSynchronize(b->stream));
+    // the cursors and lists the last run left for the next one go
+    b->keys_valid = 0;
     for (int k = 0; k < 2; k++) dev_release(b->hist[k]);
     dev_release(b->cursor);
     dev_release(b->chunks);

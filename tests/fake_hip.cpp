@@ -80,7 +80,7 @@ extern "C" {
 void fake_capacity(size_t bytes) { st().capacity = bytes; }
 void fake_free_delay(int ms) { st().free_ms = ms; }
 void fake_fail_kernel(const char *name) { st().fail_kernel = name; }
-// the next allocation of this many bytes fails
+// allocations of this many bytes fail (0: none does)
 void fake_fail_alloc(size_t bytes) { st().fail_bytes = bytes; }
 void fake_poke(size_t bytes, size_t at, int64_t value) {
   st().poke_bytes = bytes;
@@ -155,11 +155,8 @@ int hipDeviceSynchronize() {
 int hipMalloc(void **p, size_t bytes) {
   std::lock_guard<std::mutex> lock(st().mu);
   *p = nullptr;
-  if (st().fail_bytes == bytes && bytes > 0) {
-    st().fail_bytes = 0;
+  if ((st().fail_bytes == bytes && bytes > 0) || st().held + bytes > st().capacity)
     return st().last_error = kOutOfMemory;
-  }
-  if (st().held + bytes > st().capacity) return st().last_error = kOutOfMemory;
   *p = calloc(bytes ? bytes : 1, 1);
   st().blocks[*p] = bytes;
   st().held += bytes;

@@ -198,3 +198,24 @@ assert fake.fake_launches(b'k_fill_u32') == 1
 b.run(f, d, 0.0, [drift()] * 3, BEAM.current)
 assert fake.fake_launches(b'k_fill_u32') == 1
 """)
+
+
+def test_run_after_its_sort_state_was_lost_starts_afresh(fake_hip):
+    """A run on a larger grid that finds no memory for its tile lists has
+    already given up the smaller ones: the next run on the first field may not
+    start from them."""
+    fake_hip("""
+b = bunch(5_000)
+f, d = hip.FieldQuant(16, 16, 16), hip.CompDom(16, 16, 16)
+g, e = hip.FieldQuant(64, 64, 64), hip.CompDom(64, 64, 64)
+answered(2)
+b.run(f, d, 0.0, [drift()] * 2, BEAM.current)
+b.run(f, d, 0.0, [drift()] * 2, BEAM.current)
+assert fake.fake_launches(b'k_prologue_keys') == 1      # the second started warm
+for lost in (1, 2):
+    fake.fake_fail_alloc(4 * 512)                       # the cursors of 512 tiles
+    refused(lambda: b.run(g, e, 0.0, [drift()] * 2, BEAM.current))
+    fake.fake_fail_alloc(0)
+    b.run(f, d, 0.0, [drift()] * 2, BEAM.current)
+    assert fake.fake_launches(b'k_prologue_keys') == 1 + lost
+""")
