@@ -13,6 +13,7 @@
 // - A block is released by the owner's destroy or grow call, after it waited
 //   for its stream, so the next owner may use it on any stream.
 // - One lock guards the lists; hipMalloc and hipFree run outside of it.
+#include <condition_variable>
 #include <deque>
 #include <mutex>
 #include <unordered_map>
@@ -37,6 +38,10 @@ struct Cache {
   std::unordered_map<int, std::deque<Block>> kept;  // by device, oldest first
   std::unordered_map<int, size_t> kept_bytes;
   std::unordered_map<int, int> handles;
+  // blocks off the lists but not freed yet, and how often some have been
+  std::condition_variable freed;
+  int freeing = 0;
+  uint64_t times_freed = 0;
 };
 
 // Never destroyed: at process exit the runtime may be gone before it.
@@ -51,57 +56,69 @@ std::vector<Block> take_all(Cache &c, int device) {
   std::vector<Block> out(q.begin(), q.end());
   q.clear();
   c.kept_bytes[device] = 0;
+  c.freeing += !out.empty();
   return out;
 }
 
-void give_back(const std::vector<Block> &blocks) {
+// Frees what was taken off the lists (counted in freeing when it was).
+void give_back(Cache &c, const std::vector<Block> &blocks) {
+  if (blocks.empty()) return;
   for (const Block &b : blocks) (void)hipFree(b.p);
+  std::lock_guard<std::mutex> lock(c.mu);
+  c.freeing--;
+  c.times_freed++;
+  c.freed.notify_all();
+}
+
+// A kept block for the request, if there is one (the lock is held).
+void *take_kept(Cache &c, int device, size_t bytes) {
+  std::deque<Block> &q = c.kept[device];
+  auto best = q.end();
+  for (auto it = q.begin(); it != q.end(); ++it)
+    if (it->bytes >= bytes && it->bytes - it->bytes / 16 <= bytes &&
+        (best == q.end() || it->bytes < best->bytes))
+      best = it;
+  if (best == q.end()) return nullptr;
+  const Block b = *best;
+  q.erase(best);
+  c.kept_bytes[device] -= b.bytes;
+  c.used[b.p] = b;
+  return b.p;
 }
 
 }  // namespace
 
+// There is no memory only when the device has none with nothing kept and no
+// other thread in the middle of giving some back: until then it tries again.
 hipError_t dev_malloc(void **p, size_t bytes) {
   *p = nullptr;
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return e;
   Cache &c = cache();
-  {
-    std::lock_guard<std::mutex> lock(c.mu);
-    std::deque<Block> &q = c.kept[dev];
-    auto best = q.end();
-    for (auto it = q.begin(); it != q.end(); ++it)
-      if (it->bytes >= bytes && it->bytes - it->bytes / 16 <= bytes &&
-          (best == q.end() || it->bytes < best->bytes))
-        best = it;
-    if (best != q.end()) {
-      const Block b = *best;
-      q.erase(best);
-      c.kept_bytes[dev] -= b.bytes;
-      c.used[b.p] = b;
-      *p = b.p;
-      return hipSuccess;
-    }
-  }
-  e = hipMalloc(p, bytes);
-  if (e != hipSuccess) {
-    (void)hipGetLastError();
-    std::vector<Block> all;
+  for (;;) {
+    uint64_t times;
     {
       std::lock_guard<std::mutex> lock(c.mu);
-      all = take_all(c, dev);
+      if ((*p = take_kept(c, dev, bytes)) != nullptr) return hipSuccess;
+      times = c.times_freed;
     }
-    if (all.empty()) return e;
-    give_back(all);
     e = hipMalloc(p, bytes);
-    if (e != hipSuccess) {
-      (void)hipGetLastError();
-      return e;
+    std::unique_lock<std::mutex> lock(c.mu);
+    if (e == hipSuccess) {
+      c.used[*p] = Block{*p, bytes, dev};
+      return hipSuccess;
     }
+    (void)hipGetLastError();
+    *p = nullptr;
+    const std::vector<Block> all = take_all(c, dev);
+    if (all.empty()) {
+      c.freed.wait(lock, [&] { return c.freeing == 0 || c.times_freed != times; });
+      if (c.times_freed == times) return e;
+    }
+    lock.unlock();
+    give_back(c, all);
   }
-  std::lock_guard<std::mutex> lock(c.mu);
-  c.used[*p] = Block{*p, bytes, dev};
-  return hipSuccess;
 }
 
 void dev_release(void *p) {
@@ -127,8 +144,9 @@ void dev_release(void *p) {
       q.push_back(b);
       held += b.bytes;
     }
+    c.freeing += !out.empty();
   }
-  give_back(out);
+  give_back(c, out);
 }
 
 void dev_handles(int device, int change) {
@@ -140,7 +158,7 @@ void dev_handles(int device, int change) {
     h += change;
     if (h <= 0) out = take_all(c, device);
   }
-  give_back(out);
+  give_back(c, out);
 }
 
 }  // namespace izh

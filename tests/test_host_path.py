@@ -219,3 +219,42 @@ for lost in (1, 2):
     b.run(f, d, 0.0, [drift()] * 2, BEAM.current)
     assert fake.fake_launches(b'k_prologue_keys') == 1 + lost
 """)
+
+
+def test_memory_another_thread_gives_back_is_waited_for(fake_hip):
+    """Kept blocks fill the device.  The first thread that finds no memory takes
+    them all and frees them; the others wait for that instead of failing."""
+    fake_hip("""
+b = bunch(1_000)
+f = hip.FieldQuant(64, 64, 64)
+before = fake.fake_held()
+f.close()
+assert fake.fake_held() == before                       # all of it kept
+# room for the two smaller fields, but not beside what is kept
+fake.fake_capacity(before + (1 << 20))
+fake.fake_free_delay(20)
+fields, errors, gate = [], [], threading.Barrier(2)
+
+def make(grid):
+    gate.wait()
+    try:
+        fields.append(hip.FieldQuant(*grid))
+    except hip.IZHError as e:
+        errors.append(str(e))
+
+for _ in range(3):
+    threads = [threading.Thread(target=make, args=(g,)) for g in ((32, 32, 64), (32, 64, 32))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
+    while fields:
+        fields.pop().close()
+    # every block of the 64^3 grid again
+    fake.fake_free_delay(0)
+    f = hip.FieldQuant(64, 64, 64)
+    f.close()
+    fake.fake_free_delay(20)
+b.close()
+""")
