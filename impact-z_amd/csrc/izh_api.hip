@@ -560,7 +560,7 @@ int izh_rfdata_fourier(const double *coef, int n, izh_rfdata **out) {
 int izh_rfdata_destroy(izh_rfdata *d) {
   if (d && d->d_table) {
     (void)hipDeviceSynchronize();
-    (void)hipFree(d->d_table);
+    dev_free(d->d_table);
   }
   delete d;
   return IZH_OK;

@@ -32,11 +32,13 @@ int fail(int code, const char *fmt, ...);
   } while (0)
 
 // ------------------------------------------------------ device memory
-// Device memory of the bunches and fields.  dev_release keeps a block for the
-// next dev_malloc on its device instead of returning it (izh_memory.hip says
-// how much and for how long); the caller has waited for the work that uses it.
+// The library's device memory.  dev_release keeps a block for the next
+// dev_malloc on its device instead of returning it (izh_memory.hip says how
+// much and for how long); the caller has waited for the work that uses it.
+// dev_free returns it at once, as hipFree does, which waits by itself.
 hipError_t dev_malloc(void **p, size_t bytes);
 void dev_release(void *p);
+void dev_free(void *p);
 // A bunch or field comes to life (+1) or ends (-1) on a device; with the last
 // one every kept block of the device goes back.
 void dev_handles(int device, int change);

@@ -149,6 +149,21 @@ void dev_release(void *p) {
   give_back(c, out);
 }
 
+void dev_free(void *p) {
+  if (!p) return;
+  Cache &c = cache();
+  std::vector<Block> out;
+  {
+    std::lock_guard<std::mutex> lock(c.mu);
+    const auto it = c.used.find(p);
+    if (it == c.used.end()) return;
+    out.push_back(it->second);
+    c.used.erase(it);
+    c.freeing++;
+  }
+  give_back(c, out);
+}
+
 void dev_handles(int device, int change) {
   Cache &c = cache();
   std::vector<Block> out;

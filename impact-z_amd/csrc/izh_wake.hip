@@ -407,8 +407,10 @@ int wake_table_device(const izh_rfdata *d, const double **out) {
       h[3 * n + i] = d->ezpp[i];
     }
     double *p = nullptr;
-    IZH_HIP(hipMalloc((void **)&p, h.size() * sizeof(double)));
-    IZH_HIP(hipMemcpy(p, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice));
+    IZH_HIP(dev_malloc((void **)&p, h.size() * sizeof(double)));
+    const hipError_t e = hipMemcpy(p, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice);
+    if (e != hipSuccess) dev_free(p);
+    IZH_HIP(e);
     d->d_table = p;
   }
   *out = d->d_table;

@@ -258,3 +258,28 @@ for _ in range(3):
     fake.fake_free_delay(20)
 b.close()
 """)
+
+
+@pytest.mark.parametrize("call", ["b.wakefield(f, d, hip.wake(2, table=TABLE, scale=1.0))",
+                                  "hip.probe_copy(3 << 20)"])
+def test_kept_memory_is_no_obstacle_to_other_allocations(fake_hip, call):
+    """A wake's table and the copy probe find room where kept blocks fill the
+    device, and give their own memory back."""
+    fake_hip(f"""
+z = np.linspace(0.0, 1.0, 1000)
+TABLE = hip.RFData(np.stack([z, z, z, z], axis=1), fourier=False)
+b = bunch(1_000)
+f, d = hip.FieldQuant(16, 16, 16), hip.CompDom(16, 16, 16)
+b.conv1st(0.05, 1.0, 1.0)
+d.set([0, 1, 0, 1, 0, 1], [1 / 15] * 3)
+b.wakefield(f, d, hip.wake(1, 0.01, 0.02, 0.03))        # the field's own wake lines
+held = fake.fake_held()
+hip.FieldQuant(64, 64, 64).close()
+assert fake.fake_held() > held                          # kept
+fake.fake_capacity(fake.fake_held())
+{call}
+f.close()
+b.close()
+TABLE.close()
+assert fake.fake_held() == 0, fake.fake_held()
+""")
