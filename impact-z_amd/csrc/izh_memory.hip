@@ -6,8 +6,8 @@
 // 1.8 of 11.9 ms of a 64-step run on it.  So a released block is kept for the
 // next allocation of about its size.
 // - What is kept is bounded (kKeepBytes a device; the oldest blocks leave
-//   first) and goes back when an allocation fails and when the last bunch or
-//   field of the device ends.
+//   first) and goes back when an allocation fails, when the last bunch or
+//   field of the device ends and when the caller asks (izh_memory_trim).
 // - A block serves requests down to 15/16 of its size, so a handle holds at
 //   most that much more than it asked for.
 // - A block is released by the owner's destroy or grow call, after it waited
@@ -35,6 +35,7 @@ struct Block {
 struct Cache {
   std::mutex mu;
   std::unordered_map<void *, Block> used;
+  std::unordered_map<int, size_t> used_bytes;
   std::unordered_map<int, std::deque<Block>> kept;  // by device, oldest first
   std::unordered_map<int, size_t> kept_bytes;
   std::unordered_map<int, int> handles;
@@ -83,6 +84,7 @@ void *take_kept(Cache &c, int device, size_t bytes) {
   q.erase(best);
   c.kept_bytes[device] -= b.bytes;
   c.used[b.p] = b;
+  c.used_bytes[device] += b.bytes;
   return b.p;
 }
 
@@ -107,6 +109,7 @@ hipError_t dev_malloc(void **p, size_t bytes) {
     std::unique_lock<std::mutex> lock(c.mu);
     if (e == hipSuccess) {
       c.used[*p] = Block{*p, bytes, dev};
+      c.used_bytes[dev] += bytes;
       return hipSuccess;
     }
     (void)hipGetLastError();
@@ -131,6 +134,7 @@ void dev_release(void *p) {
     if (it == c.used.end()) return;   // not a block of dev_malloc's
     const Block b = it->second;
     c.used.erase(it);
+    c.used_bytes[b.device] -= b.bytes;
     if (b.bytes > kKeepBytes || c.handles[b.device] <= 0) {
       out.push_back(b);
     } else {
@@ -158,6 +162,7 @@ void dev_free(void *p) {
     const auto it = c.used.find(p);
     if (it == c.used.end()) return;
     out.push_back(it->second);
+    c.used_bytes[it->second.device] -= it->second.bytes;
     c.used.erase(it);
     c.freeing++;
   }
@@ -177,3 +182,32 @@ void dev_handles(int device, int change) {
 }
 
 }  // namespace izh
+
+using namespace izh;
+
+extern "C" {
+
+int izh_memory_info(int64_t *in_use, int64_t *kept) {
+  int dev = 0;
+  IZH_HIP(hipGetDevice(&dev));
+  Cache &c = cache();
+  std::lock_guard<std::mutex> lock(c.mu);
+  if (in_use) *in_use = (int64_t)c.used_bytes[dev];
+  if (kept) *kept = (int64_t)c.kept_bytes[dev];
+  return IZH_OK;
+}
+
+int izh_memory_trim(void) {
+  int dev = 0;
+  IZH_HIP(hipGetDevice(&dev));
+  Cache &c = cache();
+  std::vector<Block> out;
+  {
+    std::lock_guard<std::mutex> lock(c.mu);
+    out = take_all(c, dev);
+  }
+  give_back(c, out);
+  return IZH_OK;
+}
+
+}  // extern "C"

@@ -494,6 +494,15 @@ module impactz_hip
       integer(c_int64_t) :: stats(4)
       integer(c_int) :: rc
     end function
+    function izh_memory_info(in_use, kept) bind(C, name="izh_memory_info") result(rc)
+      import :: c_int, c_int64_t
+      integer(c_int64_t) :: in_use, kept
+      integer(c_int) :: rc
+    end function
+    function izh_memory_trim() bind(C, name="izh_memory_trim") result(rc)
+      import :: c_int
+      integer(c_int) :: rc
+    end function
     function izh_probe_copy(nbytes, ms) bind(C, name="izh_probe_copy") result(rc)
       import :: c_int, c_int64_t, c_double
       integer(c_int64_t), value :: nbytes

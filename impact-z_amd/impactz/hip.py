@@ -39,7 +39,8 @@ SYMBOLS = (
     "izh_wake_download", "izh_kick2wake", "izh_chgupdate", "izh_bunch_set_tuning",
     "izh_bunch_get_tuning", "izh_job_create", "izh_job_advance",
     "izh_job_query", "izh_job_finish", "izh_job_info", "izh_job_destroy",
-    "izh_bunch_create_from", "izh_diagnostic1_rows",
+    "izh_bunch_create_from", "izh_diagnostic1_rows", "izh_memory_info",
+    "izh_memory_trim",
 )
 
 # timer slots (IZH_T_*), named after the reference's Timer accumulators
@@ -231,6 +232,7 @@ def lib() -> C.CDLL:
                           C.c_int64, C.c_double, _dp]
     L.izh_run_stats.argtypes = [vp, _i64p]
     L.izh_probe_copy.argtypes = [C.c_int64, _dp]
+    L.izh_memory_info.argtypes = [_i64p, _i64p]
     L.izh_timer_enable.argtypes = [C.c_int]
     L.izh_timer_read.argtypes = [_dp, _i64p, C.c_int]
     _lib = L
@@ -268,6 +270,19 @@ def probe_copy(nbytes: int) -> float:
     ms = C.c_double()
     check(lib().izh_probe_copy(nbytes, C.byref(ms)))
     return ms.value
+
+
+def memory_info() -> tuple[int, int]:
+    """(bytes the library's handles hold, bytes it keeps for the next ones) on
+    the current device."""
+    used, kept = C.c_int64(), C.c_int64()
+    check(lib().izh_memory_info(C.byref(used), C.byref(kept)))
+    return used.value, kept.value
+
+
+def memory_trim() -> None:
+    """Give the kept device memory back (to torch, say, in the same process)."""
+    check(lib().izh_memory_trim())
 
 
 def physconst(freq: float) -> Const:
@@ -314,6 +329,9 @@ class DeviceDoubles:
         self.n = int(n)
         self.ptr = C.c_void_p()
         if DeviceDoubles._rt.hipMalloc(C.byref(self.ptr), max(self.n, 1) * 8) != 0:
+            memory_trim()   # the library may hold what is missing
+            if DeviceDoubles._rt.hipMalloc(C.byref(self.ptr), max(self.n, 1) * 8) == 0:
+                return
             raise IZHError(f"hipMalloc of {self.n} doubles failed")
 
     def upload(self, a: np.ndarray) -> None:

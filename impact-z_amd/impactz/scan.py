@@ -77,11 +77,13 @@ def c5_requests(seed: int = 11, rate: float = 20.0, duration: float = 300.0,
     return out
 
 
-def footprint(n: int, grid, precision: int) -> int:
-    """HBM bytes a job holds: the bunch (both ping-pong copies of the rows,
-    index and key words, t positions, the immutable rows, reduction and sort
-    scratch) and the field (fixed-point charge, grids, half spectra, Green
-    function), as the library allocates them."""
+def footprint(n: int, grid, precision: int, steps: int = 0) -> int:
+    """HBM bytes a job of so many steps holds: the bunch (both ping-pong copies
+    of the rows, index and key words, t positions, the immutable rows,
+    reduction and sort scratch, a record per step) and the field (fixed-point
+    charge, grids, half spectra, Green function, tables), as the library asks
+    for them.  A buffer kept from an earlier handle may be 1/15 larger
+    (hip.memory_info tells)."""
     nx, ny, nz = grid
     pe = 8 if precision == hip.FP64 else 4
     g = nx * ny * nz
@@ -92,8 +94,10 @@ def footprint(n: int, grid, precision: int) -> int:
     bunch = n * (2 * 48 + 4 * 4 + 3 * pe + 3 * 8) + 2048 * 52 * 8 \
         + 2 * (max(n // 16384, 512) + tiles + 1) * 12 + 3 * tiles * 4
     field = g * (8 + 2 * pe + 4 * pe) + ldx * ny * nz * 2 * pe + ldx * 2 * ny * nz * 2 * pe \
-        + (kx + ldx) * (ny + 1) * (nz + 1) * pe + (nx + 2) * (ny + 2) * (nz + 2) * 8
-    return int(bunch + field)
+        + (kx + ldx) * (ny + 1) * (nz + 1) * pe + (nx + 2) * (ny + 2) * (nz + 2) * 8 \
+        + (nx + ny + nz) * 2 * pe
+    # the lanes' sink, the Green function's table, the scalars: below 32 KiB
+    return int(bunch + field + steps * 45 * 8 + (32 << 10))
 
 
 class Pool:
@@ -197,7 +201,9 @@ def serve(reqs: list[Request], pool: Pool, budget_bytes: int, tuner=None,
     footprint fits the budget (and, with max_live, fewer than max_live jobs
     run), then starts as a job; every idle job gets its next block of steps
     enqueued in turn, so jobs that arrive while others run share the GPU
-    with them; finished jobs free their memory at once.  The queue is
+    with them.  A finished job's buffers are kept for the next one
+    (izh_memory_info) as long as the budget holds them beside the jobs that
+    run, and go back before they would keep a request waiting.  The queue is
     first come first served (policy "fifo") or shortest job first ("sjf":
     the waiting request with the least estimated GPU time, `est_seconds`,
     less `aging` times the seconds it has waited, so long requests are not
@@ -219,6 +225,7 @@ def serve(reqs: list[Request], pool: Pool, budget_bytes: int, tuner=None,
     lat, done_steps, records = {}, 0, {}
     peak_live, peak_used = 0, 0
     nxt = 0
+    base = hip.memory_info()[0]
     hip_sync()
     t0 = time.perf_counter()
     while nxt < len(arrivals) or queue or live:
@@ -235,8 +242,14 @@ def serve(reqs: list[Request], pool: Pool, budget_bytes: int, tuner=None,
                                queue[q]))
             ri = queue[qi]
             r = reqs[ri]
-            need = footprint(r.n, r.grid, r.precision)
-            if used + need > budget_bytes and live:
+            need = footprint(r.n, r.grid, r.precision, r.steps)
+            # what the jobs hold in fact: a kept buffer may be 1/15 larger than
+            # what its owner asked for
+            held, kept = hip.memory_info()
+            if held - base + kept + need > budget_bytes and kept:
+                hip.memory_trim()
+                kept = 0
+            if max(used, held - base) + need > budget_bytes and live:
                 break
             queue.pop(qi)
             live.append((ri, Live(r, pool, tuner(r) if tuner else 0, use_graph)))
@@ -256,7 +269,8 @@ def serve(reqs: list[Request], pool: Pool, budget_bytes: int, tuner=None,
                 done_steps += reqs[ri].n * reqs[ri].steps
                 if keep_records:
                     records[ri] = rec
-                used -= footprint(reqs[ri].n, reqs[ri].grid, reqs[ri].precision)
+                used -= footprint(reqs[ri].n, reqs[ri].grid, reqs[ri].precision,
+                                  reqs[ri].steps)
                 lv.close()
                 live.remove((ri, lv))
                 progressed = True

@@ -447,6 +447,16 @@ int izh_run_stats(const izh_bunch *b, int64_t stats[4]);
  * hardware byte counters.  Returns the kernel time in *ms (HIP events). */
 int izh_probe_copy(int64_t nbytes, double *ms);
 
+/* Device memory (no reference counterpart).  The buffers of a bunch or field
+ * that ends are kept for the next one, up to 8 GiB a device, and go back with
+ * the device's last bunch or field or when an allocation of the library finds
+ * no memory.  A kept buffer serves requests down to 15/16 of its size.
+ * izh_memory_info: bytes the library's handles hold and bytes kept on the
+ * current device (either may be null).  izh_memory_trim gives the kept ones
+ * back now, for other users of the device's memory; it waits for the device. */
+int izh_memory_info(int64_t *in_use, int64_t *kept);
+int izh_memory_trim(void);
+
 /* Per-phase kernel timers, the device counterpart of the reference's Timer
  * accumulators (src/Func/Timer.f90:10-146; t_map1, t_rhofas, t_greenf,
  * t_fft2dhpf, t_field, t_force/t_ntrslo, t_diag).  When enabled, each timed

@@ -283,3 +283,65 @@ b.close()
 TABLE.close()
 assert fake.fake_held() == 0, fake.fake_held()
 """)
+
+
+def test_memory_info_and_trim(fake_hip):
+    fake_hip("""
+assert hip.memory_info() == (0, 0)
+b = bunch(1_000)
+used, kept = hip.memory_info()
+assert used == fake.fake_held() and kept == 0
+hip.FieldQuant(32, 32, 32).close()
+after, kept = hip.memory_info()
+assert after == used and kept > 0 and used + kept == fake.fake_held()
+hip.memory_trim()
+assert hip.memory_info() == (used, 0) and fake.fake_held() == used
+# another allocation of the package finds what the library keeps
+hip.DeviceDoubles._rt = fake
+fake.hipMalloc.argtypes = [C.POINTER(C.c_void_p), C.c_size_t]
+fake.hipFree.argtypes = [C.c_void_p]
+hip.FieldQuant(32, 32, 32).close()
+fake.fake_capacity(fake.fake_held() + 1000)
+hip.DeviceDoubles(1000).close()
+b.close()
+assert hip.memory_info() == (0, 0)
+""")
+
+
+@pytest.mark.parametrize("n,grid,form", [(1_000_000, (64, 64, 64), "MIXED"),
+                                         (20_001, (16, 32, 64), "FP64"),
+                                         (300_007, (128, 64, 32), "FP64"),
+                                         (5_000, (32, 32, 32), "MIXED"),
+                                         (2_500_000, (32, 32, 32), "FP64")])
+def test_footprint_is_what_a_job_holds(fake_hip, n, grid, form):
+    """The admission footprint bounds a job's device memory."""
+    fake_hip(f"""
+from impactz import scan
+pool = scan.Pool({n})
+r = scan.Request({n}, {grid}, 40, 10.0, hip.{form})
+base = hip.memory_info()[0]
+lv = scan.Live(r, pool, use_graph=False)
+held = hip.memory_info()[0] - base
+need = scan.footprint(r.n, r.grid, r.precision, r.steps)
+assert held <= need <= 1.1 * held + (1 << 20), (held, need)
+lv.close()
+pool.close()
+""")
+
+
+def test_serve_keeps_to_its_budget(fake_hip):
+    """Jobs and the buffers kept of finished ones stay within the budget."""
+    fake_hip("""
+from impactz import scan
+pool = scan.Pool(60_000)
+reqs = [scan.Request(n, g, 6, 10.0, hip.FP64)
+        for n, g in ((10_000, (32, 32, 32)), (60_000, (16, 16, 32)), (30_000, (16, 32, 32)),
+                     (50_000, (32, 32, 32)), (20_000, (32, 16, 16)), (37_000, (32, 32, 32)))]
+base = fake.fake_held()
+budget = int(1.5 * max(scan.footprint(r.n, r.grid, r.precision) for r in reqs))
+answered(6)
+out = scan.serve(reqs, pool, budget, use_graph=False, policy="fifo")
+assert out["requests"] == 6 and out["peak_bytes"] <= budget
+assert fake.fake_peak() - base <= budget, (fake.fake_peak() - base, budget)
+pool.close()
+""")
