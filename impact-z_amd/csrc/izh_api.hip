@@ -1504,6 +1504,7 @@ int izh_field_download(izh_field *f, int which, double *host) {
   if (!f || !host) return fail(IZH_ERR_ARG, "izh_field_download: bad argument");
   if (which < IZH_RHO || which > IZH_EZ)
     return fail(IZH_ERR_ARG, "izh_field_download: unknown buffer %d", which);
+  if (which >= IZH_EX) IZH_CHECK(field_fresh_e(f));
   IZH_HIP(hipStreamSynchronize(f->stream));
   // the grid holds physical values times rho_scale (1 in FP64); rho, phi and
   // E are linear in the charge, so one factor restores physical units

@@ -1562,6 +1562,7 @@ int field_alloc(izh_field *f) {
 }
 
 int field_set_domain(izh_field *f, const izh_compdom *dom) {
+  IZH_CHECK(field_fresh_e(f));
   // the pinned staging buffer may still feed an earlier copy
   IZH_HIP(hipStreamSynchronize(f->stream));
   DevDom d{};
@@ -1774,6 +1775,7 @@ int launch_efield(izh_field *f) {
                        f->stream, (const float *)f->phi, (E4<float> *)f->e, f->nx,
                        f->ny, f->nz, f->d_dom);
   IZH_HIP(hipGetLastError());
+  f->e_stale = 0;
   return IZH_OK;
 }
 

@@ -1749,6 +1749,7 @@ struct Runner {
         IZH_CHECK(launch_wake_add(f));
       }
     }
+    f->e_stale = !makes_e;
     // second half of the step: host bookkeeping now, applied by the next pass
     IZH_CHECK(segment_push(b, *seg, pb_prev, kb_prev, z));
     refpt_after[2 * step] = b->refpt[4];

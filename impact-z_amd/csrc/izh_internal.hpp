@@ -232,6 +232,7 @@ struct izh_field {
   int bin_rows = 0, bin_tiles = 0;
   double rho_scale = 1.0;       // grid value = physical charge * rho_scale
   int have_rho = 0, have_phi = 0;
+  int e_stale = 0;              // phi is newer than e (a step that kicked from phi)
   double fixed_scale = 0;       // 2^e used by the fixed-point deposit
   double *d_wake = nullptr;     // exwake, eywake, ezwake, dEx, dEy, dEz (nz each), bins
   int have_wake = 0;
@@ -524,6 +525,9 @@ int launch_solve(izh_field *f);
 // rho and phi from launch_deposit's accumulator and Green function corners
 int launch_convolve_fx(izh_field *f);
 int launch_efield(izh_field *f);
+// E of phi where only phi was left, before the domain they share changes and
+// before E is read
+inline int field_fresh_e(izh_field *f) { return f->e_stale ? launch_efield(f) : IZH_OK; }
 int launch_gather_kick(izh_bunch *b, izh_field *f, double tau, double xycon,
                        double tcon);
 int launch_probe_copy(int64_t nbytes, double *ms);

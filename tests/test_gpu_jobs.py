@@ -124,3 +124,38 @@ def test_job_refuses_rf_and_wakes(gpu):
             hip.Job(sim.bunch, sim.field, sim.dom, 0.0, segs, 8, 0.0)
     finally:
         sim.close()
+
+
+@pytest.mark.parametrize("form", ["fp64", "mixed"])
+@pytest.mark.parametrize("passes,use_graph", [(5, False), (17, True)])
+def test_field_of_a_job_under_way(gpu, passes, use_graph, form):
+    """The field's E is that of its potential whenever it is read: a job whose
+    passes kick from the potential leaves no E grid of its own, the same steps
+    through izh_run end with one.  FP64: the fused run's 1e-10; mixed: FP32
+    potentials of the same charge, whose transforms round by 1e-5 at most."""
+    prec = gpu.MIXED if form == "mixed" else gpu.FP64
+    from impactz.beam import fodo
+    sim = _setup(gpu, 30_000, (16, 16, 32), 10.0, 5, prec, period=1)
+    sim.lattice = fodo(2, gradient=10.0)
+    sim.run_fused(passes + 1)
+    want = [sim.field.download(k) for k in (gpu.PHI, gpu.EX, gpu.EY, gpu.EZ)]
+    sim.close()
+    sim, job = _job(gpu, 30_000, (16, 16, 32), 10.0, 5, 64, use_graph, prec, period=1)
+    try:
+        print(f"field of a job: {passes} passes, graph {use_graph}, {form}", flush=True)
+        job.advance(passes)
+        assert job.info()["passes"] == passes + 1
+        for k, w in zip((gpu.PHI, gpu.EX, gpu.EY, gpu.EZ), want):
+            got = sim.field.download(k)
+            err = np.max(np.abs(got - w)) / np.max(np.abs(w))
+            assert err < (TOL if form == "fp64" else 1e-5), (k, err)
+        # reading it disturbs nothing: the job goes on to the same end
+        while job.advance(1 << 20) > 0:
+            pass
+        _, rec = job.finish()
+        rows = [sim.diag(r) for r in rec]
+    finally:
+        job.close()
+        sim.close()
+    ref, _, _ = _solo(gpu, 30_000, (16, 16, 32), 10.0, 5, 64, prec, period=1)
+    assert max(full_row_err(a, b) for a, b in zip(rows, ref)) < TOL

@@ -345,3 +345,22 @@ assert out["requests"] == 6 and out["peak_bytes"] <= budget
 assert fake.fake_peak() - base <= budget, (fake.fake_peak() - base, budget)
 pool.close()
 """)
+
+
+def test_new_domain_finds_the_field_of_the_last_run(fake_hip):
+    """A run that stops on the way may leave a potential without its E, which
+    needs the domain both belong to: it is formed before another one is set."""
+    fake_hip("""
+b = bunch(5_000)            # kicks from the potential
+f, d = hip.FieldQuant(16, 16, 16), hip.CompDom(16, 16, 16)
+job = hip.Job(b, f, d, 0.0, [drift()], 8, BEAM.current, False)
+job.advance(3)
+job.close()
+assert fake.fake_launches(b'k_efield') == 0
+d.set([0, 1, 0, 1, 0, 1], [1 / 15] * 3)
+f.upload_rho(np.ones((16, 16, 16)))
+f.update3O(d)
+assert fake.fake_launches(b'k_efield') == 1
+f.download(hip.EX)
+assert fake.fake_launches(b'k_efield') == 1
+""")
