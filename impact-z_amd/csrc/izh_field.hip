@@ -89,14 +89,15 @@ __device__ inline double igf_diff(const double *__restrict__ t, int64_t c, int64
 // cell, as the Taylor series of 1/r averaged over the cell up to eighth order.
 // With a = x^2/r^4 (b, c for y, z) it is a polynomial over r,
 //   g = (1/r) sum of C_ijk a^i b^j c^k, i + j + k <= 4, C_000 = 1,
-// whose coefficients hold the mesh sizes (igf_coefficients).  The 8-corner
+// whose coefficients hold the mesh sizes (igf_block, igf_table).  The 8-corner
 // difference of the antiderivative costs three arctangents and three
 // logarithms per corner and cancels: its relative error grows with r^3, 1e-12
-// at kIgfFar cell half diagonals and 1e-9 at 64 of cells 1:1:4, where the
-// truncated series is off by at most 4e-13 and 3e-16 (against a 20-point
-// Gauss rule in 80 bits, cells from 1:1:0.2 to 1:4:16; at ten half diagonals
-// the two meet for cubes).  So only the box within kIgfFar of the origin
-// keeps the corners.  The deposit's launch, which forms G beside the deposit,
+// at kIgfFar cell half diagonals and 1e-9 at 64 of cells 1:1:4.  The truncated
+// series is off by at most rho^-10 / 11 at rho half diagonals, 1.5e-12 at
+// kIgfFar and less than rounding from 30 on, whatever the cell (the bound is a
+// needle's; 1.1e-13 at kIgfFar for cells up to 1:1:4, 5.3e-13 for 1:4:16; at
+// ten half diagonals series and corners meet for cubes).  So only the box
+// within kIgfFar of the origin keeps the corners.  The deposit's launch, which forms G beside the deposit,
 // fell from 60 to 40 us on 128^3 (150k particles, FP64; 2.2M corners, 27 us of
 // the deposit's own) and from 245 to 199 us on 128x128x256 (10M, mixed).
 constexpr int kIgfOrder = 4;                    // pairs of derivatives
