@@ -364,3 +364,22 @@ assert fake.fake_launches(b'k_efield') == 1
 f.download(hip.EX)
 assert fake.fake_launches(b'k_efield') == 1
 """)
+
+
+def test_kept_memory_stays_within_its_bound(fake_hip):
+    """A field of more than 8 GiB ends: the oldest of its blocks go back, what
+    is kept stays below the bound but close to it, and the next field takes it."""
+    fake_hip("""
+b = bunch(1_000)
+base = hip.memory_info()[0]
+sizes = []
+for grid in ((512, 512, 256), (512, 512, 256), (256, 512, 512)):
+    f = hip.FieldQuant(*grid)
+    used = hip.memory_info()[0] - base
+    f.close()
+    held, kept = hip.memory_info()
+    assert used > 8 << 30 and held == base
+    assert (7 << 30) < kept <= (8 << 30) and fake.fake_held() == base + kept, kept
+b.close()
+assert fake.fake_held() == 0
+""")
