@@ -175,7 +175,7 @@ static void bunch_free_all(izh_bunch *b) {
   dfree(b->w0);
   dfree(b->id0);
   dfree(b->d_scal);
-  for (int k = 0; k < 2; k++) dfree(b->hist[k]);
+  dfree(b->hist);
   dfree(b->cursor);
   dfree(b->chunks);
   dfree(b->d_moments);

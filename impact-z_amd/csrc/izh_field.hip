@@ -97,9 +97,10 @@ __device__ inline double igf_diff(const double *__restrict__ t, int64_t c, int64
 // kIgfFar and less than rounding from 30 on, whatever the cell (the bound is a
 // needle's; 1.1e-13 at kIgfFar for cells up to 1:1:4, 5.3e-13 for 1:4:16; at
 // ten half diagonals series and corners meet for cubes).  So only the box
-// within kIgfFar of the origin keeps the corners.  The deposit's launch, which forms G beside the deposit,
-// fell from 60 to 40 us on 128^3 (150k particles, FP64; 2.2M corners, 27 us of
-// the deposit's own) and from 245 to 199 us on 128x128x256 (10M, mixed).
+// within kIgfFar of the origin keeps the corners.  The deposit's launch, which
+// forms G beside the deposit, fell from 60 to 40 us on 128^3 (150k particles,
+// FP64; 2.2M corners, 27 us of the deposit's own) and from 245 to 199 us on
+// 128x128x256 (10M, mixed).
 constexpr int kIgfOrder = 4;                    // pairs of derivatives
 constexpr int kIgfTerms = 35;
 constexpr double kIgfFar = 12.0;
@@ -261,8 +262,9 @@ __device__ __attribute__((always_inline)) inline void fft_conv_middle(
 // Stages [from, to) of the transform (all of them by default), in runs of
 // up to three.
 template <typename T, bool DIT>
-__device__ __attribute__((always_inline)) inline void fft_stages(cx<T> *buf, int LP, int log2L, int lines, const cx<T> *tw,
-                           bool inverse, int mask, int from = 0, int to = -1) {
+__device__ __attribute__((always_inline)) inline void fft_stages(
+    cx<T> *buf, int LP, int log2L, int lines, const cx<T> *tw, bool inverse, int mask,
+    int from = 0, int to = -1) {
   if (to < 0) to = log2L;
   int done = from;
   while (done < to) {

@@ -373,17 +373,21 @@ inline bool pass_boxes(int64_t n, int nb, int64_t nodes) {
 // Whether the passes read and write the rows by non-temporal accesses: once
 // the six rows outgrow the 256 MB last-level cache the next pass finds nothing
 // of them there, and what they push out (the field, the t positions the deposit
-// reads next, the lines a scatter is still filling) is missed.  16 steps by ordinary accesses / so (ms): 7M on 64x64x128 (mixed)
-// 8.57 / 8.15, 7M on 128^3 (FP64) 14.04 / 13.74, 10M on 64^3 (FP64) 11.35 /
-// 10.56, 10M on 128x128x256 (mixed) 18.85 / 18.34, 50M (FP64) 63.1 / 61.9;
-// below the line either sign: 2.5M on 64x64x128 (mixed) 4.40 / 4.46, 4M 6.05 /
-// 5.88, 5M on 128^3 (FP64) 11.90 / 11.87.  The first pass, which scatters
+// reads next, the lines a scatter is still filling) is missed.  16 steps by
+// ordinary accesses / so (ms): 7M on 64x64x128 (mixed) 8.57 / 8.15, 7M on 128^3
+// (FP64) 14.04 / 13.74, 10M on 64^3 (FP64) 11.35 / 10.56, 10M on 128x128x256
+// (mixed) 18.85 / 18.34, 50M (FP64) 63.1 / 61.9; below the line either sign:
+// 2.5M on 64x64x128 (mixed) 4.40 / 4.46, 4M 6.05 / 5.88, 5M on 128^3 (FP64)
+// 11.90 / 11.87.  The first pass, which scatters
 // unsorted rows, has its open lines displaced most: with it 50M 61.7 -> 61.4,
 // 10M on 128x128x256 18.36 -> 18.24.  It stores by ordinary accesses (its lines
 // fill over many groups); the later scatters, whose runs of a tile are long, go
 // past the caches too: 10M on 128x128x256 16.76 -> 16.44, 7M on 128^3 13.35 ->
 // 13.08, 10M on 128^3 16.56 -> 16.25, on 64^3 and 64x64x128 the same within 1%.
 // The t positions are read next and stay ordinary (10M on 64^3 10.56 -> 10.62).
+// Two cases past the line keep ordinary accesses, having no form without a box
+// that streams: passes that kick from the potential (5.6M to 6.3M particles on
+// 128x128x256), and a first pass whose map takes a run-time kind.
 constexpr int64_t kCacheBytes = (int64_t)256 << 20;
 inline bool pass_streams(int64_t n) { return 6 * (int64_t)sizeof(double) * n > kCacheBytes; }
 
@@ -401,7 +405,9 @@ __device__ inline void gather_phi(const T *__restrict__ phi, int i, int j, int k
   const int im = max(i - 1, 0), ip = min(i + 2, nx - 1);
   const int jm = max(j - 1, 0), jp = min(j + 2, ny - 1);
   const int km = max(k - 1, 0), kp = min(k + 2, nz - 1);
-  const auto at = [&](int a, int b, int c) { return (int64_t)a + (int64_t)sy * b + (int64_t)sz * c; };
+  const auto at = [&](int a, int b, int c) {
+    return (int64_t)a + (int64_t)sy * b + (int64_t)sz * c;
+  };
   const auto pair = [&](int b, int c) {
     const T *q = phi + at(i, b, c);
     return Pair{q[0], q[1]};
@@ -587,8 +593,9 @@ __device__ inline void gather_batched(Load ld, int64_t o, int64_t sy, int64_t sz
 // register sets, so the loads of the next slot group land in the set not
 // being worked on.
 // Two blocks (wavefronts) per SIMD (a pass without gather boxes has no more
-// than that to run); three for an in-place pass with a box, an FP32 grid and compile-time push kinds, which then spills at most 4 VGPRs and
-// gains from the extra wavefront (measured: 3%).  FP64 would spill 70 VGPRs
+// than that to run); three for an in-place pass with a box, an FP32 grid and
+// compile-time push kinds, which then spills at most 4 VGPRs and gains from the
+// extra wavefront (measured: 3%).  FP64 would spill 70 VGPRs
 // to scratch at three (32% slower); a scatter pass's LDS (70 KB) allows two.
 template <typename T, int MODE, int KB, int FORM>
 constexpr int pass_blocks_per_cu(int ka) {
@@ -597,7 +604,8 @@ constexpr int pass_blocks_per_cu(int ka) {
 }
 
 template <typename T, int MODE, int KB, int KA, int FORM>
-__global__ void __launch_bounds__(kBlock, (pass_blocks_per_cu<T, MODE, KB, FORM>(KA))) k_pass(PassCfg c) {
+__global__ void __launch_bounds__(kBlock, (pass_blocks_per_cu<T, MODE, KB, FORM>(KA)))
+k_pass(PassCfg c) {
   constexpr bool BOX = FORM != kFormPhi;
   constexpr bool kPast = FORM == kFormStream;
   constexpr bool kScatter = (MODE & kPassScatter) != 0, kKeys = (MODE & kPassKeys) != 0;
@@ -1071,7 +1079,8 @@ void launch_pass_mode(int mode, int nb, hipStream_t st, const PassCfg &pc) {
 template <typename T, int KB, int KA>
 void launch_pass_kinds(int mode, int nb, hipStream_t st, const PassCfg &pc) {
   // without a kick there is no field to take: no box, which a run-time kind
-  // would carry for nothing
+  // would carry for nothing (such a first pass then reads its rows by ordinary
+  // accesses, whatever their number)
   const bool no_box = KB == kPushAnyKind && pc.kb == kPushNone;
   if (pc.form == kFormStream && !no_box) {
     launch_pass_mode<T, KB, KA, kFormStream>(mode, nb, st, pc);
@@ -1410,14 +1419,13 @@ int bunch_alloc_fused(izh_bunch *b, int ntiles, int64_t nseg) {
     IZH_HIP(hipStreamSynchronize(b->stream));
     // the cursors and lists the last run left for the next one go
     b->keys_valid = 0;
-    for (int k = 0; k < 2; k++) dev_release(b->hist[k]);
+    dev_release(b->hist);
     dev_release(b->cursor);
     dev_release(b->chunks);
-    b->hist[0] = b->hist[1] = b->cursor = nullptr;
+    b->hist = b->cursor = nullptr;
     b->chunks = nullptr;
     b->ntiles_cap = b->nchunks_cap = 0;
-    for (int k = 0; k < 2; k++)
-      IZH_HIP(dev_malloc((void **)&b->hist[k], (size_t)ntiles * sizeof(uint32_t)));
+    IZH_HIP(dev_malloc((void **)&b->hist, (size_t)ntiles * sizeof(uint32_t)));
     IZH_HIP(dev_malloc((void **)&b->cursor, (size_t)ntiles * sizeof(uint32_t)));
     IZH_HIP(dev_malloc((void **)&b->chunks, (size_t)2 * nch * sizeof(Chunk)));
     b->ntiles_cap = ntiles;
@@ -1569,7 +1577,7 @@ struct Runner {
     g_next = warm ? b->keys_po : 0;
     g_cur = 1 - g_next;
     b->keys_valid = 0;
-    uint32_t *hist = b->hist[0];
+    uint32_t *hist = b->hist;
     // ---- device scalars
     DevScal hs{};
     if (warm) {

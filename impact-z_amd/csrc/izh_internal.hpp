@@ -58,7 +58,7 @@ constexpr int kConvRed = 8;          // 3 min, 3 max, lost, alive
 constexpr int kPartStride = kMoments + kConvRed;
 constexpr int kChunk = 16384;        // most particles per deposit chunk
 constexpr int kChunkMin = 1024;      // and the smallest such limit
-constexpr int kChunkBlocks = 256;    // chunks a bunch is cut into at least
+constexpr int kChunkBlocks = 256;    // chunks below which the limit is halved
 constexpr int kTileShift = 3;        // sort tiles of 8x8x8 cells
 constexpr uint32_t kDeadKey = 0xffffffffu;
 constexpr int kSinkBytes = 64 * 8 * 16;  // one 8-byte word per lane, 16 rows
@@ -120,8 +120,8 @@ struct DevScal {
 
 // Slots per deposit chunk of a bunch of cap slots: kChunk, halved while that
 // cuts the bunch into fewer than kChunkBlocks chunks, so a small bunch still
-// gives every CU a block, and no further, because every chunk flushes its
-// whole window.  Deposit per step, one limit of 16384 / this rule / the rule
+// gives every CU a block, but not below kChunkMin (a bunch of less than 262144
+// particles makes fewer chunks), because every chunk flushes its whole window.  Deposit per step, one limit of 16384 / this rule / the rule
 // with 1024 chunks: 100k particles on 32^3 (FP64) 28.9 / 7.9 / 7.9 us, 2M on
 // 64^3 (FP64) 47 / 30 / 57, 4M on 32^3 (FP32) 47 / 38 / 65.  By the bunch's
 // allocation, which a loss of particles does not change: a warm start takes
@@ -185,7 +185,7 @@ struct izh_bunch {
   // fused-run scratch
   izh::DevScal *d_scal = nullptr;
   izh::DevScal *h_scal = nullptr;          // pinned mirror
-  uint32_t *hist[2] = {nullptr, nullptr};   // tile histograms (ping-pong)
+  uint32_t *hist = nullptr;                 // tile histogram
   uint32_t *cursor = nullptr;               // scatter cursors per tile
   izh::Chunk *chunks = nullptr;             // deposit work list
   int64_t ntiles_cap = 0, nchunks_cap = 0;

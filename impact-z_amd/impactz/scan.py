@@ -92,7 +92,7 @@ def footprint(n: int, grid, precision: int, steps: int = 0) -> int:
     ldx = (kx + row - 1) // row * row  # x pitch of the half spectra
     tiles = max(1, (nx >> 3) * (ny >> 3) * (nz >> 3))
     bunch = n * (2 * 48 + 4 * 4 + 3 * pe + 3 * 8) + 2048 * 52 * 8 \
-        + 2 * (max(n // 16384, 512) + tiles + 1) * 12 + 3 * tiles * 4
+        + 2 * (max(n // 16384, 512) + tiles + 1) * 12 + 2 * tiles * 4
     field = g * (8 + 2 * pe + 4 * pe) + ldx * ny * nz * 2 * pe + ldx * 2 * ny * nz * 2 * pe \
         + (kx + ldx) * (ny + 1) * (nz + 1) * pe + (nx + 2) * (ny + 2) * (nz + 2) * 8 \
         + (nx + ny + nz) * 2 * pe
