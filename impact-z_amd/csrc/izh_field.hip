@@ -889,7 +889,10 @@ k_deposit_direct(DepRows d, unsigned long long *__restrict__ rho) {
 }
 
 // A grid that fits LDS: each block accumulates all of it for its share of the
-// particles and adds its nonzero nodes to the grid once.
+// particles and adds its nonzero nodes to the grid once.  On 16x16x32, us at
+// kSmallPer 512 / 1024 / 2048 / 4096: 5k particles 9.9 / 10.0 / 11.1 / 12.5, 20k
+// 8.8 / 10.0 / 11.6 / 16.3, 100k 12.9 / 11.4 / 12.1 / 16.6, 300k 20.0 / 20.4 /
+// 16.7 / 17.8: shorter shares for few particles, fewer flushes for many.
 constexpr int kSmallGrid = 8192;      // nodes: 64 KB, two blocks per CU
 constexpr int kSmallPer = 1024;       // particles per block at least
 constexpr int kSmallBlocks = 256;
@@ -924,7 +927,13 @@ k_deposit_small(DepRows d, unsigned long long *__restrict__ rho) {
 // a tile accumulates in the tile's 9x9x9 nodes.  Straight to the grid, the
 // int64 adds of scattered particles reach 17 G/s (2M on 64^3: 958 us, where
 // the positions take 10 us to read).  The order the sort leaves within a tile
-// varies from run to run and changes no bit of the sum.
+// varies from run to run and changes no bit of the sum.  The whole chain, us:
+//   kBinPer 4 / 8 / 16        20k on 32^3 25.5 / 28.4 / 35.1, 300k on 64^3 41.6 /
+//                             44.2 / 51.3, 2M on 64^3 86 / 85 / 88, 2M on 128^3
+//                             143 / 139 / 136, 10M on 128x128x256 596 / 579 / 581
+//   kBinChunk 1024 / 2048 /   100k on 32^3 28.9 / 31.9 / 38.6 / 49.2, 2M on 64^3
+//   4096 / 8192               98 / 85 / 86 / 96, 10M on 128x128x256 612 / 579 /
+//                             576 / 585
 constexpr int kBinThreads = 512;
 constexpr int kBinPer = 8;            // particles per thread of a scatter block
 constexpr int kBinLdsTiles = 8192;    // tiles a block counts in LDS (32 KB)
@@ -1665,7 +1674,10 @@ static bool bins_ready(izh_field *f, int64_t n, bool weights, int ntiles) {
 
 // izh_charge's deposit: straight to the grid up to kDirect particles (the
 // adds of a few thousand take less than the launches of anything else), the
-// whole grid in LDS up to kSmallGrid nodes, binned otherwise.
+// whole grid in LDS up to kSmallGrid nodes, binned otherwise.  The line is the
+// small grids': on 16x16x32 direct / in LDS 7.9 / 9.4 us at 1000 particles, 9.1 /
+// 9.6 at 4096, 13.2 / 9.6 at 8192.  Against the bins direct adds would stay ahead
+// longer (64^3: 8.8 / 24.6 at 4096, 12.3 / 26.7 at 16384, 958 / 85 at 2M).
 constexpr int64_t kDirect = 4096;
 int launch_deposit_granular(izh_bunch *b, izh_field *f) {
   deposit_scales(b, f);
