@@ -382,8 +382,10 @@ inline bool pass_boxes(int64_t n, int nb, int64_t nodes) {
 // unsorted rows, has its open lines displaced most: with it 50M 61.7 -> 61.4,
 // 10M on 128x128x256 18.36 -> 18.24.  It stores by ordinary accesses (its lines
 // fill over many groups); the later scatters, whose runs of a tile are long, go
-// past the caches too: 10M on 128x128x256 16.76 -> 16.44, 7M on 128^3 13.35 ->
-// 13.08, 10M on 128^3 16.56 -> 16.25, on 64^3 and 64x64x128 the same within 1%.
+// past the caches too.  32 steps by ordinary stores / so: 7M on 128^3 (FP64)
+// 24.4 / 23.9, 10M on 128x128x256 37.95 / 37.55 (mixed 30.6 / 30.0), 20M 55.7 /
+// 55.7, 10M on 64^3 18.17 / 18.27; 96 steps of 50M 278.9 / 280.4 (mixed 246.9 /
+// 246.1): the largest and the coarsest lose a little by it.
 // The t positions are read next and stay ordinary (10M on 64^3 10.56 -> 10.62).
 // Two cases past the line keep ordinary accesses, having no form without a box
 // that streams: passes that kick from the potential (5.6M to 6.3M particles on
