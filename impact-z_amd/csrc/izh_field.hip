@@ -19,6 +19,7 @@
 // natural out), so no reorder pass is needed between them.
 #include <algorithm>
 #include <array>
+#include <atomic>
 #include <cmath>
 #include <cstring>
 #include <map>
@@ -1573,8 +1574,14 @@ int field_alloc(izh_field *f) {
   return upload_tables<float>(f);
 }
 
+uint64_t next_stamp() {
+  static std::atomic<uint64_t> last{0};
+  return ++last;
+}
+
 int field_set_domain(izh_field *f, const izh_compdom *dom) {
   IZH_CHECK(field_fresh_e(f));
+  f->dom_stamp = next_stamp();
   // the pinned staging buffer may still feed an earlier copy
   IZH_HIP(hipStreamSynchronize(f->stream));
   DevDom d{};

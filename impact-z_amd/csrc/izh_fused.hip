@@ -1574,11 +1574,11 @@ struct Runner {
     // the keys of the last scan put them in at the next scatter.  The
     // previous run on this bunch and field left its last scan (keys,
     // cursors, chunks) in slot b->keys_po: start from it.
-    const bool warm = b->keys_valid && b->keys_field == f && b->keys_grid[0] == nx &&
-                      b->keys_grid[1] == ny && b->keys_grid[2] == nz;
+    const bool warm = b->keys_valid && b->keys_stamp == f->dom_stamp;
     g_next = warm ? b->keys_po : 0;
     g_cur = 1 - g_next;
     b->keys_valid = 0;
+    f->dom_stamp = next_stamp();
     uint32_t *hist = b->hist;
     // ---- device scalars
     DevScal hs{};
@@ -1819,8 +1819,7 @@ struct Runner {
     f->have_phi = 1;
     b->keys_valid = 1;
     b->keys_po = g_next;
-    b->keys_field = f;
-    b->keys_grid[0] = nx; b->keys_grid[1] = ny; b->keys_grid[2] = nz;
+    b->keys_stamp = f->dom_stamp;
     return IZH_OK;
   }
 };

@@ -196,8 +196,7 @@ struct izh_bunch {
   // Sort keys, their scan (cursor) and first deposit chunks left by the last
   // izh_run for the next one; any other change to the particles clears this.
   int keys_valid = 0;
-  const izh_field *keys_field = nullptr;
-  int keys_grid[3] = {0, 0, 0};
+  uint64_t keys_stamp = 0;  // the dom_stamp their run left: its key grids are there
   int keys_po = 0;  // chunk slot holding the next run's first deposit grouping
 };
 
@@ -225,6 +224,7 @@ struct izh_field {
   const double *igf_tab = nullptr;
   const void *tw_x = nullptr, *tw_y = nullptr, *tw_z = nullptr;
   izh::DevDom *d_dom = nullptr; // domain the kernels read
+  uint64_t dom_stamp = 0;       // names its contents, another one with each change
   izh::DevDom *h_dom = nullptr; // pinned staging for host-set domains
   // izh_charge's bins (launch_deposit_granular), made by its first large bunch
   char *bin = nullptr;
@@ -517,6 +517,7 @@ int scratch_setup(int device);
 int launch_download(izh_bunch *b, double *pts9, bool *no_memory);
 int launch_clone(const izh_bunch *src, izh_bunch *dst, int64_t offset, int64_t n, double w);
 int field_set_domain(izh_field *f, const izh_compdom *dom);
+uint64_t next_stamp();  // never given out before in this process
 int launch_deposit(izh_bunch *b, izh_field *f, const Chunk *chunks, const KeyGrid *kgrid,
                    const int64_t *d_nchunks, int64_t max_chunks);
 int launch_deposit_granular(izh_bunch *b, izh_field *f);

@@ -383,3 +383,30 @@ for grid in ((512, 512, 256), (512, 512, 256), (256, 512, 512)):
 b.close()
 assert fake.fake_held() == 0
 """)
+
+
+def test_run_starts_warm_only_on_what_its_last_run_left(fake_hip):
+    """The sort state of a run goes with the key grids in its field: a field made
+    at the place of one that has ended, and a field whose domain another bunch
+    has set, hold other ones."""
+    fake_hip("""
+def cold():
+    before = fake.fake_launches(b'k_prologue_keys')
+    b.run(f, d, 0.0, [drift()] * 2, BEAM.current)
+    return fake.fake_launches(b'k_prologue_keys') - before
+
+b, other = bunch(5_000), bunch(6_000)
+f, d = hip.FieldQuant(16, 16, 16), hip.CompDom(16, 16, 16)
+answered(2)
+assert cold() and not cold() and not cold()
+for _ in range(5):
+    f.close()
+    f = hip.FieldQuant(16, 16, 16)
+    assert cold() and not cold()
+other.run(f, d, 0.0, [drift()] * 2, BEAM.current)
+assert cold() and not cold()
+other.conv1st(0.05, 1.0, 1.0)
+d.set([0, 1, 0, 1, 0, 1], [1 / 15] * 3)
+other.charge(d, f)
+assert cold() and not cold()
+""")
