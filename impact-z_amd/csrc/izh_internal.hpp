@@ -121,11 +121,11 @@ struct DevScal {
 // Slots per deposit chunk of a bunch of cap slots: kChunk, halved while that
 // cuts the bunch into fewer than kChunkBlocks chunks, so a small bunch still
 // gives every CU a block, but not below kChunkMin (a bunch of less than 262144
-// particles makes fewer chunks), because every chunk flushes its whole window.  Deposit per step, one limit of 16384 / this rule / the rule
-// with 1024 chunks: 100k particles on 32^3 (FP64) 28.9 / 7.9 / 7.9 us, 2M on
-// 64^3 (FP64) 47 / 30 / 57, 4M on 32^3 (FP32) 47 / 38 / 65.  By the bunch's
-// allocation, which a loss of particles does not change: a warm start takes
-// the list of the run before.
+// particles makes fewer chunks), because every chunk flushes its whole window.
+// Deposit per step, one limit of 16384 / this rule / the rule with 1024 chunks:
+// 100k particles on 32^3 (FP64) 28.9 / 7.9 / 7.9 us, 2M on 64^3 (FP64) 47 / 30 /
+// 57, 4M on 32^3 (FP32) 47 / 38 / 65.  By the bunch's allocation, which a loss
+// of particles does not change: a warm start takes the list of the run before.
 inline int chunk_len(int64_t cap) {
   int c = kChunk;
   while (c > kChunkMin && cap < (int64_t)c * kChunkBlocks) c >>= 1;
